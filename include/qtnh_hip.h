@@ -406,15 +406,15 @@ void qtnh_tune_split_tile(int shape);
  * gates on high bits, which loops over the rest.  (The diagonal kernel and the
  * kernels for gates on the lowest 6 bits size their grids to the state.) */
 void qtnh_tune_stream(int max_blocks);
-/* Tile bits (3..13, default 12) of fused circuit runs, and how many of the
- * lowest state bits every tile keeps (0..8, default 4; 2^low x 16 bytes are
- * contiguous in each tile row).  Results do not depend on them. */
+/* Tile bits (3..13) of fused circuit runs, and how many of the lowest state
+ * bits every tile keeps (0..8; 2^low x 16 bytes are contiguous in each tile
+ * row).  Until set, by the state's size: 10 and 3 up to 18 qubits, 11 and 3 at
+ * 19, 12 and 4 from 20.  Results do not depend on them. */
 void qtnh_tune_circuit(int tile_bits, int low_bits);
-/* Kernel for large states with 12-bit tiles: 2 (default) register-blocked
- * (ops applied to 16 amplitudes per thread in registers, one LDS round trip
- * per phase of ops on 4 tile bits), 3 register-blocked with the next tile
- * streamed into a second LDS buffer during the current tile's phases, 1
- * pipelined (per-op LDS passes), 0 plain.  Results do not depend on it. */
+/* Kernel of fused runs: 2 (default) keeps 4 to 16 amplitudes per thread in
+ * registers through the run (tiles of 4 to 12 bits), 1 pipelined (per-op LDS
+ * passes, many 12-bit tiles), 0 plain (per-op LDS passes).  3 is accepted and
+ * runs as 2.  Results do not depend on it. */
 void qtnh_tune_circuit_pipeline(int mode);
 
 #ifdef __cplusplus

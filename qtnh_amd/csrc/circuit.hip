@@ -39,6 +39,7 @@ typedef double double2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kMaxTileBits = 13;  // 2^13 amplitudes = 128 KiB of LDS
 constexpr int kMaxOpQubits = 3;
+constexpr int kMinRegBits = 2, kMaxRegBits = 4;  // register bits of circuit_reg_kernel
 
 struct TileOp {
   int kind;                 // 0: dense gate, 1: diagonal
@@ -46,7 +47,6 @@ struct TileOp {
   int pos[kMaxOpQubits];    // tile bit of op-index bit j (j = 0 most significant)
   int zpos[kMaxOpQubits];   // the same tile bits, ascending
   uint32_t coef;            // first coefficient (complex units)
-  uint32_t rcode;           // register form (circuit_rb_kernel): kind | kb << 1 | reg bit j << (3 + 2 j)
   // Diagonals only: qubits outside the tile.  Byte 0: their count; byte 1 + j:
   // bit of the run's tile number holding the j-th of them (op order).  Their
   // values are fixed within a tile and pick one block of 2^kb coefficients.
@@ -66,14 +66,8 @@ __device__ __forceinline__ uint32_t coef_count(const TileOp &op) {
   return op.kind == 1 ? (1u << (op.kb + (op.outer & 0xffu))) : (1u << (2 * op.kb));
 }
 
-// A phase of a run: consecutive 1- and 2-qubit ops whose bits lie in 4 tile
-// bits (pmask), applied to 16 amplitudes held in registers by each thread; or
-// (lds = 1) a single 3-qubit op applied in LDS.
-struct PhaseDesc {
-  uint32_t op_begin, op_end;
-  uint32_t pmask;
-  uint32_t lds;
-};
+struct RegOp;
+struct RegChunk;
 
 struct RunDesc {
   const TileOp *ops;
@@ -86,8 +80,16 @@ struct RunDesc {
   uint32_t coef_begin;  // first coefficient of op_begin (ops' coefficients are contiguous)
   int tb;               // tile bits
   int n_outer;          // popcount(outer_mask)
-  const PhaseDesc *phases;  // register phases of this run (12-bit tiles), or null
-  uint32_t ph_begin, ph_end;
+  // Register form (circuit_reg_kernel): its ops, coefficients, staging chunks
+  // [chunk_begin, chunk_end) and first register bits (packed).
+  const RegOp *rops;
+  const double2_t *rcoef;
+  const RegChunk *rchunks;
+  uint32_t chunk_begin, chunk_end;
+  uint32_t map0;
+  uint32_t where_in, where_out;  // state bits of the first and the last register bits (8 bits each)
+  int rbits;  // register bits (0: no register form)
+  int has3;   // a run of the launch may hold dense 3-qubit gates
 };
 
 constexpr int kChunkOps = 32;     // ops staged in LDS at a time
@@ -421,345 +423,461 @@ __global__ void __launch_bounds__(kPipeNT, 1)
   }
 }
 
-// Register-blocked runs (12-bit tiles, 256 threads): per phase, each thread
-// takes the 16 tile amplitudes that differ only in the phase's 4 bits from
-// LDS into registers, applies the phase's ops there (compile-time indexing:
-// one instantiation per op shape and register-bit assignment) and writes them
-// back; one LDS round trip and one barrier per phase instead of per op.  The
-// ops do exactly the arithmetic of gate_in_lds / diag_in_lds.  LDS slots are
-// XOR-swizzled (slot = l ^ ((l >> 4) & 15)) so that phases over the low tile
-// bits do not fall on one bank.
-// Read-only tables (ops, phases, coefficients) seen through the constant
-// address space: uniform reads become scalar loads, which do not wait behind
-// the vector-memory counter (and so not behind an LDS DMA in flight).
-typedef const __attribute__((address_space(4))) double2_t *ccoef_t;
+// Register-resident runs: a thread holds 2^R amplitudes of its tile in
+// registers for the whole run.  The tile's index bits split into R register
+// bits (the same for every thread) and the thread bits.  Dense gates act on
+// register bits with compile-time indexing; a diagonal may use any bit (its
+// register bits pick among up to 8 coefficients, its thread bits and the bits
+// outside the tile pick which ones, per lane), so only dense gates ask for
+// other register bits.  Such a change passes the tile through LDS.  The first
+// register bits are those of the first gates, read straight from the state.
+//
+// What bounds it (28 qubits, 12-bit tiles, R = 4): a run of one gate takes
+// 1.66 ms, 5.2 TB/s, what an in-place pass reaches here in workgroups of
+// 64 KiB (5.4 TB/s by a plain kernel); each 1-qubit gate adds 106 us of FP64
+// issue once that passes the memory's time (14 instructions per amplitude at
+// the 33 T a second the card reaches: 114), a diagonal 44, an exchange 100.
+// Four workgroups per compute unit (half the LDS: real and imaginary parts
+// are exchanged one after the other; at most 128 VGPRs) hide one another's
+// loads and exchanges.  The 28-qubit depth-6 random circuit went from 56.2 to
+// 37.7 ms with this form (from a tile kept in LDS between phases, 64 KiB and
+// two workgroups per compute unit, whose op switch copied the amplitudes).
+//
+// The op list and its coefficients are staged in LDS by chunks; an op is one
+// 16-byte record, read by every lane from one address and made uniform.
+//
+// Arithmetic: that of gate_in_lds / diag_in_lds.  Their sums start from 0.0:
+// here the first product's leading term is fma(x, y, +0.0), which is x * y
+// rounded, with an exact -0 turned into the +0 that adding to 0.0 gives, one
+// instruction where a multiply and an add were.  (Only a product that
+// underflows to -0 keeps its sign where 0.0 + -0 gave +0, and that shows only
+// if every other term of the sum is -0 as well.)
+struct RegOp {
+  // One bit per op form.  1-qubit gates on register bits 3..0 (kRegG1): one
+  // record may hold several, applied from the highest bit down, their
+  // coefficients one after another.  0 ends a chunk.
+  uint32_t code;
+  uint32_t coef;  // first coefficient (of the run's list)
+  // Diagonals: tile positions of the thread bits in bytes 0..2, the least
+  // significant last (31, a zero bit, where there are fewer than three), and
+  // their count in byte 3.  kRegSpecial: 0 for a dense 3-qubit gate, else a
+  // change of register bits: kRegRemapFlag and their tile positions, 4 bits each.
+  uint32_t lane;
+  uint32_t outer;  // diagonals: bits of the tile number, likewise (63: a zero bit; no count)
+};
+constexpr int kRegG1 = 0, kRegG2 = 4, kRegSpecial = 16, kRegD0 = 17, kRegD1 = 18, kRegD2 = 22, kRegD3 = 28;
+constexpr uint32_t kRegRemapFlag = 1u << 31, kRegNoLane = 0x1f1f1f, kRegNoOuter = 0x3f3f3f;
+constexpr int kRegOps = 48, kRegCoef = 384;  // per chunk: with a 32 KiB half tile, four workgroups fit 160 KiB
+struct RegChunk {
+  uint32_t op_begin, op_end, coef_begin, coef_end;
+};
+
+// Read-only tables seen through the constant address space: uniform reads
+// become scalar loads.
 template <typename T>
 __device__ __forceinline__ const __attribute__((address_space(4))) T *as_const(const T *p) {
   return (const __attribute__((address_space(4))) T *)(p);
 }
 
-// Field-by-field copies out of the constant address space (scalar loads).
-__device__ __forceinline__ TileOp load_op(const __attribute__((address_space(4))) TileOp *p) {
-  TileOp t;
-  t.kind = p->kind;
-  t.kb = p->kb;
+// Tile element l's LDS slot: l with its low five bits mixed with bits 5..11,
+// so that the lanes of an access fall on different banks for nearly every
+// choice of register bits (the vectors were searched for; at most two-way for
+// contiguous ones).  Linear over XOR.
+__host__ __device__ __forceinline__ uint32_t reg_slot(uint32_t l) {
+  constexpr uint32_t kMix[7] = {31, 11, 28, 26, 25, 3, 9};
+  uint32_t s = l;
 #pragma unroll
-  for (int j = 0; j < kMaxOpQubits; ++j) {
-    t.pos[j] = p->pos[j];
-    t.zpos[j] = p->zpos[j];
-  }
-  t.coef = p->coef;
-  t.rcode = p->rcode;
-  t.outer = p->outer;
-  return t;
-}
-__device__ __forceinline__ PhaseDesc load_phase(const __attribute__((address_space(4))) PhaseDesc *p) {
-  PhaseDesc d;
-  d.op_begin = p->op_begin;
-  d.op_end = p->op_end;
-  d.pmask = p->pmask;
-  d.lds = p->lds;
-  return d;
+  for (int i = 0; i < 7; ++i) s ^= (0u - ((l >> (5 + i)) & 1u)) & kMix[i];
+  return s;
 }
 
-template <int KB, int A, int B, int C>
-__device__ __forceinline__ void reg_gate(double2_t (&v)[16], ccoef_t g) {
-  constexpr int K = 1 << KB;
-  constexpr int M = (1 << A) | (KB > 1 ? (1 << B) : 0) | (KB > 2 ? (1 << C) : 0);
+// Deposit over runs of set bits: mask is uniform, so its few runs are walked
+// by scalar code.
+__device__ __forceinline__ uint64_t deposit_runs(uint32_t v, uint64_t mask) {
+  uint64_t r = 0;
+  while (mask) {
+    const int lo = __builtin_ctzll(mask);
+    const uint64_t up = ~(mask >> lo);
+    const int len = up ? __builtin_ctzll(up) : 64;
+    const uint32_t part = len >= 32 ? v : v & ((1u << len) - 1u);
+    r |= (uint64_t)part << lo;
+    v = len >= 32 ? 0 : v >> len;
+    mask = lo + len >= 64 ? 0 : mask >> (lo + len) << (lo + len);
+  }
+  return r;
+}
+
+__device__ __forceinline__ uint64_t deposit_runs64(uint64_t v, uint64_t mask) {
+  uint64_t r = 0;
+  while (mask) {
+    const int lo = __builtin_ctzll(mask);
+    const uint64_t up = ~(mask >> lo);
+    const int len = up ? __builtin_ctzll(up) : 64;
+    const uint64_t field = len >= 64 ? ~0ull : (1ull << len) - 1ull;
+    r |= (v & field) << lo;
+    v = len >= 64 ? 0 : v >> len;
+    mask &= ~(field << lo);
+  }
+  return r;
+}
+
+// x = a + b and x = a - b into the register x already has: the amplitudes keep
+// their registers through every op, so the op loop needs no copies where its
+// cases meet (32 moves per op with plain assignments).
+__device__ __forceinline__ void add_to(double &x, double a, double b) {
+  asm("v_add_f64 %0, %1, %2" : "+v"(x) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void sub_to(double &x, double a, double b) {
+  asm("v_add_f64 %0, %1, -%2" : "+v"(x) : "v"(a), "v"(b));
+}
+
+// x g, as the first term of a sum from 0.0.
+__device__ __forceinline__ double2_t cmul_first(double2_t x, double2_t g) {
+  return double2_t{__builtin_fma(x.x, g.x, 0.0) - x.y * g.y, __builtin_fma(x.x, g.y, 0.0) + x.y * g.x};
+}
+
+template <int R, int A>
+__device__ __forceinline__ void rg_gate1(double (&re)[1 << R], double (&im)[1 << R], const double2_t *g) {
+  const double2_t g00 = g[0], g01 = g[1], g10 = g[2], g11 = g[3];
 #pragma unroll
-  for (int r0 = 0; r0 < 16; ++r0) {
+  for (int r = 0; r < (1 << R); ++r) {
+    if ((r >> A) & 1) continue;
+    const int s = r | (1 << A);
+    const double2_t a = {re[r], im[r]}, b = {re[s], im[s]};
+    const double2_t p0 = cmul_first(a, g00), q0 = cmul2(b, g10);
+    const double2_t p1 = cmul_first(a, g01), q1 = cmul2(b, g11);
+    add_to(re[r], p0.x, q0.x);
+    add_to(im[r], p0.y, q0.y);
+    add_to(re[s], p1.x, q1.x);
+    add_to(im[s], p1.y, q1.y);
+  }
+}
+
+// KB-qubit gate on register bits A, B, C (most significant first).
+template <int R, int KB, int A, int B, int C>
+__device__ __forceinline__ void rg_gate(double (&re)[1 << R], double (&im)[1 << R], const double2_t *g) {
+  constexpr int K = 1 << KB;
+  constexpr int M = (1 << A) | (1 << B) | (KB > 2 ? (1 << C) : 0);
+#pragma unroll
+  for (int r0 = 0; r0 < (1 << R); ++r0) {
     if (r0 & M) continue;
-    // 3-qubit gates: re-read the 64 coefficients per group instead of holding
-    // them in registers (a compiler barrier, no code).
-    if (KB == 3) asm volatile("" ::: "memory");
     int idx[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       int x = r0;
       if ((c >> (KB - 1)) & 1) x |= 1 << A;
-      if (KB > 1 && ((c >> (KB - 2)) & 1)) x |= 1 << B;
+      if ((c >> (KB - 2)) & 1) x |= 1 << B;
       if (KB > 2 && (c & 1)) x |= 1 << C;
       idx[c] = x;
     }
-    double2_t in[K];
+    // Every output's sum over all terms but the last, term by term; the last
+    // term's addition then puts output o in the registers of input o, which no
+    // sum needs any more (the last input's own output comes last).
+    double ar[K], ai[K];
 #pragma unroll
-    for (int c = 0; c < K; ++c) in[c] = v[idx[c]];
+    for (int i = 0; i < K; ++i) {
+      const double2_t x = {re[idx[i]], im[idx[i]]};
 #pragma unroll
-    for (int o = 0; o < K; ++o) {
-      if (KB == 3) asm volatile("" ::: "memory");  // one output's 8 coefficients live at a time
-      double2_t acc = {0.0, 0.0};
-#pragma unroll
-      for (int i = 0; i < K; ++i) {
-        const double2_t p = cmul2(in[i], g[i * K + o]);
-        acc.x = acc.x + p.x;
-        acc.y = acc.y + p.y;
+      for (int o = 0; o < K; ++o) {
+        if (o % 4 == 0) asm volatile("" ::: "memory");  // four coefficients live at a time (a compiler barrier, no code)
+        const double2_t p = i == 0 ? cmul_first(x, g[o]) : cmul2(x, g[i * K + o]);
+        if (i == 0) {
+          ar[o] = p.x;
+          ai[o] = p.y;
+        } else if (i + 1 < K) {
+          ar[o] = ar[o] + p.x;
+          ai[o] = ai[o] + p.y;
+        } else {
+          add_to(re[idx[o]], ar[o], p.x);
+          add_to(im[idx[o]], ai[o], p.y);
+        }
       }
-      v[idx[o]] = acc;
     }
   }
 }
 
-template <int KB, int A, int B, int C>
-__device__ __forceinline__ void reg_diag(double2_t (&v)[16], ccoef_t d) {
+// Diagonal whose register bits are those of MASK: d holds 2^popcount(MASK)
+// coefficients, indexed by them (highest bit most significant).
+template <int R, int MASK>
+__device__ __forceinline__ void rg_diag(double (&re)[1 << R], double (&im)[1 << R], const double2_t *d) {
+  constexpr int NB = __builtin_popcount(MASK);
+  constexpr int H = NB > 2 ? 2 : 1, NC = (1 << NB) / H;  // at most four coefficients live at a time
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    int c = KB > 0 ? (r >> A) & 1 : 0;
-    if (KB > 1) c = (c << 1) | ((r >> B) & 1);
-    if (KB > 2) c = (c << 1) | ((r >> C) & 1);
-    v[r] = cmul2(v[r], d[c]);
-  }
-}
-
-__device__ __forceinline__ void apply_reg_op(double2_t (&v)[16], uint32_t code, ccoef_t g) {
-  switch (code) {
-    case 2: reg_gate<1, 0, 0, 0>(v, g); break;
-    case 10: reg_gate<1, 1, 0, 0>(v, g); break;
-    case 18: reg_gate<1, 2, 0, 0>(v, g); break;
-    case 26: reg_gate<1, 3, 0, 0>(v, g); break;
-    case 36: reg_gate<2, 0, 1, 0>(v, g); break;
-    case 68: reg_gate<2, 0, 2, 0>(v, g); break;
-    case 100: reg_gate<2, 0, 3, 0>(v, g); break;
-    case 12: reg_gate<2, 1, 0, 0>(v, g); break;
-    case 76: reg_gate<2, 1, 2, 0>(v, g); break;
-    case 108: reg_gate<2, 1, 3, 0>(v, g); break;
-    case 20: reg_gate<2, 2, 0, 0>(v, g); break;
-    case 52: reg_gate<2, 2, 1, 0>(v, g); break;
-    case 116: reg_gate<2, 2, 3, 0>(v, g); break;
-    case 28: reg_gate<2, 3, 0, 0>(v, g); break;
-    case 60: reg_gate<2, 3, 1, 0>(v, g); break;
-    case 92: reg_gate<2, 3, 2, 0>(v, g); break;
-    case 1: reg_diag<0, 0, 0, 0>(v, g); break;
-    case 3: reg_diag<1, 0, 0, 0>(v, g); break;
-    case 11: reg_diag<1, 1, 0, 0>(v, g); break;
-    case 19: reg_diag<1, 2, 0, 0>(v, g); break;
-    case 27: reg_diag<1, 3, 0, 0>(v, g); break;
-    case 37: reg_diag<2, 0, 1, 0>(v, g); break;
-    case 69: reg_diag<2, 0, 2, 0>(v, g); break;
-    case 101: reg_diag<2, 0, 3, 0>(v, g); break;
-    case 13: reg_diag<2, 1, 0, 0>(v, g); break;
-    case 77: reg_diag<2, 1, 2, 0>(v, g); break;
-    case 109: reg_diag<2, 1, 3, 0>(v, g); break;
-    case 21: reg_diag<2, 2, 0, 0>(v, g); break;
-    case 53: reg_diag<2, 2, 1, 0>(v, g); break;
-    case 117: reg_diag<2, 2, 3, 0>(v, g); break;
-    case 29: reg_diag<2, 3, 0, 0>(v, g); break;
-    case 61: reg_diag<2, 3, 1, 0>(v, g); break;
-    case 93: reg_diag<2, 3, 2, 0>(v, g); break;
-    // The host emits only the codes above (reg_code_ok).  With no default
-    // path, each leaf of the compiler's branch tree is a case, and the 16
-    // amplitudes are not copied to a merge register set on the way (32 64-bit
-    // moves per thread per op, measured in the gfx950 code).
-    default: __builtin_unreachable();
-  }
-}
-
-__device__ __forceinline__ int rb_slot(int l) { return l ^ ((l >> 4) & 15); }
-
-// A 3-qubit op on the swizzled 12-bit tile: the arithmetic of gate_in_lds<3> / diag_in_lds<3>.
-__device__ __forceinline__ void rb_lds_op3(double2_t *buf, const TileOp &op, ccoef_t g) {
-  if (op.kind == 1) {
-    // The 8 coefficients are read once (uniform loads) and selected per element.
-    double2_t d[8];
+  for (int h = 0; h < H; ++h) {
+    if (h) asm volatile("" ::: "memory");  // (a compiler barrier, no code)
+    double2_t c[NC];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) d[c] = g[c];
-    for (int l = threadIdx.x; l < 4096; l += 256) {
-      const int b0 = (l >> op.pos[0]) & 1, b1 = (l >> op.pos[1]) & 1, b2 = (l >> op.pos[2]) & 1;
-      const double2_t lo = b1 ? (b2 ? d[3] : d[2]) : (b2 ? d[1] : d[0]);
-      const double2_t hi = b1 ? (b2 ? d[7] : d[6]) : (b2 ? d[5] : d[4]);
-      buf[rb_slot(l)] = cmul2(buf[rb_slot(l)], b0 ? hi : lo);
-    }
-    return;
-  }
-  int comb[8];
+    for (int i = 0; i < NC; ++i) c[i] = d[h * NC + i];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    int off = 0;
+    for (int r = 0; r < (1 << R); ++r) {
+      int i = 0;
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      if ((c >> (2 - j)) & 1) off |= 1 << op.pos[j];
-    comb[c] = off;
-  }
-  for (int gi = threadIdx.x; gi < 512; gi += 256) {
-    asm volatile("" ::: "memory");  // coefficients re-read per group, not held in registers
-    int base = gi;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int p = op.zpos[j];
-      base = ((base >> p) << (p + 1)) | (base & ((1 << p) - 1));
-    }
-    double2_t in[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) in[c] = buf[rb_slot(base + comb[c])];
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      double2_t acc = {0.0, 0.0};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const double2_t p = cmul2(in[i], g[i * 8 + o]);
-        acc.x = acc.x + p.x;
-        acc.y = acc.y + p.y;
-      }
-      buf[rb_slot(base + comb[o])] = acc;
+      for (int b = R - 1; b >= 0; --b)
+        if ((MASK >> b) & 1) i = (i << 1) | ((r >> b) & 1);
+      if (i / NC != h) continue;
+      i %= NC;
+      // All products before the first result takes its register.
+      const double xc = re[r] * c[i].x, ys = im[r] * c[i].y, xs = re[r] * c[i].y, yc = im[r] * c[i].x;
+      sub_to(re[r], xc, ys);
+      add_to(im[r], xs, yc);
     }
   }
 }
 
-// Split of a 12-bit tile for the register-blocked layout: its lowest 8 state
-// bits (taken from the thread index) and the other 4.
-__device__ __forceinline__ void rb_masks(const RunDesc &R, uint64_t &lo_mask, uint64_t &rest) {
-  lo_mask = 0;
-  rest = R.tile_mask;
-  for (int b = 0; b < 8; ++b) {
-    const uint64_t low = rest & (0 - rest);
-    lo_mask |= low;
-    rest ^= low;
+// Register bit k sits at tile bit (map >> 4 k) & 15.
+template <int R>
+__device__ __forceinline__ uint32_t reg_mask(uint32_t map) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int k = 0; k < R; ++k) m |= 1u << ((map >> (4 * k)) & 15u);
+  return m;
+}
+// Tile index of this thread's element 0: the thread's bits with zeros at the register bits.
+template <int R>
+__device__ __forceinline__ uint32_t reg_base(uint32_t tid, uint32_t map) {
+  uint32_t m = reg_mask<R>(map), base = tid;
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t low = m & (0u - m);
+    m ^= low;
+    base = ((base & ~(low - 1u)) << 1) | (base & (low - 1u));
   }
+  return base;
 }
 
-// The phases of run R on tile t, held in the swizzled buffer; ends with a barrier.
-__device__ __forceinline__ void rb_phases(double2_t *buf, const RunDesc &R, uint64_t t, int tid) {
-  const auto phases = as_const(R.phases);
-  const auto ops = as_const(R.ops);
-  const ccoef_t coef = as_const(R.coef);
-  for (uint32_t ph = R.ph_begin; ph < R.ph_end; ++ph) {
-    const PhaseDesc P = load_phase(phases + ph);
-    if (P.lds) {
-      // A 3-qubit op, in LDS (its tile bits index the swizzled buffer through rb_slot).
-      const TileOp op = load_op(ops + P.op_begin);
-      rb_lds_op3(buf, op, coef + op.coef + (op.kind == 1 ? outer_sel(op, t) : 0u));
-      lds_barrier();
-      continue;
+// This thread's 2^R elements of a tile under one set of register bits: element
+// r sits at lane | the state bits of r's register bits.
+template <int R>
+struct RegRefs {
+  uint64_t lane = 0;
+  uint64_t bit[R] = {};
+  // where: state bits of the register bits (8 bits each).
+  __device__ __forceinline__ void set(uint32_t tid, uint64_t tile_mask, uint32_t where) {
+    uint64_t regs = 0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      bit[k] = 1ull << ((where >> (8 * k)) & 63u);
+      regs |= bit[k];
     }
-    // The phase's 4 tile bits as values (ascending): register index r sets bit
-    // k -> tile bit pb[k].  The thread's base element is tid with zero bits
-    // inserted at those 4 positions (the tile's other 8 bits, in order).
-    int pb[4];
-    uint32_t pm = P.pmask;
-    int base = tid;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      pb[k] = (int)(pm & (0u - pm));
-      pm ^= (uint32_t)pb[k];
-      base = ((base & ~(pb[k] - 1)) << 1) | (base & (pb[k] - 1));
-    }
-    // rb_slot is linear over XOR and base has no phase bit set, so each slot is
-    // rb_slot(base) XOR a uniform term.
-    const int slot0 = rb_slot(base);
-    int slot[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      slot[r] = slot0 ^ rb_slot(((r & 1) ? pb[0] : 0) | ((r & 2) ? pb[1] : 0) | ((r & 4) ? pb[2] : 0) |
-                                ((r & 8) ? pb[3] : 0));
-    double2_t v[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = buf[slot[r]];
-    // The next op's descriptor is requested before the current op runs.
-    TileOp op = load_op(ops + P.op_begin);
-    for (uint32_t o = P.op_begin; o < P.op_end; ++o) {
-      const TileOp nxt = load_op(ops + (o + 1 < P.op_end ? o + 1 : o));
-      apply_reg_op(v, op.rcode, coef + op.coef + (op.kind == 1 ? outer_sel(op, t) : 0u));
-      op = nxt;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) buf[slot[r]] = v[r];
-    lds_barrier();
+    lane = deposit_runs(tid, tile_mask & ~regs);
   }
-}
-
-// This thread's 16 elements of tile t of run R (element l = tid + 256 j) and
-// their global offsets.
-struct RbTileRefs {
-  __attribute__((address_space(1))) double2_t *psi;
-  uint64_t lo_off;
-  uint64_t hb[4];  // state-bit values of the tile's 4 upper bits, ascending
-  // Offset of element tid + 256 j.
-  __device__ __forceinline__ uint64_t off(int j) const {
-    return lo_off | ((j & 1) ? hb[0] : 0) | ((j & 2) ? hb[1] : 0) | ((j & 4) ? hb[2] : 0) | ((j & 8) ? hb[3] : 0);
+  __device__ __forceinline__ uint64_t off(int r) const {
+    uint64_t o = lane;
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if ((r >> k) & 1) o |= bit[k];
+    return o;
   }
 };
-__device__ __forceinline__ RbTileRefs rb_refs(const RunDesc &R, uint64_t t, int tid) {
-  uint64_t lo_mask, rest;
-  rb_masks(R, lo_mask, rest);
-  RbTileRefs f;
-  f.psi = (__attribute__((address_space(1))) double2_t *)(R.psi + deposit(t, R.outer_mask));
-  f.lo_off = deposit(tid, lo_mask);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    f.hb[k] = rest & (0 - rest);
-    rest ^= f.hb[k];
-  }
-  return f;
-}
 
-// Write tile t of run R back from the swizzled buffer (element l = tid + 256 j).
-// Global address space: the stores cannot alias LDS.
-__device__ __forceinline__ void rb_store(const double2_t *buf, const RbTileRefs &f, int tid) {
-#pragma unroll
-  for (int j = 0; j < 16; ++j) __builtin_nontemporal_store(buf[rb_slot(tid + 256 * j)], f.psi + f.off(j));
-}
-
-__global__ void __launch_bounds__(256, 2) circuit_rb_kernel(const RunDesc *__restrict__ runs, int nruns,
-                                                            uint64_t total_tiles) {
-  __shared__ double2_t buf[1 << 12];
-  const int tid = threadIdx.x;
-  for (uint64_t gt = blockIdx.x; gt < total_tiles; gt += gridDim.x) {
-    const RunDesc &R = runs[find_run(runs, nruns, gt)];
-    const uint64_t t = gt - R.first;
-    // Gather: element l = tid + 256 j (its low 8 tile bits are the thread's).
-    const RbTileRefs f = rb_refs(R, t, tid);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) buf[rb_slot(tid + 256 * j)] = __builtin_nontemporal_load(f.psi + f.off(j));
-    __syncthreads();
-    rb_phases(buf, R, t, tid);
-    rb_store(buf, f, tid);
-    __syncthreads();
-  }
-}
-
-// Register-blocked runs with the next tile's loads in flight: as
-// circuit_rb_kernel (two 256-thread workgroups per CU, one 64 KiB tile each),
-// but each thread issues the loads of its 16 elements of the next tile into
-// registers before the phases of the current tile, so HBM reads overlap the
-// phases (the LDS-only barriers between phases do not wait for them), and
-// moves them into the buffer after the current tile's write-back.  Same
-// ops, same order, same arithmetic as circuit_rb_kernel.
-__global__ void __launch_bounds__(256, 2) circuit_rbp_kernel(const RunDesc *__restrict__ runs, int nruns,
-                                                             uint64_t total_tiles) {
-  __shared__ double2_t buf[1 << 12];
-  const int tid = threadIdx.x;
+// KD: most qubits of a dense gate among the launch's ops.
+template <int R, int KD, int MINW>
+__global__ void __launch_bounds__(256, MINW)
+    circuit_reg_kernel(const RunDesc *__restrict__ runs, int nruns, uint64_t total_tiles, int lds_tb) {
+  constexpr int E = 1 << R;
+  extern __shared__ double smem[];
+  double2_t *cbuf = reinterpret_cast<double2_t *>(smem + (1u << lds_tb));
+  uint4 *obuf = reinterpret_cast<uint4 *>(cbuf + kRegCoef);
+  const uint32_t thread = threadIdx.x;
+  const RegChunk *staged = nullptr;  // the chunk now in LDS
   uint64_t gt = blockIdx.x;
   if (gt >= total_tiles) return;  // uniform: the whole workgroup leaves
-  double2_t pre[16];
-  {
-    const RunDesc &R = runs[find_run(runs, nruns, gt)];
-    const RbTileRefs f = rb_refs(R, gt - R.first, tid);
+  int run = find_run(runs, nruns, gt), run_in = -1, run_out = -1;
+  RegRefs<R> in, out;
+  double2_t amp[E];
+  // Threads past the tile's (tiles of fewer bits than the launch's widest)
+  // repeat another's work: the same values to the same slots, nothing to the
+  // state.  (Their loads are over before the barriers of an exchange let the
+  // others store; without an exchange they write nothing at all.)
+  auto load = [&](int ri, uint64_t tile) {
+    const RunDesc &D = runs[ri];
+    if (run_in != ri) in.set(thread & ((1u << (D.tb - R)) - 1u), D.tile_mask, D.where_in);
+    run_in = ri;
+    const auto src =
+        (const __attribute__((address_space(1))) double2_t *)(D.psi + deposit_runs64(tile - D.first, D.outer_mask));
 #pragma unroll
-    for (int j = 0; j < 16; ++j) pre[j] = __builtin_nontemporal_load(f.psi + f.off(j));
-#pragma unroll
-    for (int j = 0; j < 16; ++j) buf[rb_slot(tid + 256 * j)] = pre[j];
-    lds_barrier();
-  }
+    for (int r = 0; r < E; ++r) amp[r] = src[in.off(r)];
+  };
+  load(run, gt);
   while (true) {
+    const RunDesc &D = runs[run];
+    const uint64_t t = gt - D.first;
+    const uint32_t nth = 1u << (D.tb - R);
+    const bool live = thread < nth;
+    const uint32_t tid = thread & (nth - 1u);
+    const RegOp *ops = D.rops;
+    const double2_t *coef = D.rcoef;
+    double2_t *psi = D.psi + deposit_runs64(t, D.outer_mask);
+    const auto chunks = as_const(D.rchunks);
+    // Stages chunk c; the barrier before it ends the previous chunk's reads.
+    auto stage = [&](const RegChunk *c, const RegChunk &h) {
+      if (staged == c) return;
+      staged = c;
+      __syncthreads();
+      for (uint32_t i = thread; i < h.op_end - h.op_begin; i += blockDim.x)
+        obuf[i] = reinterpret_cast<const uint4 *>(ops)[h.op_begin + i];
+      if (thread < 2) obuf[h.op_end - h.op_begin + thread] = uint4{0, 0, 0, 0};
+      for (uint32_t i = thread; i < h.coef_end - h.coef_begin; i += blockDim.x) cbuf[i] = coef[h.coef_begin + i];
+      __syncthreads();
+    };
+    uint32_t map = D.map0;
+    uint32_t base = reg_base<R>(tid, map);
+    double re[E], im[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      re[r] = amp[r].x;
+      im[r] = amp[r].y;
+    }
     const uint64_t gn = gt + gridDim.x;
     const bool more = gn < total_tiles;  // uniform
-    if (more) {
-      const RunDesc &Rn = runs[find_run(runs, nruns, gn)];
-      const RbTileRefs f = rb_refs(Rn, gn - Rn.first, tid);
-#pragma unroll
-      for (int j = 0; j < 16; ++j) pre[j] = __builtin_nontemporal_load(f.psi + f.off(j));
+    const int run_next = more ? find_run(runs, nruns, gn) : run;
+    for (uint32_t ci = D.chunk_begin; ci < D.chunk_end; ++ci) {
+      RegChunk h;
+      h.op_begin = chunks[ci].op_begin;
+      h.op_end = chunks[ci].op_end;
+      h.coef_begin = chunks[ci].coef_begin;
+      h.coef_end = chunks[ci].coef_end;
+      stage(D.rchunks + ci, h);
+      const uint32_t c0 = h.coef_begin;
+      uint32_t i = 0, code, co, lane, outer;
+      uint4 rec = obuf[0];
+      // Takes the record read ahead and reads the next one (a chunk ends with code 0).
+      auto next = [&]() {
+        code = __builtin_amdgcn_readfirstlane(rec.x);
+        co = __builtin_amdgcn_readfirstlane(rec.y) - c0;
+        lane = __builtin_amdgcn_readfirstlane(rec.z);
+        outer = __builtin_amdgcn_readfirstlane(rec.w);
+        rec = obuf[++i];
+      };
+      // A diagonal's coefficients of this lane: outer bits, then thread bits, pick the block.
+      auto block = [&](int nr) {
+        uint32_t s = 0;
+        if (outer != kRegNoOuter) {
+          s = (uint32_t)((t >> (outer & 63u)) & 1u) << 2 | (uint32_t)((t >> ((outer >> 8) & 63u)) & 1u) << 1 |
+              (uint32_t)((t >> ((outer >> 16) & 63u)) & 1u);
+          s <<= lane >> 24;
+        }
+        const uint32_t l = ((base >> (lane & 31u)) & 1u) << 2 | ((base >> ((lane >> 8) & 31u)) & 1u) << 1 |
+                           ((base >> ((lane >> 16) & 31u)) & 1u);
+        return cbuf + co + ((s | l) << nr);
+      };
+      // Every form is an `if` of its own that changes the amplitudes in place
+      // (not one of a switch's exclusive branches): the compiler structures
+      // those one after another with copies of the amplitudes between them.
+      // A diagonal's form repeats while the records stay of that form.
+      next();
+      while (code) {
+        if (code & 0xfu) {
+          const double2_t *g = cbuf + co;
+#define QTNH_REG_G1(A)                    \
+  if constexpr (A < R)                    \
+    if (code & (1u << A)) {               \
+      rg_gate1<R, A>(re, im, g);          \
+      g += 4;                             \
     }
-    const RunDesc &R = runs[find_run(runs, nruns, gt)];
-    const uint64_t t = gt - R.first;
-    rb_phases(buf, R, t, tid);
-    rb_store(buf, rb_refs(R, t, tid), tid);
-    if (!more) break;
-    // Every wave has read the buffer for its stores: refill it with the next
-    // tile (waiting here for its loads only, issued before the stores).
-    lds_barrier();
+          QTNH_REG_G1(3)
+          QTNH_REG_G1(2)
+          QTNH_REG_G1(1)
+          QTNH_REG_G1(0)
+#undef QTNH_REG_G1
+          next();
+        }
+#define QTNH_REG_DIAG(BIT, NEED, MASK)                                   \
+  if constexpr (NEED < R)                                                \
+    while (code & (1u << BIT)) {                                         \
+      rg_diag<R, MASK>(re, im, block(__builtin_popcount(MASK)));         \
+      next();                                                            \
+    }
+        if (code & (0x1fu << kRegD0)) {
+          QTNH_REG_DIAG(17, 0, 0)
+          QTNH_REG_DIAG(18, 0, 1)
+          QTNH_REG_DIAG(19, 1, 2)
+          QTNH_REG_DIAG(20, 2, 4)
+          QTNH_REG_DIAG(21, 3, 8)
+        }
+        if (code & (0x3fu << kRegD2)) {
+          QTNH_REG_DIAG(22, 1, 3)
+          QTNH_REG_DIAG(23, 2, 5)
+          QTNH_REG_DIAG(24, 2, 6)
+          QTNH_REG_DIAG(25, 3, 9)
+          QTNH_REG_DIAG(26, 3, 10)
+          QTNH_REG_DIAG(27, 3, 12)
+        }
+        if (code & (0xfu << kRegD3)) {
+          QTNH_REG_DIAG(28, 2, 7)
+          QTNH_REG_DIAG(29, 3, 11)
+          QTNH_REG_DIAG(30, 3, 13)
+          QTNH_REG_DIAG(31, 3, 14)
+        }
+#undef QTNH_REG_DIAG
+        if constexpr (KD > 1) if (code & (0xfffu << kRegG2)) {
+#define QTNH_REG_CASE(BIT, NEED, CALL) \
+  if constexpr (NEED < R)              \
+    if (code & (1u << BIT)) CALL;
+          QTNH_REG_CASE(4, 1, (rg_gate<R, 2, 0, 1, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(5, 2, (rg_gate<R, 2, 0, 2, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(6, 3, (rg_gate<R, 2, 0, 3, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(7, 1, (rg_gate<R, 2, 1, 0, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(8, 2, (rg_gate<R, 2, 1, 2, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(9, 3, (rg_gate<R, 2, 1, 3, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(10, 2, (rg_gate<R, 2, 2, 0, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(11, 2, (rg_gate<R, 2, 2, 1, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(12, 3, (rg_gate<R, 2, 2, 3, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(13, 3, (rg_gate<R, 2, 3, 0, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(14, 3, (rg_gate<R, 2, 3, 1, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(15, 3, (rg_gate<R, 2, 3, 2, 0>(re, im, cbuf + co)))
+#undef QTNH_REG_CASE
+          next();
+        }
+        if (code & (1u << kRegSpecial)) {
+          if constexpr (KD > 2 && R > 2)
+            if (!(lane & kRegRemapFlag)) rg_gate<R, 3, 2, 1, 0>(re, im, cbuf + co);
+          if (lane & kRegRemapFlag) {
+            const uint32_t s0 = reg_slot(base);
+            uint32_t sb[R];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) buf[rb_slot(tid + 256 * j)] = pre[j];
-    lds_barrier();
+            for (int k = 0; k < R; ++k) sb[k] = reg_slot(1u << ((map >> (4 * k)) & 15u));
+            map = lane;
+            base = reg_base<R>(tid, map);
+            const uint32_t s1 = reg_slot(base);
+            uint32_t sn[R];
+#pragma unroll
+            for (int k = 0; k < R; ++k) sn[k] = reg_slot(1u << ((map >> (4 * k)) & 15u));
+            auto slot = [](uint32_t s, const uint32_t (&b)[R], int r) {
+#pragma unroll
+              for (int k = 0; k < R; ++k)
+                if ((r >> k) & 1) s ^= b[k];
+              return s;
+            };
+            lds_barrier();  // the previous exchange has been read
+#pragma unroll
+            for (int r = 0; r < E; ++r) smem[slot(s0, sb, r)] = re[r];
+            lds_barrier();
+#pragma unroll
+            for (int r = 0; r < E; ++r) re[r] = smem[slot(s1, sn, r)];
+            lds_barrier();
+#pragma unroll
+            for (int r = 0; r < E; ++r) smem[slot(s0, sb, r)] = im[r];
+            lds_barrier();
+#pragma unroll
+            for (int r = 0; r < E; ++r) im[r] = smem[slot(s1, sn, r)];
+          }
+          next();
+        }
+      }
+    }
+    // Write back under the last register bits.
+    if (run_out != run) out.set(tid, D.tile_mask, D.where_out);
+    run_out = run;
+    const auto dst = (__attribute__((address_space(1))) double2_t *)(psi);
+    if (live) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) dst[out.off(r)] = double2_t{re[r], im[r]};
+    }
+    if (!more) break;
     gt = gn;
+    run = run_next;
+    load(run, gt);
   }
 }
 
@@ -844,6 +962,8 @@ __global__ void __launch_bounds__(kZThreads) zfinal_kernel(const double *__restr
 }  // namespace qtnh_hip
 
 using qtnh_hip::c128;
+using qtnh_hip::RegChunk;
+using qtnh_hip::RegOp;
 using qtnh_hip::RunDesc;
 using qtnh_hip::TileOp;
 
@@ -871,8 +991,19 @@ struct qtnh_circuit_s {
   };
   std::vector<Run> runs;
   std::vector<TileOp> tops;  // host copy of the compiled ops
-  qtnh_hip::PhaseDesc *d_phases = nullptr;
-  std::vector<std::pair<uint32_t, uint32_t>> run_phases;  // per run: [begin, end) into the phases
+  // Register forms of the runs, by register bits (null: not built).
+  struct RegForm {
+    void *dev = nullptr;  // ops, chunks, coefficients
+    const RegOp *ops = nullptr;
+    const RegChunk *chunks = nullptr;
+    const qtnh_hip::double2_t *coef = nullptr;
+    struct Run {
+      uint32_t chunk_begin, chunk_end, map0, where_in, where_out;
+    };
+    std::vector<Run> runs;
+  };
+  RegForm forms[qtnh_hip::kMaxRegBits + 1];
+  bool has3 = false;  // a dense 3-qubit gate among the compiled ops
   // Uploaded run descriptors of fused runs, per state buffer: a repeated run
   // on the same state launches kernels only (no copy), so it can be captured
   // into a graph.  Cleared when the circuit is recompiled.
@@ -892,11 +1023,22 @@ struct qtnh_circuit_s {
 namespace qtnh_hip {
 namespace {
 
-int g_tile_bits = 12;
-// Large states with 12-bit tiles: 2 register-blocked kernel, 1 pipelined LDS
-// kernel, 0 plain LDS kernel.
+int g_tile_bits = 0;  // 0: by the state's size (default_tile)
+// 2 (and 3): register kernel for tiles of 4 to 12 bits; 1: pipelined LDS kernel
+// for many 12-bit tiles; 0: plain LDS kernel.
 int g_circuit_mode = 2;
 int g_low_bits = 4;  // lowest state bits in every tile: 2^4 x 16 B = 256 B contiguous rows
+
+// Tile bits and low bits of an n-qubit circuit where nothing else is set.
+// 12-bit tiles make the fewest passes, which large states need; a state of
+// fewer tiles than compute units is bound by one tile's latency and takes
+// smaller tiles, more passes over more workgroups (12 / 10-bit tiles: QFT-12
+// 35 / 24 us, random circuits of 16 and 18 qubits 168 / 124 and 163 / 126; 11
+// bits at 19 qubits 262 / 228; at 20 qubits 372 us with 12 bits, 431 with 11).
+void default_tile(int n, int *tb, int *low) {
+  *tb = g_tile_bits ? g_tile_bits : n <= 18 ? 10 : n == 19 ? 11 : 12;
+  *low = g_tile_bits ? g_low_bits : n <= 19 ? 3 : 4;
+}
 
 // State bits an op needs inside the tile: all of a gate's; none of a
 // diagonal's (a qubit outside the tile is fixed per tile and selects the
@@ -947,11 +1089,14 @@ void retire_compiled(qtnh_circuit_s &c) {
   for (auto &kv : c.desc_cache)
     if (kv.second.d) c.retired.push_back(kv.second.d);
   c.desc_cache.clear();
-  for (void *p : {(void *)c.d_ops, (void *)c.d_coef, (void *)c.d_phases})
+  for (void *p : {(void *)c.d_ops, (void *)c.d_coef})
     if (p) c.retired.push_back(p);
+  for (auto &f : c.forms) {
+    if (f.dev) c.retired.push_back(f.dev);
+    f = qtnh_circuit_s::RegForm{};
+  }
   c.d_ops = nullptr;
   c.d_coef = nullptr;
-  c.d_phases = nullptr;
   c.compiled_tb = -1;
 }
 
@@ -963,77 +1108,228 @@ void free_compiled(qtnh_circuit_s &c) {
   c.retired.clear();
 }
 
-// Whether a register-phase op code is one of apply_reg_op's cases: a gate on
-// 1 or 2 register bits, or a diagonal on 0-2 of them, bits distinct.
-bool reg_code_ok(uint32_t code) {
-  const uint32_t kind = code & 1u, kb = (code >> 1) & 3u;
-  if (kb > 2 || (kind == 0 && kb == 0) || (code >> (3 + 2 * kb)) != 0) return false;
-  return kb < 2 || ((code >> 3) & 3u) != ((code >> 5) & 3u);
+// Register bits for a launch of runs of tb-bit tiles: 64 to 256 threads per
+// tile.  More amplitudes per thread mean fewer exchanges and less decoding per
+// amplitude, fewer mean more waves per tile, which small tiles need (random
+// circuit of 16 qubits, 10-bit tiles: 124 us with 2 register bits, 138 with 3,
+// 171 with 4; 24 qubits, 12-bit tiles: 3.74 ms with 2, 2.19 with 3, 1.88 with
+// 4).  A dense 3-qubit gate needs three.
+int reg_bits(int tb, bool has3) { return std::max(has3 ? 3 : kMinRegBits, std::min(tb - 8, kMaxRegBits)); }
+
+// Register forms a circuit with tb-bit tiles needs: the one for its own runs,
+// and the widest (launches that mix circuits of several widths).
+bool wants_form(const qtnh_circuit_s &c, int tb, int R) {
+  if (tb < kMaxRegBits || tb > 12) return false;
+  return R == kMaxRegBits || R == reg_bits(tb, c.has3);
 }
 
-// Register phases of a 12-bit-tile run: consecutive ops whose tile bits fit 4,
-// padded with the highest free tile bits (threads then vary in the low bits).
-void plan_phases(std::vector<TileOp> &tops, uint32_t begin, uint32_t end, std::vector<PhaseDesc> &out) {
-  uint32_t cur = 0, pb = begin;
-  auto mask_of_op = [&](const TileOp &t) {
+// The register form (R register bits) of run r: appends its ops, coefficients
+// and staging chunks.  Consecutive ops whose dense gates fit R tile bits share
+// their register bits; free ones take the highest tile bits, so that threads
+// vary in the lowest (a read or write of the state then covers whole 128-byte
+// lines; where the first or last gates need one of the lowest three bits, an
+// exchange is put before or after them instead).
+void plan_reg_run(const qtnh_circuit_s &c, const qtnh_circuit_s::Run &r, int R, std::vector<RegOp> &ops,
+                  std::vector<double> &coef, std::vector<RegChunk> &chunks,
+                  qtnh_circuit_s::RegForm::Run *fr) {
+  const int tb = (int)r.tbits.size();
+  struct Seg {
+    uint32_t begin, end;
+    int pos[kMaxRegBits];  // tile bit of each register bit
+  };
+  auto tile_bit = [&](int q) {
+    const auto it = std::lower_bound(r.tbits.begin(), r.tbits.end(), c.n - 1 - q);
+    return it != r.tbits.end() && *it == c.n - 1 - q ? (int)(it - r.tbits.begin()) : -1;
+  };
+  std::vector<Seg> segs;
+  uint32_t cur = 0, begin = r.begin;
+  bool fixed = false;
+  int fpos[kMaxRegBits];
+  auto close = [&](uint32_t end) {
+    if (end == begin) return;
+    Seg s;
+    s.begin = begin;
+    s.end = end;
+    if (fixed) {
+      memcpy(s.pos, fpos, sizeof(fpos));
+    } else {
+      uint32_t m = cur;
+      for (int b = tb - 1; b >= 0 && __builtin_popcount(m) < R; --b) m |= 1u << b;
+      int k = 0;
+      for (int b = 0; b < tb; ++b)
+        if ((m >> b) & 1) s.pos[k++] = b;
+    }
+    segs.push_back(s);
+    begin = end;
+    cur = 0;
+    fixed = false;
+  };
+  for (uint32_t i = r.begin; i < r.end; ++i) {
+    const auto &op = c.ops[i];
+    if (op.kind == 1) continue;
     uint32_t m = 0;
-    for (int j = 0; j < t.kb; ++j) m |= 1u << t.pos[j];
+    for (int j = 0; j < op.k; ++j) m |= 1u << tile_bit(op.q[j]);
+    if (op.k == 3) {
+      // Its qubits take register bits 2, 1, 0 in this order.
+      if (cur) close(i);  // (diagonals alone join this gate's register bits)
+      fixed = true;
+      for (int j = 0; j < 3; ++j) fpos[2 - j] = tile_bit(op.q[j]);
+      cur = m;
+      for (int b = tb - 1, k = 3; k < R; --b)
+        if (!((cur >> b) & 1)) {
+          fpos[k++] = b;
+          cur |= 1u << b;
+        }
+    } else if (__builtin_popcount(cur | m) > R) {
+      close(i);
+      cur = m;
+    } else {
+      cur |= m;
+    }
+  }
+  close(r.end);
+  auto pack = [&](const int *pos) {
+    uint32_t m = 0;
+    for (int k = 0; k < R; ++k) m |= (uint32_t)pos[k] << (4 * k);
     return m;
   };
-  auto close = [&](uint32_t pe) {
-    if (pe == pb) return;
-    if (tops[pb].kb == 3) {
-      PhaseDesc ph;
-      ph.op_begin = pb;
-      ph.op_end = pe;
-      ph.pmask = 0;
-      ph.lds = 1;
-      tops[pb].rcode = 0;
-      out.push_back(ph);
-      return;
-    }
-    uint32_t m = cur;
-    for (int b = 11; b >= 0 && __builtin_popcount(m) < 4; --b) m |= 1u << b;
-    PhaseDesc ph;
-    ph.op_begin = pb;
-    ph.op_end = pe;
-    ph.pmask = m;
-    ph.lds = 0;
-    // Register bit of tile bit p: its rank among the phase's 4 bits.
-    auto regbit = [&](int p) { return __builtin_popcount(m & ((1u << p) - 1)); };
-    for (uint32_t i = pb; i < pe; ++i) {
-      TileOp &t = tops[i];
-      uint32_t code = (uint32_t)t.kind | ((uint32_t)t.kb << 1);
-      for (int j = 0; j < t.kb; ++j) code |= (uint32_t)regbit(t.pos[j]) << (3 + 2 * j);
-      t.rcode = code;
-    }
-    out.push_back(ph);
+  int top[kMaxRegBits];
+  for (int k = 0; k < R; ++k) top[k] = tb - R + k;
+  // Whether the state is read and written in whole lines under these register bits.
+  auto whole_lines = [&](const int *pos) {
+    for (int k = 0; k < R; ++k)
+      if (pos[k] < std::min(3, tb - R)) return false;
+    return true;
   };
-  for (uint32_t i = begin; i < end; ++i) {
-    const uint32_t m = mask_of_op(tops[i]);
-    if (tops[i].kb == 3) {
-      close(i);
-      pb = i;
-      close(i + 1);
-      pb = i + 1;
-      cur = 0;
-      continue;
+  uint32_t chunk_op = (uint32_t)ops.size(), chunk_coef = (uint32_t)(coef.size() / 2);
+  auto end_chunk = [&]() {
+    if (ops.size() == chunk_op) return;
+    chunks.push_back(RegChunk{chunk_op, (uint32_t)ops.size(), chunk_coef, (uint32_t)(coef.size() / 2)});
+    chunk_op = (uint32_t)ops.size();
+    chunk_coef = (uint32_t)(coef.size() / 2);
+  };
+  auto room = [&](size_t ncoef) {
+    if (ops.size() - chunk_op + 1 > (size_t)kRegOps || coef.size() / 2 - chunk_coef + ncoef > (size_t)kRegCoef)
+      end_chunk();
+  };
+  uint32_t map = 0;
+  auto remap = [&](const int *pos) {
+    if (pack(pos) == map) return;
+    map = pack(pos);
+    room(0);
+    ops.push_back(RegOp{1u << kRegSpecial, (uint32_t)(coef.size() / 2), map | kRegRemapFlag, 0});
+  };
+  map = fr->map0 = pack(!segs.empty() && whole_lines(segs[0].pos) ? segs[0].pos : top);
+  for (const Seg &s : segs) {
+    remap(s.pos);
+    auto reg_bit = [&](int tbit) {
+      for (int k = 0; k < R; ++k)
+        if (s.pos[k] == tbit) return k;
+      return -1;
+    };
+    for (uint32_t i = s.begin; i < s.end; ++i) {
+      const auto &op = c.ops[i];
+      const size_t ncoef = op.coef.size() / 2;
+      room(ncoef);
+      RegOp o{0, (uint32_t)(coef.size() / 2), 0, 0};
+      if (op.kind == 0) {
+        const int a = reg_bit(tile_bit(op.q[0])), b = op.k > 1 ? reg_bit(tile_bit(op.q[1])) : 0;
+        // A 1-qubit gate joins the record before it if its register bit is below all of that one's.
+        RegOp *prev = ops.size() > chunk_op ? &ops.back() : nullptr;
+        const bool join = op.k == 1 && prev && prev->code && prev->code < 16u && (prev->code & ((2u << a) - 1u)) == 0;
+        if (join)
+          prev->code |= 1u << a;
+        else
+          o.code = 1u << (op.k == 1 ? kRegG1 + a : op.k == 2 ? kRegG2 + 3 * a + (b > a ? b - 1 : b) : kRegSpecial);
+        coef.insert(coef.end(), op.coef.begin(), op.coef.end());
+        if (!join) ops.push_back(o);
+        continue;
+      }
+      // Table order, most significant first: outer bits, thread bits, register bits from the highest.
+      int order[3], no = 0, nl = 0, nr = 0, regs = 0;
+      o.lane = kRegNoLane;
+      o.outer = kRegNoOuter;
+      for (int j = 0; j < op.k; ++j)
+        if (tile_bit(op.q[j]) < 0) {
+          const int sb = c.n - 1 - op.q[j];
+          const int below = (int)(std::lower_bound(r.tbits.begin(), r.tbits.end(), sb) - r.tbits.begin());
+          o.outer = (o.outer >> 8) | (uint32_t)(sb - below) << 16;
+          order[no++] = j;
+        }
+      for (int j = 0; j < op.k; ++j)
+        if (tile_bit(op.q[j]) >= 0 && reg_bit(tile_bit(op.q[j])) < 0) {
+          o.lane = (o.lane >> 8) | (uint32_t)tile_bit(op.q[j]) << 16;
+          order[no + nl++] = j;
+        }
+      for (int k = R - 1; k >= 0; --k)
+        for (int j = 0; j < op.k; ++j)
+          if (tile_bit(op.q[j]) >= 0 && reg_bit(tile_bit(op.q[j])) == k) {
+            order[no + nl + nr++] = j;
+            regs |= 1 << k;
+          }
+      o.lane |= (uint32_t)nl << 24;
+      const int hi = 31 - __builtin_clz((unsigned)regs | 1u), lo = __builtin_ctz((unsigned)regs | 16u);
+      o.code = 1u << (nr == 0   ? kRegD0
+                      : nr == 1 ? kRegD1 + hi
+                      : nr == 2 ? kRegD2 + hi * (hi - 1) / 2 + lo
+                                : kRegD3 + 3 - __builtin_ctz(~(unsigned)regs));
+      for (int x = 0; x < (1 << op.k); ++x) {
+        int idx = 0;
+        for (int m = 0; m < op.k; ++m)
+          if ((x >> (op.k - 1 - m)) & 1) idx |= 1 << (op.k - 1 - order[m]);
+        coef.push_back(op.coef[2 * idx]);
+        coef.push_back(op.coef[2 * idx + 1]);
+      }
+      ops.push_back(o);
     }
-    if (__builtin_popcount(cur | m) > 4) {
-      close(i);
-      pb = i;
-      cur = 0;
-    }
-    cur |= m;
   }
-  close(end);
+  if (!segs.empty() && !whole_lines(segs.back().pos)) remap(top);
+  end_chunk();
+  auto where = [&](uint32_t packed) {
+    uint32_t w = 0;
+    for (int k = 0; k < R; ++k) w |= (uint32_t)r.tbits[(packed >> (4 * k)) & 15u] << (8 * k);
+    return w;
+  };
+  fr->where_in = where(fr->map0);
+  fr->where_out = where(map);
+}
+
+// Builds and uploads the register form of R bits of the planned runs.
+qtnh_status build_form(qtnh_ctx_t ctx, qtnh_circuit_s &c, int R) {
+  std::vector<RegOp> ops;
+  std::vector<RegChunk> chunks;
+  std::vector<double> coef;
+  auto &f = c.forms[R];
+  for (const auto &r : c.runs) {
+    qtnh_circuit_s::RegForm::Run fr;
+    fr.chunk_begin = (uint32_t)chunks.size();
+    plan_reg_run(c, r, R, ops, coef, chunks, &fr);
+    fr.chunk_end = (uint32_t)chunks.size();
+    f.runs.push_back(fr);
+  }
+  auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t ob = pad(ops.size() * sizeof(RegOp)), cb = pad(chunks.size() * sizeof(RegChunk)),
+               fb = coef.size() * sizeof(double);
+  std::vector<char> host(ob + cb + fb + 16);
+  if (!ops.empty()) memcpy(host.data(), ops.data(), ops.size() * sizeof(RegOp));
+  if (!chunks.empty()) memcpy(host.data() + ob, chunks.data(), chunks.size() * sizeof(RegChunk));
+  if (!coef.empty()) memcpy(host.data() + ob + cb, coef.data(), fb);
+  qtnh_status st = check_hip(ctx, hipMalloc(&f.dev, host.size()), "circuit form alloc");
+  if (st) return st;
+  f.ops = (const RegOp *)f.dev;
+  f.chunks = (const RegChunk *)((char *)f.dev + ob);
+  f.coef = (const double2_t *)((char *)f.dev + ob + cb);
+  return check_hip(ctx, hipMemcpyAsync(f.dev, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream),
+                   "circuit form upload");
 }
 
 // Tile shape for an n-qubit circuit: the autotuned one of this context, else the process default.
 void tile_shape(qtnh_ctx_t ctx, int n, int *tb, int *low) {
   const bool tuned = n < 64 && ctx->circ_tb[n] > 0;
-  *tb = tuned ? ctx->circ_tb[n] : g_tile_bits;
-  *low = tuned ? ctx->circ_low[n] : g_low_bits;
+  default_tile(n, tb, low);
+  if (!tuned) return;
+  *tb = ctx->circ_tb[n];
+  *low = ctx->circ_low[n];
 }
 
 qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
@@ -1056,6 +1352,8 @@ qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
     }
   }
   plan_runs(c, tb, low);
+  c.has3 = false;
+  for (const auto &op : c.ops) c.has3 = c.has3 || (op.kind == 0 && op.k == 3);
   std::vector<TileOp> tops(std::max<size_t>(c.ops.size(), 1));
   std::vector<double> coef;
   for (const auto &r : c.runs) {
@@ -1104,23 +1402,7 @@ qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
     }
   }
   if (coef.empty()) coef.assign(2, 0.0);
-  std::vector<PhaseDesc> phases;
-  c.run_phases.clear();
-  for (const auto &r : c.runs) {
-    const uint32_t p0 = (uint32_t)phases.size();
-    if (r.tbits.size() == 12) plan_phases(tops, r.begin, r.end, phases);
-    c.run_phases.push_back({p0, (uint32_t)phases.size()});
-  }
-  for (const auto &ph : phases)
-    for (uint32_t i = ph.op_begin; !ph.lds && i < ph.op_end; ++i)
-      if (!reg_code_ok(tops[i].rcode)) return set_error(ctx, QTNH_EINVAL, "circuit: register op form (planner)");
-  if (phases.empty()) phases.resize(1);
   qtnh_status st = check_hip(ctx, hipMalloc((void **)&c.d_ops, tops.size() * sizeof(TileOp)), "circuit alloc");
-  if (!st) st = check_hip(ctx, hipMalloc((void **)&c.d_phases, phases.size() * sizeof(PhaseDesc)), "circuit alloc");
-  if (!st)
-    st = check_hip(ctx, hipMemcpyAsync(c.d_phases, phases.data(), phases.size() * sizeof(PhaseDesc),
-                                       hipMemcpyHostToDevice, ctx->stream),
-                   "circuit upload");
   if (!st) st = check_hip(ctx, hipMalloc((void **)&c.d_coef, coef.size() * sizeof(double)), "circuit alloc");
   if (!st)
     st = check_hip(ctx, hipMemcpyAsync(c.d_ops, tops.data(), tops.size() * sizeof(TileOp), hipMemcpyHostToDevice,
@@ -1130,14 +1412,19 @@ qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
     st = check_hip(ctx, hipMemcpyAsync(c.d_coef, coef.data(), coef.size() * sizeof(double), hipMemcpyHostToDevice,
                                        ctx->stream),
                    "circuit upload");
+  for (int R = kMinRegBits; R <= kMaxRegBits && !st; ++R)
+    if (wants_form(c, std::min(tb, c.n), R)) st = build_form(ctx, c, R);
   if (st) {
     // Only this attempt's buffers: no launch has used them (retired forms stay).
     (void)hipStreamSynchronize(ctx->stream);
-    for (void *p : {(void *)c.d_ops, (void *)c.d_coef, (void *)c.d_phases})
+    for (void *p : {(void *)c.d_ops, (void *)c.d_coef})
       if (p) (void)hipFree(p);
+    for (auto &f : c.forms) {
+      if (f.dev) (void)hipFree(f.dev);
+      f = qtnh_circuit_s::RegForm{};
+    }
     c.d_ops = nullptr;
     c.d_coef = nullptr;
-    c.d_phases = nullptr;
     c.compiled_tb = -1;
     return st;
   }
@@ -1148,13 +1435,23 @@ qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
   return QTNH_OK;
 }
 
-RunDesc make_desc(const qtnh_circuit_s &c, size_t ri, c128 *psi, uint64_t first) {
+// Descriptor of run ri on psi, with its register form of R bits (0: none).
+RunDesc make_desc(const qtnh_circuit_s &c, size_t ri, c128 *psi, uint64_t first, int R) {
   const qtnh_circuit_s::Run &r = c.runs[ri];
   RunDesc d;
   memset(&d, 0, sizeof(d));
-  d.phases = c.d_phases;
-  d.ph_begin = c.run_phases[ri].first;
-  d.ph_end = c.run_phases[ri].second;
+  if (R) {
+    const auto &f = c.forms[R];
+    d.rops = f.ops;
+    d.rcoef = f.coef;
+    d.rchunks = f.chunks;
+    d.chunk_begin = f.runs[ri].chunk_begin;
+    d.chunk_end = f.runs[ri].chunk_end;
+    d.map0 = f.runs[ri].map0;
+    d.where_in = f.runs[ri].where_in;
+    d.where_out = f.runs[ri].where_out;
+    d.rbits = R;
+  }
   d.ops = c.d_ops;
   d.coef = c.d_coef;
   d.psi = (double2_t *)psi;
@@ -1174,6 +1471,53 @@ RunDesc make_desc(const qtnh_circuit_s &c, size_t ri, c128 *psi, uint64_t first)
 
 uint64_t desc_tiles(const RunDesc &d) { return 1ull << d.n_outer; }
 
+// Run ri of circuit c on psi, one of a launch's runs.
+struct RunRef {
+  const qtnh_circuit_s *c;
+  size_t ri;
+  c128 *psi;
+};
+
+// Appends one launch's descriptors.  All runs of a launch take register forms
+// of one width: the width these tiles want, where every circuit has built it,
+// else the widest.
+void add_group(const std::vector<RunRef> &refs, std::vector<RunDesc> &descs, std::vector<size_t> &starts) {
+  starts.push_back(descs.size());
+  int tb_max = 0;
+  bool has3 = false;
+  for (const RunRef &r : refs) {
+    tb_max = std::max(tb_max, (int)r.c->runs[r.ri].tbits.size());
+    has3 = has3 || r.c->has3;
+  }
+  int R = reg_bits(tb_max, has3);
+  for (const RunRef &r : refs)
+    if (!r.c->forms[R].dev) {
+      R = kMaxRegBits;
+      break;
+    }
+  for (const RunRef &r : refs)
+    if (!r.c->forms[R].dev) {
+      R = 0;
+      break;
+    }
+  uint64_t first = 0;
+  for (const RunRef &r : refs) {
+    descs.push_back(make_desc(*r.c, r.ri, r.psi, first, R));
+    descs.back().has3 = has3;
+    first += desc_tiles(descs.back());
+  }
+}
+
+// One workgroup per tile (a grid of resident workgroups walking the tiles ran
+// 10% longer at 28 qubits: its workgroups stay in step, all loading at a time).
+template <int R, int KD, int MINW>
+void launch_reg(qtnh_ctx_t ctx, const RunDesc *d, int nr, uint64_t total, int tb) {
+  const unsigned threads = std::max(64, 1 << (tb - R));
+  const unsigned blocks = (unsigned)std::min<uint64_t>(total, 1u << 30);
+  const size_t lds = (sizeof(double) << tb) + kRegCoef * sizeof(double2_t) + (kRegOps + 2) * sizeof(RegOp);
+  hipLaunchKernelGGL((circuit_reg_kernel<R, KD, MINW>), dim3(blocks), dim3(threads), lds, ctx->stream, d, nr, total, tb);
+}
+
 // Launches groups of runs: group g covers descs [starts[g], starts[g+1]), one
 // launch each, in order.  The descriptors go to the device in one copy.
 // Launches the run groups [starts[g], starts[g+1]) of descriptors already on
@@ -1192,20 +1536,16 @@ qtnh_status launch_groups(qtnh_ctx_t ctx, const RunDesc *dd, const std::vector<R
     }
     const int nr = (int)(e - b);
     bool all12 = true;
-    for (size_t i = b; i < e; ++i) all12 = all12 && descs[i].tb == kPipeTB && descs[i].ph_end > descs[i].ph_begin;
-    if (all12 && total >= 2ull * ctx->num_cus && g_circuit_mode == 3) {
-      const unsigned rbk = (unsigned)std::min<uint64_t>(total, (uint64_t)ctx->num_cus * 2);
-      hipLaunchKernelGGL(circuit_rbp_kernel, dim3(rbk), dim3(256), 0, ctx->stream, dd + b, nr, total);
-      st = check_hip(ctx, hipGetLastError(), "circuit pipelined register-blocked launch");
-      if (st) return st;
-      continue;
-    }
-    // Register-blocked for any number of tiles: one barrier per phase instead of
-    // one per op also shortens single-tile runs (QFT-12: 90 us instead of 115).
-    if (all12 && g_circuit_mode == 2) {
-      const unsigned rbk = (unsigned)std::min<uint64_t>(total, (uint64_t)ctx->num_cus * 2);
-      hipLaunchKernelGGL(circuit_rb_kernel, dim3(rbk), dim3(256), 0, ctx->stream, dd + b, nr, total);
-      st = check_hip(ctx, hipGetLastError(), "circuit register-blocked launch");
+    for (size_t i = b; i < e; ++i) all12 = all12 && descs[i].tb == kPipeTB;
+    if (descs[b].rbits && g_circuit_mode >= 2) {
+      const bool g3 = descs[b].has3 != 0;
+      if (descs[b].rbits == 2)
+        launch_reg<2, 2, 4>(ctx, dd + b, nr, total, tbmax);
+      else if (descs[b].rbits == 3)
+        g3 ? launch_reg<3, 3, 4>(ctx, dd + b, nr, total, tbmax) : launch_reg<3, 2, 4>(ctx, dd + b, nr, total, tbmax);
+      else
+        g3 ? launch_reg<4, 3, 3>(ctx, dd + b, nr, total, tbmax) : launch_reg<4, 2, 4>(ctx, dd + b, nr, total, tbmax);
+      st = check_hip(ctx, hipGetLastError(), "circuit register launch");
       if (st) return st;
       continue;
     }
@@ -1271,8 +1611,7 @@ qtnh_status run_fused(qtnh_ctx_t ctx, qtnh_circuit_s &c, c128 *psi) {
                      "(run it once on the state before capturing)");
   qtnh_circuit_s::DescCache dc;
   for (size_t ri = 0; ri < c.runs.size(); ++ri) {
-    dc.starts.push_back(dc.h.size());
-    dc.h.push_back(make_desc(c, ri, psi, 0));
+    add_group({RunRef{&c, ri, psi}}, dc.h, dc.starts);
   }
   dc.starts.push_back(dc.h.size());
   if (dc.h.empty()) return QTNH_OK;
@@ -1410,14 +1749,10 @@ qtnh_status circuit_advance(qtnh_ctx_t ctx, int count, const qtnh_circuit_t *cs,
   std::vector<RunDesc> descs;
   std::vector<size_t> starts;
   for (int k = 0; k < kmax; ++k) {
-    starts.push_back(descs.size());
-    uint64_t first = 0;
-    for (int i = 0; i < count; ++i) {
-      if (k >= nrun[i]) continue;
-      RunDesc d = make_desc(*cs[i], (size_t)(first_run[i] + k), (c128 *)states[i], first);
-      first += desc_tiles(d);
-      descs.push_back(d);
-    }
+    std::vector<RunRef> refs;
+    for (int i = 0; i < count; ++i)
+      if (k < nrun[i]) refs.push_back(RunRef{cs[i], (size_t)(first_run[i] + k), (c128 *)states[i]});
+    add_group(refs, descs, starts);
   }
   starts.push_back(descs.size());
   return launch_run_groups(ctx, descs, starts);
@@ -1575,7 +1910,9 @@ qtnh_status qtnh_circuit_info(qtnh_circuit_t c, int *n_qubits, uint64_t *n_ops, 
     qtnh_circuit_s tmp;
     tmp.n = c->n;
     tmp.ops = c->ops;
-    plan_runs(tmp, c->tuned_tb > 0 ? c->tuned_tb : g_tile_bits, c->tuned_tb > 0 ? c->tuned_low : g_low_bits);
+    int tb = c->tuned_tb, low = c->tuned_low;
+    if (tb <= 0) default_tile(c->n, &tb, &low);
+    plan_runs(tmp, tb, low);
     *n_runs = tmp.runs.size();
   }
   return QTNH_OK;
@@ -1618,14 +1955,10 @@ qtnh_status qtnh_circuit_run_batch(qtnh_ctx_t ctx, int count, const qtnh_circuit
   std::vector<RunDesc> descs;
   std::vector<size_t> starts;
   for (size_t s = 0; s < steps; ++s) {
-    starts.push_back(descs.size());
-    uint64_t first = 0;
-    for (int i = 0; i < count; ++i) {
-      if (s >= cs[i]->runs.size()) continue;
-      RunDesc d = make_desc(*cs[i], s, (c128 *)states[i], first);
-      first += desc_tiles(d);
-      descs.push_back(d);
-    }
+    std::vector<RunRef> refs;
+    for (int i = 0; i < count; ++i)
+      if (s < cs[i]->runs.size()) refs.push_back(RunRef{cs[i], s, (c128 *)states[i]});
+    add_group(refs, descs, starts);
   }
   starts.push_back(descs.size());
   return launch_run_groups(ctx, descs, starts);
@@ -1697,7 +2030,8 @@ qtnh_status qtnh_autotune_circuit(qtnh_ctx_t ctx, int n_qubits, int *tile_bits, 
   st = check_hip(ctx, hipEventCreate(&e0), "autotune event");
   if (!st) st = check_hip(ctx, hipEventCreate(&e1), "autotune event");
   double best = 1e30;
-  int btb = g_tile_bits, blow = g_low_bits;
+  int btb, blow;
+  default_tile(np, &btb, &blow);
   for (const auto &cd : cand) {
     if (st) break;
     if (cd[0] > std::max(np, 10)) continue;

@@ -225,3 +225,51 @@ def test_circuit_tune_keeps_results(kind, n):
     got = dev(x)
     c.run(got, _lib.RUN_FUSED)
     assert same_bits(host(got), host(want))
+
+
+def _mixed_circuit(n, n_ops, dense3, seed):
+    """Random ops of every form: dense gates of 1, 2 (both qubit orders) and
+    optionally 3 qubits, diagonals of 1-3, all with unequal coefficients."""
+    rng = np.random.default_rng(seed)
+    c = ops.Circuit(n)
+    for _ in range(n_ops):
+        k = int(rng.integers(1, min(n, 3) + 1))
+        q = [int(v) for v in rng.choice(n, k, replace=False)]
+        if rng.random() < 0.5 and (k < 3 or dense3):
+            c.gate(q, (rng.standard_normal(1 << 2 * k) + 1j * rng.standard_normal(1 << 2 * k)) / (1 << k))
+        else:
+            c.diag(q, np.exp(1j * rng.standard_normal(1 << k)))
+    return c
+
+
+@pytest.mark.parametrize("dense3", [False, True])
+@pytest.mark.parametrize("n,tb,low", [(4, 4, 4), (5, 12, 4), (8, 6, 2), (9, 9, 3), (11, 10, 3), (13, 11, 3),
+                                      (12, 12, 4), (14, 12, 0), (15, 7, 4)])
+def test_register_runs_bitexact(n, tb, low, dense3):
+    """Every width of the register form (2 to 4 register bits; the smallest and
+    largest tiles; tiles of less than a wave), with more ops than one staged
+    chunk holds and gates on the lowest bits, where the state cannot be read
+    under the first gates' register bits."""
+    c = _mixed_circuit(n, 130, dense3, 100 * n + tb)
+    x = rnd_state(n, n)
+    ref = oracle_run(c, x)
+    ops.tune_circuit(tb, low)
+    try:
+        s = dev(x)
+        c.run(s)
+        assert same_bits(host(s), ref), (n, tb, low, dense3)
+    finally:
+        ops.tune_circuit(12)
+
+
+@pytest.mark.parametrize("dense3", [False, True])
+def test_register_runs_of_several_widths_in_one_launch(dense3):
+    """A batch whose circuits want different register bits and tile sizes."""
+    sizes = [4, 7, 10, 11, 13, 16]
+    cs = [_mixed_circuit(n, 60, dense3 and n == 11, n) for n in sizes]
+    xs = [rnd_state(n, 50 + n) for n in sizes]
+    refs = [oracle_run(c, x) for c, x in zip(cs, xs)]
+    states = [dev(x) for x in xs]
+    ops.run_batch(cs, states)
+    for n, s, ref in zip(sizes, states, refs):
+        assert same_bits(host(s), ref), n
