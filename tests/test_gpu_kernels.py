@@ -170,6 +170,33 @@ def test_permute_bitexact(case):
     assert same_bits(host(y), oracle.permute(x, dims, p))
 
 
+def _ragged_cases():
+    rng = np.random.default_rng(15)
+    cases = [([63, 65], [1, 0]), ([64, 129], [1, 0]), ([127, 3, 62], [2, 1, 0]), ([5000, 3], [1, 0]),
+             ([3, 4097], [1, 0]), ([2, 3, 2, 5, 2, 7, 2, 3], [7, 5, 3, 1, 6, 4, 2, 0]), ([3] * 11, None),
+             ([17, 1, 16, 9, 1], [3, 4, 0, 2, 1]), ([40, 30, 16], [1, 0, 2]), ([40, 30, 15], [1, 0, 2]),
+             ([7, 11, 13, 2], [2, 0, 1, 3]), ([1, 6, 1], [2, 1, 0]), ([48, 35, 21, 22, 18], [4, 1, 3, 0, 2]),
+             ([200, 300, 11], [2, 1, 0]), ([6, 0, 5], [2, 0, 1])]
+    for i in range(24):
+        r = int(rng.integers(2, 8))
+        d = [int(v) for v in rng.integers(1, [3, 12, 40][i % 3], r)]
+        while np.prod(d) > 2000000:
+            d[int(np.argmax(d))] //= 2
+        cases.append((d, [int(v) for v in rng.permutation(r)]))
+    return [(d, p if p else [int(v) for v in rng.permutation(len(d))]) for d, p in cases]
+
+
+@pytest.mark.parametrize("case", _ragged_cases(), ids=lambda c: "x".join(map(str, c[0])))
+def test_permute_ragged_bitexact(case):
+    """Dims that are no powers of two: cut axes with and without remainders,
+    tiles from one element run to the largest, dims of 1 and 0, merged axes,
+    inner axes kept (above and below the gather's line) and moved."""
+    dims, ptup = case
+    x = rnd(int(np.prod(dims)), len(dims))
+    got = host(ops.permute(dev(x), dims, ptup))
+    assert same_bits(got, oracle.permute(x, dims, ptup))
+
+
 def test_permute_roundtrip_rank24():
     dims = [2] * 24
     p = list(range(24))
