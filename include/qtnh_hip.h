@@ -393,8 +393,8 @@ void qtnh_tune_permute(int a, int b, int u_target, int order, int nt, int blocks
  * restores the default tile and clears the tuned shapes; 0 uses the set tile
  * for every permutation.  Results do not depend on it. */
 void qtnh_tune_permute_auto(int on);
-/* Block width (64 or 128 complex columns, 0: chosen by size) of the FP64
- * complex GEMM. */
+/* Tiles of the FP64 complex GEMM: 0 (default) 64 x 64, 32 x 64 or 32 x 32 by
+ * size, 64 always 64 x 64; 128 is accepted and runs as 64. */
 void qtnh_tune_zgemm(int bn);
 /* Number of 8-bit slices (1..8, default 5) of QTNH_PREC_SPLIT contractions. */
 void qtnh_tune_split(int slices);

@@ -715,11 +715,15 @@ ContractRoute contract_route(int rA, const uint64_t *dA, int rB, const uint64_t 
   R.N = P.N;
   R.K = P.K;
   R.direct = use_direct(P);
-  R.ws_bytes = 0;
+  R.ws_bytes = R.limit_bytes = 0;
   if (!R.direct) {
     GemmRoute L;
     gemm_layout(P, dA, dB, precision, L);
-    R.ws_bytes = L.bytes;
+    R.ws_bytes = R.limit_bytes = L.bytes;
+    // A fixed workspace takes a shape if the chunks of its size class fit, also
+    // where it runs with fewer: the limit does not move with the tiles.
+    const uint64_t large = L.split || L.splitk ? 1 : zgemm_chunks_large(P.M, P.N, P.K);
+    if (large > 1) R.limit_bytes = std::max(L.bytes, L.bytes - L.sbytes + pad_c128(P.M * P.N * large));
   }
   return R;
 }

@@ -123,6 +123,7 @@ qtnh_status launch_contract(qtnh_ctx_t ctx, const c128 *A, int rA, const uint64_
 struct ContractRoute {
   bool direct;
   uint64_t M, N, K, ws_bytes;
+  uint64_t limit_bytes;  // what a fixed workspace is compared with (at least ws_bytes)
 };
 ContractRoute contract_route(int rA, const uint64_t *dA, int rB, const uint64_t *dB, int nw, const uint16_t *wires,
                              const uint16_t *repl1, const uint16_t *repl2, int precision);
@@ -168,6 +169,8 @@ qtnh_status launch_zgemm_f64(qtnh_ctx_t ctx, const c128 *A, const c128 *B, c128 
 // Depth chunks launch_zgemm_f64 uses for this shape (1: none); with more than
 // one it needs `partials` of chunks * M * N elements.
 uint64_t zgemm_chunks(uint64_t M, uint64_t N, uint64_t K);
+// Most chunks of a shape whose operands and partials are large.
+uint64_t zgemm_chunks_large(uint64_t M, uint64_t N, uint64_t K);
 
 // C[MxN] = A[MxK] * Bt[NxK]^T for few outputs: each sum in `chunks` ordered
 // chunks over separate workgroups (partials: M*N*chunks elements), then summed
@@ -178,7 +181,7 @@ qtnh_status launch_zgemm_splitk(qtnh_ctx_t ctx, const c128 *A, const c128 *Bt, c
 // ---- grouped launches: many independent problems in one launch, each a
 // contiguous range of blocks starting at `first` (descriptors sorted by it).
 // One GEMM of launch_zgemm_grouped: C[MxN] = A[MxK] * B[KxN], all contiguous
-// row-major; `tiles` output tiles (64 x block width) times the depth chunks of
+// row-major; `tiles` square output tiles of the launch's edge times the depth chunks of
 // zgemm_chunk_shape (chunk c sums k in [c kc, (c + 1) kc) into C + c cstride).
 struct ZGroupDesc {
   const c128 *A;
@@ -212,13 +215,14 @@ struct PermDesc {
   int nb;
   int8_t sbit[64];
 };
-qtnh_status launch_zgemm_grouped(qtnh_ctx_t ctx, int bn, const ZGroupDesc *d, int nd, uint64_t total_blocks);
+qtnh_status launch_zgemm_grouped(qtnh_ctx_t ctx, int tile, const ZGroupDesc *d, int nd, uint64_t total_blocks);
 qtnh_status launch_zgemm_grouped_sum(qtnh_ctx_t ctx, const ZSumDesc *d, int nd, uint64_t total_blocks);
 qtnh_status launch_splitk_grouped(qtnh_ctx_t ctx, const SkDesc *d, int nd, uint64_t total_partial,
                                   uint64_t total_final);
 qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, uint64_t total_blocks);
-// Block width (64 or 128) and depth chunks (length on BK steps, count) of launch_zgemm_f64.
-int zgemm_block_n(uint64_t M, uint64_t N);
+// Tile edge (32 or 64) of a shape in grouped launches, and the depth chunks
+// (length on BK steps, count) of launch_zgemm_f64, which they share.
+int zgemm_group_tile(uint64_t M, uint64_t N);
 void zgemm_chunk_shape(uint64_t M, uint64_t N, uint64_t K, uint64_t *kc, uint64_t *nchunks);
 // Terms per chunk of the split-K route (a multiple of its workgroup size).
 uint64_t splitk_chunk_len(uint64_t K, uint64_t chunks);

@@ -947,7 +947,7 @@ struct Wave {
   std::vector<std::vector<char>> grouped;  // [network][step]
   std::vector<std::vector<int>> singles;   // [step index]: networks whose step runs alone
   std::vector<PermDesc> pin, pout;
-  std::vector<ZGroupDesc> zg[2];  // block width 64, 128
+  std::vector<ZGroupDesc> zg[2];  // tiles of 32 x 32, 64 x 64
   std::vector<ZSumDesc> zsum;
   std::vector<SkDesc> sk;
   std::vector<GRange> r_pin, r_pout, r_zg[2], r_zsum, r_sk;
@@ -1146,8 +1146,8 @@ struct Wave {
           sk.push_back(d);
           r_sk[s].e = (uint32_t)sk.size();
         } else {
-          const int bi = zgemm_block_n(R.M, R.N) == 128 ? 1 : 0;
-          const uint64_t bn = bi ? 128 : 64;
+          const uint64_t edge = zgemm_group_tile(R.M, R.N);
+          const int bi = edge == 64 ? 1 : 0;
           uint64_t kc = 0, nch = 1;
           zgemm_chunk_shape(R.M, R.N, R.K, &kc, &nch);
           ZGroupDesc d;
@@ -1159,7 +1159,7 @@ struct Wave {
           d.K = R.K;
           d.kc = kc;
           d.cstride = nch > 1 ? R.M * R.N : 0;
-          d.tiles = ((R.N + bn - 1) / bn) * ((R.M + 63) / 64);
+          d.tiles = ((R.N + edge - 1) / edge) * ((R.M + edge - 1) / edge);
           d.first = r_zg[bi][s].blocks;
           r_zg[bi][s].blocks += d.tiles * nch;
           zg[bi].push_back(d);
@@ -1301,7 +1301,7 @@ struct Wave {
     if (a.e > a.b) st = launch_permute_grouped(ctx, d_pin + a.b, (int)(a.e - a.b), a.blocks);
     for (int bi = 0; bi < 2 && !st; ++bi) {
       const GRange &z = r_zg[bi][s];
-      if (z.e > z.b) st = launch_zgemm_grouped(ctx, bi ? 128 : 64, d_zg[bi] + z.b, (int)(z.e - z.b), z.blocks);
+      if (z.e > z.b) st = launch_zgemm_grouped(ctx, bi ? 64 : 32, d_zg[bi] + z.b, (int)(z.e - z.b), z.blocks);
     }
     const GRange &c = r_zsum[s];
     if (!st && c.e > c.b) st = launch_zgemm_grouped_sum(ctx, d_zsum + c.b, (int)(c.e - c.b), c.blocks);

@@ -70,11 +70,11 @@ qtnh_status qtnh_contract_c128_noalloc(qtnh_ctx_t ctx, const void *A, int rA, co
   if (st || !nC) return st;
   const qtnh_hip::ContractRoute R =
       qtnh_hip::contract_route(rA, dA, rB, dB, nw, wires, repl1, repl2, precision);
-  if (R.ws_bytes > kScratchBytes)
+  if (R.limit_bytes > kScratchBytes)
     return qtnh_hip::set_error(ctx, QTNH_EINVAL,
                                "contract_noalloc: this contraction needs %llu bytes of workspace; the static "
                                "scratch holds %llu (use qtnh_contract_c128)",
-                               (unsigned long long)R.ws_bytes, (unsigned long long)kScratchBytes);
+                               (unsigned long long)R.limit_bytes, (unsigned long long)kScratchBytes);
   st = qtnh_hip::enter_ctx(ctx);
   if (st) return st;
   void *ws = nullptr;

@@ -3,12 +3,14 @@
 //
 // Each 16x16 complex output tile keeps a real and an imaginary accumulator
 // and takes four v_mfma_f64_16x16x4_f64 per 4-deep k step:
-//   Cr += Ar*Br, Cr += (-Ai)*Bi, Ci += Ar*Bi, Ci += Ai*Br.
-// A workgroup of 4 waves owns a BM x BN complex tile, each wave a 32 x (BN/2)
-// sub-tile (2 x BN/32 MFMA tiles).  Operands are staged through LDS BK complex
-// deep; the global loads of stage s+1 are issued into registers before the
-// MFMAs of stage s, so memory latency hides behind the (slow, 64-cycle) f64
-// MFMAs.
+//   Cr += Ar*Br, Ci += Ar*Bi, Cr += (-Ai)*Bi, Ci += Ai*Br.
+// A workgroup of 2 x 2 waves owns a BM x BN complex tile.  Operands are staged
+// through two LDS buffers BK complex deep: the loads of stage s + 1 are issued
+// into registers before the MFMAs of stage s and written to the other buffer
+// between them, so that a stage costs one barrier and the matrix cores (64
+// cycles per f64 MFMA) wait for little else.  Every kFold terms the
+// accumulators are added into a second set: sums of partial sums, whose error
+// does not grow with the depth as one long sum's does.
 #include <algorithm>
 
 #include "internal.hpp"
@@ -22,110 +24,184 @@ typedef double double2_t __attribute__((ext_vector_type(2)));
 constexpr int BK = 16;
 constexpr int kThreads = 256;
 
+constexpr int kFold = 256;  // terms per accumulator set
+
 template <int BM, int BN>
 struct ZTile {
   static constexpr int LDA = BK + 1;  // padded LDS rows (complex elements)
   static constexpr int LDB = BN + 1;
-  static constexpr int A_PER = BM * BK / kThreads;  // complex loads per thread per stage
+  static constexpr int kA = BM * LDA, kBuf = kA + BK * LDB;  // one stage's LDS elements
+  static constexpr int A_PER = BM * BK / kThreads;            // complex loads per thread per stage
   static constexpr int B_PER = BK * BN / kThreads;
-  static constexpr int WN = BN / 2;                 // wave tile: 32 x WN
-  static constexpr int TN = WN / 16;                // MFMA tiles along n per wave
-  static_assert(BM == 64, "two waves of 32 rows");
-  static_assert(A_PER >= 1 && B_PER >= 1, "tile too small");
+  static constexpr int TM = BM / 32, TN = BN / 32;  // MFMA tiles per wave
+  static_assert(A_PER >= 1 && B_PER >= 1 && TM >= 1 && TN >= 1, "tile too small");
 };
 
-// One BM x BN output tile `tile` (row-major over the tile grid) of
-// C = A * B over depth chunk `chunk` (k in [chunk kc, (chunk + 1) kc)), written
-// to C + chunk cstride.  As / Bs: the workgroup's LDS staging buffers.
+// Compile-time flags of a stage.
+struct No {
+  static constexpr bool value = false;
+};
+struct Yes {
+  static constexpr bool value = true;
+};
+
+// The BM x BN output tile at (m0, n0) of C = A * B over k in [kb, ke), written
+// to C.  lds: the workgroup's 2 kBuf staging elements.
 template <int BM, int BN>
 __device__ __forceinline__ void zgemm_tile(const c128 *__restrict__ A, const c128 *__restrict__ B,
-                                           c128 *__restrict__ C, uint64_t M, uint64_t N, uint64_t K, uint64_t lda,
-                                           uint64_t ldb, uint64_t ldc, uint64_t kc, uint64_t cstride, uint64_t tile,
-                                           uint64_t chunk, double2_t *As, double2_t *Bs) {
+                                           c128 *__restrict__ C, uint64_t M, uint64_t N, uint64_t lda, uint64_t ldb,
+                                           uint64_t ldc, uint64_t kb, uint64_t ke, uint64_t m0, uint64_t n0,
+                                           double2_t *lds) {
   using Z = ZTile<BM, BN>;
+  constexpr int TM = Z::TM, TN = Z::TN;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = (wave >> 1) * 32;  // wave tile origin inside the block tile
-  const int wn = (wave & 1) * Z::WN;
-  const uint64_t ntn = (N + BN - 1) / BN;
-  const uint64_t m0 = (tile / ntn) * BM;
-  const uint64_t n0 = (tile % ntn) * BN;
-  const uint64_t kb = chunk * kc;
-  const uint64_t ke = kb + kc < K ? kb + kc : K;
-  C += chunk * cstride;
+  const int wm = (wave >> 1) * (BM / 2);  // wave tile origin inside the block tile
+  const int wn = (wave & 1) * (BN / 2);
 
-  double4_t accR[2][Z::TN], accI[2][Z::TN];
+  double4_t accR[TM][TN], accI[TM][TN], sumR[TM][TN], sumI[TM][TN];
+  const double4_t zero4 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < Z::TN; ++j) {
-      accR[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-      accI[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-    }
+    for (int j = 0; j < TN; ++j) accR[i][j] = accI[i][j] = zero4;
 
-  const double2_t zero = {0.0, 0.0};
-  const double2_t *A2 = reinterpret_cast<const double2_t *>(A);
-  const double2_t *B2 = reinterpret_cast<const double2_t *>(B);
-  double2_t pa[Z::A_PER], pb[Z::B_PER];
-  auto fetch = [&](uint64_t k0) {
+  // Loads of a stage: A rows 16 apart and B rows kThreads / BN apart.  Rows and
+  // columns past the result's take the last one's values (their outputs are not
+  // stored); terms past the depth take the last one's address and become zeros
+  // on their way to LDS.
+  constexpr int kBStep = kThreads / BN, kLoads = Z::A_PER + Z::B_PER;
+  const int ar = tid / BK, ac = tid % BK, br = tid / BN, bc = tid % BN;
+  const double2_t *pa[Z::A_PER];
 #pragma unroll
-    for (int r = 0; r < Z::A_PER; ++r) {
-      const int idx = tid + r * kThreads;
-      const int ar = idx / BK, ac = idx % BK;
-      const uint64_t gm = m0 + ar, gk = k0 + ac;
-      pa[r] = (gm < M && gk < ke) ? A2[gm * lda + gk] : zero;
-    }
+  for (int r = 0; r < Z::A_PER; ++r) {
+    const uint64_t m = m0 + ar + r * 16;
+    pa[r] = reinterpret_cast<const double2_t *>(A) + (m < M ? m : M - 1) * lda;
+  }
+  const double2_t *pb = reinterpret_cast<const double2_t *>(B) + (n0 + bc < N ? n0 + bc : N - 1);
+  double2_t v[kLoads];
+  auto load = [&](int i, uint64_t k0, auto tail) {
+    uint64_t k = i < Z::A_PER ? k0 + ac : k0 + br + (i - Z::A_PER) * kBStep;
+    if (decltype(tail)::value) k = k < ke ? k : ke - 1;
+    v[i] = i < Z::A_PER ? pa[i < Z::A_PER ? i : 0][k] : pb[k * ldb];
+  };
+  auto put = [&](int i, double2_t *buf, uint64_t k0, auto tail) {
+    double2_t x = v[i];
+    if (decltype(tail)::value && (i < Z::A_PER ? k0 + ac : k0 + br + (i - Z::A_PER) * kBStep) >= ke)
+      x = double2_t{0.0, 0.0};
+    if (i < Z::A_PER)
+      buf[(ar + i * 16) * Z::LDA + ac] = x;
+    else
+      buf[Z::kA + (br + (i - Z::A_PER) * kBStep) * Z::LDB + bc] = x;
+  };
+  struct Frag {
+    double2_t x[TM + TN];  // A rows, then B columns
+  };
+  constexpr int kReads = TM + TN;
+  auto read = [&](Frag &f, int i, const double2_t *buf, int kk) {
+    const int kl = kk + (lane >> 4);
+    f.x[i] = i < TM ? buf[(wm + i * 16 + (lane & 15)) * Z::LDA + kl]
+                    : buf[Z::kA + kl * Z::LDB + wn + (i - TM) * 16 + (lane & 15)];
+  };
+  // The four products of a step; between(n) after the n-th MFMA: the memory
+  // work of the stage, a piece at a time, under the MFMAs (64 cycles each,
+  // issued in order: anything between two groups of them leaves the matrix
+  // core idle).  The last argument negates A.
+  constexpr int kMfma = 4 * TM * TN;
+  auto mma = [&](const Frag &f, auto between) {
 #pragma unroll
-    for (int r = 0; r < Z::B_PER; ++r) {
-      const int idx = tid + r * kThreads;
-      const int br = idx / BN, bc = idx % BN;
-      const uint64_t gk = k0 + br, gn = n0 + bc;
-      pb[r] = (gk < ke && gn < N) ? B2[gk * ldb + gn] : zero;
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const double2_t x = f.x[i], y = f.x[TM + j];
+          if (p == 0) accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.x, accR[i][j], 0, 0, 0);
+          if (p == 1) accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.y, accI[i][j], 0, 0, 0);
+          if (p == 2) accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.y, accR[i][j], 0, 0, 1);
+          if (p == 3) accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.x, accI[i][j], 0, 0, 0);
+          between((p * TM + i) * TN + j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+  };
+  // Pieces [0, count) dealt evenly over a step's MFMAs.
+  auto deal = [&](int n, int count, auto piece) {
+#pragma unroll
+    for (int q = 0; q < count; ++q)
+      if (q * kMfma / count == n) piece(q);
+  };
+  bool folded = false;
+  int cur = 0, until = kFold / BK;
+  Frag f0, f1;
+  // One stage at k0: each fragment step is read a step ahead; the next stage
+  // goes from registers to the other buffer (last read before the barrier of
+  // the stage before) and the one after it is requested in its place; the
+  // barrier comes before the last step, whose MFMAs cover the next stage's
+  // first read.  PUT / GET: there is such a stage; *_TAIL: it may be partial.
+  auto stage = [&](uint64_t k0, auto put_it, auto put_tail, auto get_it, auto get_tail) {
+    const double2_t *buf = lds + cur;
+    double2_t *next = lds + (Z::kBuf - cur);
+    mma(f0, [&](int n) { deal(n, kReads, [&](int q) { read(f1, q, buf, 4); }); });
+    mma(f1, [&](int n) { deal(n, kReads, [&](int q) { read(f0, q, buf, 8); }); });
+    mma(f0, [&](int n) {
+      deal(n, kReads, [&](int q) { read(f1, q, buf, 12); });
+      deal(n, kLoads, [&](int q) {
+        if (decltype(put_it)::value) put(q, next, k0 + BK, put_tail);
+        if (decltype(get_it)::value) load(q, k0 + 2 * BK, get_tail);
+      });
+    });
+    cur = Z::kBuf - cur;
+    if (decltype(put_it)::value) lds_barrier();
+    mma(f1, [&](int n) {
+      if (decltype(put_it)::value) deal(n, kReads, [&](int q) { read(f0, q, next, 0); });
+    });
+    if (--until == 0 && decltype(put_it)::value) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          sumR[i][j] = folded ? sumR[i][j] + accR[i][j] : accR[i][j];
+          sumI[i][j] = folded ? sumI[i][j] + accI[i][j] : accI[i][j];
+          accR[i][j] = accI[i][j] = zero4;
+        }
+      folded = true;
+      until = kFold / BK;
     }
   };
-  fetch(kb);
-  for (uint64_t k0 = kb; k0 < ke; k0 += BK) {
 #pragma unroll
-    for (int r = 0; r < Z::A_PER; ++r) {
-      const int idx = tid + r * kThreads;
-      As[(idx / BK) * Z::LDA + idx % BK] = pa[r];
-    }
+  for (int i = 0; i < kLoads; ++i) load(i, kb, Yes{});
 #pragma unroll
-    for (int r = 0; r < Z::B_PER; ++r) {
-      const int idx = tid + r * kThreads;
-      Bs[(idx / BN) * Z::LDB + idx % BN] = pb[r];
-    }
-    __syncthreads();
-    if (k0 + BK < ke) fetch(k0 + BK);  // in flight during the MFMAs below
+  for (int i = 0; i < kLoads; ++i) put(i, lds, kb, Yes{});
+  if (kb + BK < ke) {
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      const int kl = kk + (lane >> 4);
-      double2_t a[2], b[Z::TN];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = As[(wm + i * 16 + (lane & 15)) * Z::LDA + kl];
-#pragma unroll
-      for (int j = 0; j < Z::TN; ++j) b[j] = Bs[kl * Z::LDB + wn + j * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const double nai = -a[i].y;
-#pragma unroll
-        for (int j = 0; j < Z::TN; ++j) {
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, accR[i][j], 0, 0, 0);
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, b[j].y, accR[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].y, accI[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].x, accI[i][j], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
+    for (int i = 0; i < kLoads; ++i) load(i, kb + BK, Yes{});
   }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < kReads; ++i) read(f0, i, lds, 0);
+  uint64_t k0 = kb;
+  for (; k0 + 3 * BK <= ke; k0 += BK) stage(k0, Yes{}, No{}, Yes{}, No{});
+  if (k0 + 2 * BK < ke) {
+    stage(k0, Yes{}, No{}, Yes{}, Yes{});
+    k0 += BK;
+  }
+  if (k0 + BK < ke) {
+    stage(k0, Yes{}, Yes{}, No{}, No{});
+    k0 += BK;
+  }
+  stage(k0, No{}, No{}, No{}, No{});
+  lds_barrier();  // the buffers are free for another tile
   // Result layout of the 16x16 f64 MFMA (measured on gfx950): lane l holds
   // column l % 16 of rows l / 16 + 4 v, v = 0..3.
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < Z::TN; ++j)
+    for (int j = 0; j < TN; ++j) {
+      if (folded) {
+        accR[i][j] = sumR[i][j] + accR[i][j];
+        accI[i][j] = sumI[i][j] + accI[i][j];
+      }
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const uint64_t gm = m0 + wm + i * 16 + (lane >> 4) + 4 * v;
@@ -137,19 +213,33 @@ __device__ __forceinline__ void zgemm_tile(const c128 *__restrict__ A, const c12
           C[gm * ldc + gn] = out;
         }
       }
+    }
 }
 
-// blockIdx.x: output tile; blockIdx.y: depth chunk (one chunk: the whole
-// depth, into C; several: partial tiles at C + chunk cstride).
+// Workgroup blk of `total` as a position in the tile order: workgroups are
+// dealt to the 8 XCDs in turn, and XCD x takes the x-th stretch of the order,
+// so that the tiles that share operand rows and columns meet in one L2.
+__device__ __forceinline__ uint32_t xcd_order(uint32_t blk, uint32_t total) {
+  const uint32_t q = total >> 3, r = total & 7u, x = blk & 7u;
+  return x * q + (x < r ? x : r) + (blk >> 3);
+}
+
+// One BM x BN tile of one depth chunk per workgroup (chunk c: k in [c kc,
+// (c + 1) kc), written to C + c cstride).  Tiles in groups of 8 tile rows,
+// down each column of a group.
 template <int BM, int BN>
-__global__ void __launch_bounds__(kThreads) zgemm_f64_kernel(const c128 *__restrict__ A, const c128 *__restrict__ B,
+__global__ void __launch_bounds__(kThreads, 2) zgemm_f64_kernel(const c128 *__restrict__ A, const c128 *__restrict__ B,
                                                              c128 *__restrict__ C, uint64_t M, uint64_t N, uint64_t K,
                                                              uint64_t lda, uint64_t ldb, uint64_t ldc, uint64_t kc,
-                                                             uint64_t cstride) {
-  using Z = ZTile<BM, BN>;
-  __shared__ double2_t As[BM * Z::LDA];
-  __shared__ double2_t Bs[BK * Z::LDB];
-  zgemm_tile<BM, BN>(A, B, C, M, N, K, lda, ldb, ldc, kc, cstride, blockIdx.x, blockIdx.y, As, Bs);
+                                                             uint64_t cstride, uint32_t ntm, uint32_t ntn) {
+  __shared__ double2_t lds[2 * ZTile<BM, BN>::kBuf];
+  const uint32_t tiles = ntm * ntn, l = xcd_order(blockIdx.x, gridDim.x);
+  const uint32_t chunk = l / tiles, tile = l - chunk * tiles;
+  const uint32_t group = tile / (8 * ntn), rows = min(8u, ntm - 8 * group), in = tile - group * 8 * ntn;
+  const uint32_t tm = 8 * group + in % rows, tn = in / rows;
+  const uint64_t kb = chunk * kc, ke = kb + kc < K ? kb + kc : K;
+  zgemm_tile<BM, BN>(A, B, C + chunk * cstride, M, N, lda, ldb, ldc, kb, ke, (uint64_t)tm * BM, (uint64_t)tn * BN,
+                     lds);
 }
 
 // Index of the descriptor whose block range holds block blk (descriptors
@@ -169,17 +259,16 @@ __device__ __forceinline__ int find_desc(const D *__restrict__ d, int nd, uint64
 
 // Many GEMMs in one launch: each block of a grid-stride walk over every
 // GEMM's (chunk, tile) blocks computes one tile, exactly as zgemm_f64_kernel.
-template <int BN>
-__global__ void __launch_bounds__(kThreads) zgemm_grouped_kernel(const ZGroupDesc *__restrict__ d, int nd,
+template <int BM, int BN>
+__global__ void __launch_bounds__(kThreads, 2) zgemm_grouped_kernel(const ZGroupDesc *__restrict__ d, int nd,
                                                                  uint64_t total) {
-  using Z = ZTile<64, BN>;
-  __shared__ double2_t As[64 * Z::LDA];
-  __shared__ double2_t Bs[BK * Z::LDB];
+  __shared__ double2_t lds[2 * ZTile<BM, BN>::kBuf];
   for (uint64_t blk = blockIdx.x; blk < total; blk += gridDim.x) {
     const ZGroupDesc &D = d[find_desc(d, nd, blk)];
-    const uint64_t local = blk - D.first;
-    zgemm_tile<64, BN>(D.A, D.B, D.C, D.M, D.N, D.K, D.K, D.N, D.N, D.kc, D.cstride, local % D.tiles,
-                       local / D.tiles, As, Bs);
+    const uint64_t local = blk - D.first, chunk = local / D.tiles, tile = local % D.tiles;
+    const uint64_t ntn = (D.N + BN - 1) / BN, kb = chunk * D.kc, ke = kb + D.kc < D.K ? kb + D.kc : D.K;
+    zgemm_tile<BM, BN>(D.A, D.B, D.C + chunk * D.cstride, D.M, D.N, D.K, D.N, D.N, kb, ke, tile / ntn * BM,
+                       tile % ntn * BN, lds);
   }
 }
 
@@ -301,33 +390,70 @@ qtnh_status launch_zgemm_splitk(qtnh_ctx_t ctx, const c128 *A, const c128 *Bt, c
   return check_hip(ctx, hipGetLastError(), "splitk final launch");
 }
 
-// Block width: 0 picks by size (64 x 128 tiles run at occupancy 1 and win
-// while 64 x 64 tiles would number under 2048, about 8 per compute unit;
-// past that the occupancy-3 64 x 64 kernel hides latency better), or 64 / 128.
+// Block width asked for: 0 none, 64 or 128.
 static int g_zgemm_bn = 0;
 
 extern "C" void qtnh_tune_zgemm(int bn) { g_zgemm_bn = (bn == 64 || bn == 128) ? bn : 0; }
 
-// Depth chunks of a GEMM with few output tiles: enough chunks that tiles x
-// chunks reaches about kZgemmTargetBlocks workgroups, each summing at least
-// kZgemmMinChunk terms.  Depends on the shape only (the network planner sizes
-// workspaces with it), so every caller of a shape runs the same chunks.
-constexpr uint64_t kZgemmTargetBlocks = 1024, kZgemmMinChunk = 256;
-
-static int zgemm_bn(uint64_t M, uint64_t N) {
-  int bn = g_zgemm_bn;
-  if (bn == 0) bn = (((M + 63) / 64) * ((N + 63) / 64) < 2048) ? 128 : 64;
-  if (N < 128) bn = 64;
-  return bn;
-}
-
-uint64_t zgemm_chunks(uint64_t M, uint64_t N, uint64_t K) {
-  const int bn = zgemm_bn(M, N);
+// Most depth chunks of a shape whose operands are large: about 1024 tiles
+// times chunks of 64 x 128 tiles, 256 terms each.  (Their partials are
+// workspace that callers with a fixed one have to find room for.)
+uint64_t zgemm_chunks_large(uint64_t M, uint64_t N, uint64_t K) {
+  const uint64_t bn = (N < 128 || ((M + 63) / 64) * ((N + 63) / 64) >= 2048) ? 64 : 128;
   const uint64_t tiles = ((N + bn - 1) / bn) * ((M + 63) / 64);
-  if (tiles == 0 || tiles * 2 > kZgemmTargetBlocks || K < 2 * kZgemmMinChunk) return 1;
-  const uint64_t want = (kZgemmTargetBlocks + tiles - 1) / tiles;
-  return std::max<uint64_t>(1, std::min<uint64_t>(want, K / kZgemmMinChunk));
+  if (tiles == 0 || tiles * 2 > 1024 || K < 512) return 1;
+  return std::max<uint64_t>(1, std::min<uint64_t>((1024 + tiles - 1) / tiles, K / 256));
 }
+
+// Tile and depth chunks of a shape: the least estimated time over the tiles
+// and chunk counts, from measured rates: 5 us for a launch, its first loads and
+// its stores; a 16-deep stage of a 64 x 64 tile 1.9 us of a compute unit, of a
+// 32 x 64 tile 0.96, of a 32 x 32 tile 0.5 (1.0 and 0.6 where a compute unit
+// has only one); the second kernel that sums depth chunks 5.5 us and its
+// traffic.  A launch takes as long as the fullest of 256 compute units.
+// Depends on the shape only: the network planner sizes workspaces with it, and
+// every caller of a shape runs the same chunks.  (64 x 64 tiles or 64 x 128
+// ones alone, the rule before: 512^3 92 us, now 25 with 32 x 32 tiles; 256 x
+// 512 x 256 85 and 14; 700^3 107 and 57; 4096^3 8.10 and 7.74 ms.)
+struct ZShape {
+  int bm, bn;
+  uint64_t kc, chunks;
+};
+static ZShape zgemm_shape(uint64_t M, uint64_t N, uint64_t K) {
+  struct Tile {
+    int bm, bn;
+    double stage, alone;  // us per stage of a compute unit, and more where it has one workgroup
+  };
+  static const Tile kTiles[] = {{64, 64, 1.9, 0.0}, {32, 64, 0.96, 0.04}, {32, 32, 0.5, 0.1}};
+  // Up to here operands, result and partials fit the 64 MiB of the contraction without allocation.
+  const uint64_t room = (uint64_t)(60 << 20) / sizeof(c128);
+  const uint64_t large = zgemm_chunks_large(M, N, K), own = M * K + K * N + M * N;
+  ZShape best{64, 64, K, 1};
+  double t_best = 0.0;
+  for (const Tile &t : kTiles) {
+    if (g_zgemm_bn && t.bm != 64) continue;
+    const uint64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    uint64_t last = 0;
+    for (uint64_t want = 1; want <= 64; want += want < 4 ? 1 : want / 2) {
+      uint64_t kc = (K + want - 1) / want;
+      if (want > 1) kc = (kc + BK - 1) / BK * BK;
+      const uint64_t chunks = (K + kc - 1) / kc;
+      if (chunks > 1 && (kc < 64 || chunks == last)) continue;
+      if (chunks > large && own + chunks * M * N > room) continue;
+      last = chunks;
+      const double per = (double)((tiles * chunks + 255) / 256), stages = (double)((kc + BK - 1) / BK);
+      double us = 5.0 + stages * (per * t.stage + (per > 1 ? 0.0 : t.alone));
+      if (chunks > 1) us += 5.5 + (double)(M * N) * 16.0 * (double)(chunks + 1) / 4.5e6;
+      if (t_best == 0.0 || us < 0.97 * t_best) {
+        t_best = us;
+        best = ZShape{t.bm, t.bn, kc, chunks};
+      }
+    }
+  }
+  return best;
+}
+
+uint64_t zgemm_chunks(uint64_t M, uint64_t N, uint64_t K) { return zgemm_shape(M, N, K).chunks; }
 
 // C = sum over chunks of part[c] (M x N each), in chunk order.
 __global__ void zgemm_chunk_sum_kernel(const double2_t *__restrict__ part, double2_t *__restrict__ C, uint64_t M,
@@ -344,30 +470,32 @@ __global__ void zgemm_chunk_sum_kernel(const double2_t *__restrict__ part, doubl
   }
 }
 
+template <int BM, int BN>
+static void launch_tile_gemm(qtnh_ctx_t ctx, const c128 *A, const c128 *B, c128 *out, uint64_t M, uint64_t N,
+                             uint64_t K, uint64_t lda, uint64_t ldb, uint64_t ld, uint64_t cstride, const ZShape &z) {
+  const uint32_t ntm = (uint32_t)((M + BM - 1) / BM), ntn = (uint32_t)((N + BN - 1) / BN);
+  hipLaunchKernelGGL((zgemm_f64_kernel<BM, BN>), dim3((unsigned)(ntm * ntn * z.chunks)), dim3(kThreads), 0, ctx->stream,
+                     A, B, out, M, N, K, lda, ldb, ld, z.kc, cstride, ntm, ntn);
+}
+
 qtnh_status launch_zgemm_f64(qtnh_ctx_t ctx, const c128 *A, const c128 *B, c128 *C, uint64_t M, uint64_t N, uint64_t K,
                              uint64_t lda, uint64_t ldb, uint64_t ldc, c128 *partials) {
-  const int bn = zgemm_bn(M, N);
-  const uint64_t tiles = ((N + bn - 1) / bn) * ((M + 63) / 64);
-  if (tiles > 0x7fffffffull) return set_error(ctx, QTNH_EUNSUPPORTED, "zgemm: grid too large");
-  const uint64_t chunks = zgemm_chunks(M, N, K);
-  if (chunks > 1 && !partials) return set_error(ctx, QTNH_EINVAL, "zgemm: depth chunks need a partial buffer");
-  const uint64_t kc = chunks > 1 ? (K + chunks - 1) / chunks : K;
-  const uint64_t kcr = chunks > 1 ? (kc + BK - 1) / BK * BK : K;  // chunk bounds on BK steps
-  const uint64_t nchunks = chunks > 1 ? (K + kcr - 1) / kcr : 1;
-  c128 *out = chunks > 1 ? partials : C;
-  const uint64_t out_ld = chunks > 1 ? N : ldc;
-  const uint64_t cstride = chunks > 1 ? M * N : 0;
-  const dim3 grid((unsigned)tiles, (unsigned)nchunks);
-  if (bn == 128)
-    hipLaunchKernelGGL((zgemm_f64_kernel<64, 128>), grid, dim3(kThreads), 0, ctx->stream, A, B, out, M, N, K, lda, ldb,
-                       out_ld, kcr, cstride);
+  const ZShape z = zgemm_shape(M, N, K);
+  const uint64_t tiles = ((N + z.bn - 1) / z.bn) * ((M + z.bm - 1) / z.bm);
+  if (tiles > 0x7fffffffull / z.chunks) return set_error(ctx, QTNH_EUNSUPPORTED, "zgemm: grid too large");
+  if (z.chunks > 1 && !partials) return set_error(ctx, QTNH_EINVAL, "zgemm: depth chunks need a partial buffer");
+  c128 *out = z.chunks > 1 ? partials : C;
+  const uint64_t ld = z.chunks > 1 ? N : ldc, cstride = z.chunks > 1 ? M * N : 0;
+  if (z.bm == 64)
+    launch_tile_gemm<64, 64>(ctx, A, B, out, M, N, K, lda, ldb, ld, cstride, z);
+  else if (z.bn == 64)
+    launch_tile_gemm<32, 64>(ctx, A, B, out, M, N, K, lda, ldb, ld, cstride, z);
   else
-    hipLaunchKernelGGL((zgemm_f64_kernel<64, 64>), grid, dim3(kThreads), 0, ctx->stream, A, B, out, M, N, K, lda, ldb,
-                       out_ld, kcr, cstride);
+    launch_tile_gemm<32, 32>(ctx, A, B, out, M, N, K, lda, ldb, ld, cstride, z);
   qtnh_status st = check_hip(ctx, hipGetLastError(), "zgemm launch");
-  if (st || nchunks <= 1) return st;
+  if (st || z.chunks <= 1) return st;
   hipLaunchKernelGGL(zgemm_chunk_sum_kernel, dim3(grid_for(M * N, 256, 65536)), dim3(256), 0, ctx->stream,
-                     (const double2_t *)partials, (double2_t *)C, M, N, ldc, nchunks);
+                     (const double2_t *)partials, (double2_t *)C, M, N, ldc, z.chunks);
   return check_hip(ctx, hipGetLastError(), "zgemm chunk sum launch");
 }
 
@@ -376,24 +504,27 @@ uint64_t splitk_chunk_len(uint64_t K, uint64_t chunks) {
   return ((K + chunks - 1) / chunks + kSkThreads - 1) / kSkThreads * kSkThreads;
 }
 
-int zgemm_block_n(uint64_t M, uint64_t N) { return zgemm_bn(M, N); }
-
 // Depth chunks of launch_zgemm_f64 on BK steps: (chunk length, chunk count).
 void zgemm_chunk_shape(uint64_t M, uint64_t N, uint64_t K, uint64_t *kc_out, uint64_t *n_out) {
-  const uint64_t chunks = zgemm_chunks(M, N, K);
-  const uint64_t kc = chunks > 1 ? (K + chunks - 1) / chunks : K;
-  const uint64_t kcr = chunks > 1 ? (kc + BK - 1) / BK * BK : K;
-  *kc_out = kcr;
-  *n_out = chunks > 1 ? (K + kcr - 1) / kcr : 1;
+  const ZShape z = zgemm_shape(M, N, K);
+  *kc_out = z.kc;
+  *n_out = z.chunks;
 }
 
-qtnh_status launch_zgemm_grouped(qtnh_ctx_t ctx, int bn, const ZGroupDesc *d, int nd, uint64_t total) {
+// Tile edge of a shape's GEMM in grouped launches (other shapes fill the GPU
+// beside it): 64 where that wastes little of its tiles, else 32.
+int zgemm_group_tile(uint64_t M, uint64_t N) {
+  auto padded = [&](uint64_t b) { return ((M + b - 1) / b) * ((N + b - 1) / b) * b * b; };
+  return M > 32 && N > 32 && padded(64) * 4 <= padded(32) * 5 ? 64 : 32;
+}
+
+qtnh_status launch_zgemm_grouped(qtnh_ctx_t ctx, int tile, const ZGroupDesc *d, int nd, uint64_t total) {
   if (nd <= 0 || total == 0) return QTNH_OK;
   const unsigned grid = (unsigned)std::min<uint64_t>(total, (uint64_t)ctx->num_cus * 8);
-  if (bn == 128)
-    hipLaunchKernelGGL(zgemm_grouped_kernel<128>, dim3(grid), dim3(kThreads), 0, ctx->stream, d, nd, total);
+  if (tile == 64)
+    hipLaunchKernelGGL((zgemm_grouped_kernel<64, 64>), dim3(grid), dim3(kThreads), 0, ctx->stream, d, nd, total);
   else
-    hipLaunchKernelGGL(zgemm_grouped_kernel<64>, dim3(grid), dim3(kThreads), 0, ctx->stream, d, nd, total);
+    hipLaunchKernelGGL((zgemm_grouped_kernel<32, 32>), dim3(grid), dim3(kThreads), 0, ctx->stream, d, nd, total);
   return check_hip(ctx, hipGetLastError(), "grouped zgemm launch");
 }
 

@@ -256,7 +256,7 @@ def tune_permute_auto(on=True):
 
 
 def tune_zgemm(bn=0):
-    """Block width (64 or 128 complex columns; 0 chooses by size) of the FP64 complex GEMM (process-wide)."""
+    """Tiles of the FP64 complex GEMM (process-wide): 0 by size, 64 or 128 always 64 x 64."""
     lib().qtnh_tune_zgemm(bn)
 
 

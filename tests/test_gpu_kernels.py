@@ -516,3 +516,28 @@ def test_norm2_and_scale():
     y = host(t)
     exp = (x.real * 0.5 - x.imag * -2.0) + 1j * (x.real * -2.0 + x.imag * 0.5)
     assert same_bits(y, exp)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 1025, 33), (64, 1024, 17), (31, 65, 1040), (65, 2049, 32), (100, 700, 31),
+                                   (257, 129, 47), (63, 64, 1025), (200, 300, 257), (129, 1000, 512), (96, 96, 2049),
+                                   (1, 5000, 300), (5000, 2, 300), (513, 511, 49), (1500, 1400, 48)])
+def test_contract_gemm_every_tile_and_depth(m, n, k):
+    """Tiles of 64 x 64, 32 x 64 and 32 x 32, with and without depth chunks;
+    results one below and above tile edges; depths of whole stages and of one
+    term more or less.  A NaN in the last row of A and an infinity in the last
+    column of B reach only that row and column (rows, columns and terms past
+    the operands' ends are read again or zeroed, never mixed in)."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)) + 1j * rng.standard_normal((m, k))
+    b = rng.standard_normal((k, n)) + 1j * rng.standard_normal((k, n))
+    ref = a @ b
+    got, _, _ = ops.contract(dev(a), [m, k], dev(b), [k, n], [(1, 0)])
+    got = host(got).reshape(m, n)
+    assert np.linalg.norm(got - ref) <= 1e-12 * np.linalg.norm(ref)
+    a[-1, k // 2] = np.nan
+    b[k - 1, -1] = np.inf
+    got, _, _ = ops.contract(dev(a), [m, k], dev(b), [k, n], [(1, 0)])
+    got = host(got).reshape(m, n)
+    assert np.isnan(got[-1]).all() and not np.isfinite(got[:, -1]).any()
+    inner = np.linalg.norm(got[:-1, :-1] - ref[:-1, :-1])
+    assert inner <= 1e-12 * max(np.linalg.norm(ref[:-1, :-1]), 1e-300)
