@@ -110,65 +110,229 @@ __global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *
   }
 }
 
-// The leading run of one network's steps that are small direct contractions
-// (a chain): descriptors [first, first + count), in step order.
+// Steps of a network's leading run of small direct contractions (operands and
+// result of at most 2^12 elements) run in its chain: one workgroup steps
+// through them.  On 256 grid-circuit networks that is 97% of the steps, which
+// would be 600 grouped launches.
+constexpr uint64_t kChainMaxElems = 1ull << 12;
+// ... and the run ends at a step of more products than one workgroup should do
+// (2287 us without this limit, 2231 with it, 2253 with 2^14, on 32 networks of 4 x 5
+// grid circuits).
+constexpr uint64_t kChainMaxProducts = 1ull << 15;
+constexpr int kChainBits = 12;
+constexpr uint32_t kChainLds = 4096;   // elements of intermediates held in LDS
+constexpr uint32_t kChainStage = 64;   // largest leaf staged ahead (elements)
+enum : uint32_t {  // ChainStep::ctl: LDS offset of the result, log2 of its elements << 16, log2 of the terms << 20 and
+  kChainGlobalA = 1u << 24,    // A, B are read from global memory
+  kChainGlobalB = 1u << 25,
+  kChainStoreLds = 1u << 26,   // the result goes to LDS, to global memory
+  kChainStoreGlobal = 1u << 27,
+  kChainWait = 1u << 28,       // ... from where a later step of the chain reads it
+  kChainSmall = 1u << 29,      // all in LDS, at most 256 elements of 2 or 4 terms
+};
+struct alignas(16) ChainStep {
+  uint32_t base;              // LDS offset of A | of B << 16
+  uint32_t ctl;
+  uint32_t flip0, flip1;      // what counting the closed tuple up flips, by ctz(t + 1): A offset | B offset << 16
+  uint32_t mask[kChainBits];  // result bit: A offset | B offset << 16
+  uint32_t flip[kChainBits - 2];  // flips for ctz 2, 3, ...
+  const double2_t *a, *b;     // operands in global memory
+  double2_t *c;
+  uint32_t na, nb;            // elements of A, B to stage, if leaves small enough
+};
+static_assert(sizeof(ChainStep) == 144, "nine 16-byte pieces");
 struct ChainDesc {
   uint32_t first, count;
 };
 
-// Chains, one workgroup each: the workgroup runs its network's chain steps in
-// order, each element as grouped_direct_kernel computes it (same terms, same
-// order, same arithmetic), with a barrier between steps.  A step reads only
-// the network's leaves and the results of earlier steps of its chain, written
-// by the same workgroup: all of it stays on one compute unit, and the barrier
-// (which waits for the stores) orders those writes before the next step's
-// reads.  Replaces one grouped launch per step index for these steps.
-__global__ void __launch_bounds__(kGThreads) chain_direct_kernel(const GDesc *__restrict__ descs,
-                                                                 const ChainDesc *__restrict__ chains, int nchains) {
-  __shared__ uint64_t flip_a[64], flip_b[64];
-  for (int c = blockIdx.x; c < nchains; c += gridDim.x) {
-    const ChainDesc ch = chains[c];
-    for (uint32_t k = 0; k < ch.count; ++k) {
-      const GDesc &D = descs[ch.first + k];
-      __syncthreads();  // the previous step's results are stored; its mask readers are done
-      if ((int)threadIdx.x < D.kbits) {
-        uint64_t fa = 0, fb = 0;
-        for (int j = 0; j <= (int)threadIdx.x; ++j) {
-          fa |= 1ull << D.ka[j];
-          fb |= 1ull << D.kb[j];
-        }
-        flip_a[threadIdx.x] = fa;
-        flip_b[threadIdx.x] = fb;
-      }
-      __syncthreads();
-      const uint64_t K = 1ull << D.kbits;
-      for (uint64_t e = threadIdx.x; e < D.nC; e += kGThreads) {
-        uint64_t oa = 0, ob = 0;
-        for (int p = 0; p < D.ncb; ++p) {
-          if (!((e >> p) & 1ull)) continue;
-          if (D.abit[p] >= 0)
-            oa |= 1ull << D.abit[p];
-          else
-            ob |= 1ull << D.bbit[p];
-        }
-        double ar = 0.0, ai = 0.0;
-        uint64_t xa = oa, xb = ob;
-        for (uint64_t t = 0; t < K; ++t) {
-          const double2_t a = D.A[xa], b = D.B[xb];
-          double pr, pi;
-          cmul_parts(a.x, a.y, b.x, b.y, &pr, &pi);
-          ar = ar + pr;
-          ai = ai + pi;
-          if (t + 1 < K) {
-            const int cb = __builtin_ctzll(t + 1);
-            xa ^= flip_a[cb];
-            xb ^= flip_b[cb];
-          }
-        }
-        D.C[e] = double2_t{ar, ai};
+// A pointer read from LDS has no known address space: accesses through it would
+// be flat ones, which the LDS barrier waits for.
+using GlobalIn = const __attribute__((address_space(1))) double2_t *;
+using GlobalOut = __attribute__((address_space(1))) double2_t *;
+
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+__device__ __forceinline__ void chain_mac(double &ar, double &ai, double2_t a, double2_t b) {
+  double pr, pi;
+  cmul_parts(a.x, a.y, b.x, b.y, &pr, &pi);
+  ar = ar + pr;
+  ai = ai + pi;
+}
+
+// Chains, one workgroup each.  What bounds them is latency, step after step:
+// so intermediates stay in LDS where they fit (a step's result goes to global
+// memory only for readers outside the chain), and a wave of its own brings each
+// step's record to LDS five steps ahead and its leaf operands one step ahead,
+// requested three steps before that; the others read nothing from memory.  Nine
+// steps in ten are tiny: their offsets are computed in the step before, so that
+// operand reads follow the barrier at once.  32 networks of 4 x 5 grid
+// circuits, depth 12, 361 steps each: 1146 us with records, operands and results
+// in global memory, 216 us so (385 with every wave loading one step ahead).
+// Each element is computed as grouped_direct_kernel does (same terms, same
+// order, same arithmetic).
+template <bool AL, bool BL>
+__device__ __forceinline__ void chain_step_elements(const ChainStep &D, double2_t *lds, uint32_t ctl, uint32_t low,
+                                                    int tid) {
+  const GlobalIn ga = (GlobalIn)D.a, gb = (GlobalIn)D.b;
+  const GlobalOut gc = (GlobalOut)D.c;
+  const uint32_t n = 1u << (ctl >> 16 & 15), K = 1u << (ctl >> 20 & 15);
+  const uint32_t base = D.base, f0 = D.flip0, f1 = D.flip1;
+  auto get_a = [&](uint32_t x) { return AL ? lds[(base + x) & 0xffffu] : ga[x & 0xffffu]; };
+  auto get_b = [&](uint32_t x) { return BL ? lds[(base + x) >> 16] : gb[x >> 16]; };
+  for (uint32_t e = tid; e < n; e += kGThreads) {
+    uint32_t x = low;
+#pragma unroll
+    for (int p = 8; p < kChainBits; ++p) x ^= (0u - ((e >> p) & 1u)) & D.mask[p];
+    double ar = 0.0, ai = 0.0;
+    if (K < 4) {
+      chain_mac(ar, ai, get_a(x), get_b(x));
+      if (K == 2) chain_mac(ar, ai, get_a(x ^ f0), get_b(x ^ f0));
+    } else {
+      // Four terms' operands are requested before their products are added, in order.
+      for (uint32_t t = 0;;) {
+        const uint32_t x1 = x ^ f0, x2 = x1 ^ f1, x3 = x2 ^ f0;
+        const double2_t a0 = get_a(x), a1 = get_a(x1), a2 = get_a(x2), a3 = get_a(x3);
+        const double2_t b0 = get_b(x), b1 = get_b(x1), b2 = get_b(x2), b3 = get_b(x3);
+        chain_mac(ar, ai, a0, b0);
+        chain_mac(ar, ai, a1, b1);
+        chain_mac(ar, ai, a2, b2);
+        chain_mac(ar, ai, a3, b3);
+        t += 4;
+        if (t == K) break;
+        x = x3 ^ D.flip[__builtin_ctz(t) - 2];
       }
     }
-    __syncthreads();  // the next chain's masks are written after this one's readers finish
+    if (ctl & kChainStoreLds) lds[(ctl & 0xffffu) + e] = double2_t{ar, ai};
+    if (ctl & kChainStoreGlobal) gc[e] = double2_t{ar, ai};
+  }
+}
+
+__global__ void __launch_bounds__(kGThreads + 64) chain_direct_kernel(const ChainStep *__restrict__ steps,
+                                                                      const ChainDesc *__restrict__ chains,
+                                                                      int nchains) {
+  __shared__ double2_t lds[kChainLds + 4 * kChainStage];  // intermediates; two stages of (A leaf, B leaf)
+  __shared__ ChainStep ring[8];
+  constexpr int kPieces = sizeof(ChainStep) / 16;
+  const int tid = threadIdx.x;
+  for (int c = blockIdx.x; c < nchains; c += gridDim.x) {
+    const ChainDesc ch = chains[c];
+    __syncthreads();  // the previous chain's readers are done
+    if (tid >= kGThreads) {
+      // The last wave loads for the others.  In step k it requests record k + 8
+      // and the leaves of step k + 4, and stores what it requested in step
+      // k - 3: record k + 5 (slot last read in step k - 3) and the leaves of
+      // step k + 1 (the stage last read in step k - 1).
+      const uint32_t lane = tid - kGThreads;
+      const uint4 *src = reinterpret_cast<const uint4 *>(steps + ch.first);
+      uint4 *rpieces = reinterpret_cast<uint4 *>(ring);
+      struct Ahead {
+        uint4 rec;       // a piece of the record
+        double2_t a, b;  // elements of the leaves
+      };
+      const uint32_t piece = lane < kPieces ? lane : 0;
+      auto request_record = [&](uint32_t k, Ahead &x) {
+        x.rec = src[(uint64_t)min(k, ch.count - 1) * kPieces + piece];
+      };
+      // (A lane without an element loads something valid: a load under a
+      // condition would be waited for where it is merged with its absence.)
+      auto request_leaves = [&](uint32_t k, Ahead &x) {
+        const ChainStep &D = ring[k & 7];
+        const uint32_t left = k < ch.count ? ~0u : 0u;
+        const uint64_t pa = (uint64_t)(D.a + lane), pb = (uint64_t)(D.b + lane), none = (uint64_t)src;
+        x.a = *(GlobalIn)(lane < (D.na & left) ? pa : none);
+        x.b = *(GlobalIn)(lane < (D.nb & left) ? pb : none);
+      };
+      auto store_record = [&](uint32_t k, const Ahead &x) {
+        if (lane < kPieces) rpieces[(k & 7) * kPieces + lane] = x.rec;
+      };
+      auto store_leaves = [&](uint32_t k, const Ahead &x) {
+        double2_t *stage = lds + kChainLds + (k & 1) * 2 * kChainStage;
+        stage[lane] = x.a;
+        stage[kChainStage + lane] = x.b;
+      };
+      if (lane < 5 * kPieces && lane < ch.count * kPieces) rpieces[lane] = src[lane];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      Ahead s0, s1, s2, s3;
+      request_leaves(0, s0);
+      request_record(5, s1);
+      request_leaves(1, s1);
+      request_record(6, s2);
+      request_leaves(2, s2);
+      request_record(7, s3);
+      request_leaves(3, s3);
+      store_leaves(0, s0);
+      lds_barrier();
+      auto step = [&](uint32_t k, Ahead &request, const Ahead &arrived) {
+        request_record(k + 8, request);
+        request_leaves(k + 4, request);
+        store_record(k + 5, arrived);
+        store_leaves(k + 1, arrived);
+        lds_barrier();
+        return k + 1 < ch.count;
+      };
+      for (uint32_t k = 0;; k += 4)
+        if (!step(k, s0, s1) || !step(k + 1, s1, s2) || !step(k + 2, s2, s3) || !step(k + 3, s3, s0)) break;
+    } else {
+      uint32_t on[8];  // bit p of the thread's element, as a mask
+#pragma unroll
+      for (int p = 0; p < 8; ++p) on[p] = 0u - ((uint32_t)(tid >> p) & 1u);
+      // The head of step k's record (k is wave-uniform) and the offsets of the thread's first element.
+      auto head = [&](uint32_t k, uint4 &h, uint32_t &x) {
+        const ChainStep &D = ring[k & 7];
+        h = *reinterpret_cast<const uint4 *>(&D);
+        x = 0;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) x ^= on[p] & D.mask[p];
+      };
+      uint4 h;
+      uint32_t x;
+      lds_barrier();
+      head(0, h, x);
+      for (uint32_t k = 0; k < ch.count; ++k) {
+        const uint32_t ctl = uniform(h.y);
+        uint4 hn;
+        uint32_t xn;
+        if (ctl & kChainSmall) {
+          const uint32_t n = 1u << (ctl >> 16 & 15);
+          if ((uint32_t)(tid & ~63) < n) {  // wave-uniform; lanes past n read in range (their masks are zero)
+            const uint32_t p0 = h.x + x, p1 = h.x + (x ^ h.z);
+            const double2_t a0 = lds[p0 & 0xffffu], b0 = lds[p0 >> 16], a1 = lds[p1 & 0xffffu], b1 = lds[p1 >> 16];
+            double ar = 0.0, ai = 0.0;
+            if (ctl >> 20 & 2) {
+              const uint32_t x2 = x ^ h.z ^ h.w, p2 = h.x + x2, p3 = h.x + (x2 ^ h.z);
+              const double2_t a2 = lds[p2 & 0xffffu], b2 = lds[p2 >> 16], a3 = lds[p3 & 0xffffu], b3 = lds[p3 >> 16];
+              head(k + 1, hn, xn);
+              chain_mac(ar, ai, a0, b0);
+              chain_mac(ar, ai, a1, b1);
+              chain_mac(ar, ai, a2, b2);
+              chain_mac(ar, ai, a3, b3);
+            } else {
+              head(k + 1, hn, xn);
+              chain_mac(ar, ai, a0, b0);
+              chain_mac(ar, ai, a1, b1);
+            }
+            if ((uint32_t)tid < n) lds[(ctl & 0xffffu) + tid] = double2_t{ar, ai};
+          } else {
+            head(k + 1, hn, xn);
+          }
+        } else {
+          const ChainStep &D = ring[k & 7];
+          if (!(ctl & (kChainGlobalA | kChainGlobalB)))
+            chain_step_elements<true, true>(D, lds, ctl, x, tid);
+          else if (!(ctl & kChainGlobalA))
+            chain_step_elements<true, false>(D, lds, ctl, x, tid);
+          else if (!(ctl & kChainGlobalB))
+            chain_step_elements<false, true>(D, lds, ctl, x, tid);
+          else
+            chain_step_elements<false, false>(D, lds, ctl, x, tid);
+          if (ctl & kChainWait) __builtin_amdgcn_s_waitcnt(0);
+          head(k + 1, hn, xn);
+        }
+        h = hn;
+        x = xn;
+        lds_barrier();
+      }
+    }
   }
 }
 
@@ -196,6 +360,7 @@ uint64_t mix(uint64_t a, uint64_t b) {
 }  // namespace qtnh_hip
 
 using qtnh_hip::c128;
+using qtnh_hip::ChainStep;
 using qtnh_hip::GDesc;
 
 struct qtnh_net_s {
@@ -237,6 +402,8 @@ struct qtnh_net_s {
   // Grouped-launch descriptor of each direct power-of-two step, without its
   // device pointers and launch position (filled in per batch placement).
   std::vector<GDesc> gdesc;
+  // Records of the steps of the network's chain, without device pointers.
+  std::vector<ChainStep> chain;
   // Device copy of leaf_data: uploaded by the first blocking run on a device
   // and read in place by later ones (leaf values cannot change once added;
   // adding a leaf drops the copy).
@@ -253,6 +420,7 @@ namespace {
 uint64_t block_elems(const qtnh_net_s &n) { return round16(n.leaf_elems) + round16(n.arena_elems); }
 
 GDesc gdesc_template(const qtnh_net_s &net, size_t s);
+void plan_chain(qtnh_net_s &net);
 
 // A network in split precision uses the split GEMM only for steps where it
 // is the faster: 128 x 128 output tiles over M x 2N (the embedded real
@@ -405,6 +573,7 @@ void finish_plan(qtnh_net_s &net) {
   net.gdesc.assign(net.steps.size(), GDesc{});
   for (size_t s = 0; s < net.steps.size(); ++s)
     if (net.steps[s].direct && net.steps[s].binary) net.gdesc[s] = gdesc_template(net, s);
+  plan_chain(net);
   net.planned = true;
 }
 
@@ -843,6 +1012,74 @@ GDesc gdesc_template(const qtnh_net_s &net, size_t s) {
   return d;
 }
 
+// The network's chain: records of its leading small direct steps.  Their
+// intermediates get LDS offsets by first fit over their lifetimes; one that
+// does not fit, or that a step outside the chain reads, goes to its arena place.
+void plan_chain(qtnh_net_s &net) {
+  auto small = [&](int x) { return net.nodes[x].size <= kChainMaxElems; };
+  size_t count = 0;
+  while (count < net.steps.size()) {
+    const auto &st = net.steps[count];
+    if (!st.direct || !st.binary || !small(st.a) || !small(st.b) || !small(st.c)) break;
+    if (net.nodes[st.c].size << net.gdesc[count].kbits > kChainMaxProducts) break;
+    ++count;
+  }
+  std::vector<size_t> reader(net.nodes.size(), net.steps.size());  // step that reads a node
+  for (size_t s = 0; s < net.steps.size(); ++s) reader[net.steps[s].a] = reader[net.steps[s].b] = s;
+  std::vector<int64_t> slot(net.nodes.size(), -1);
+  Arena arena;
+  net.chain.assign(count, ChainStep{});
+  for (size_t s = 0; s < count; ++s) {
+    const auto &st = net.steps[s];
+    const GDesc &g = net.gdesc[s];
+    ChainStep &d = net.chain[s];
+    uint32_t f = 0;
+    for (int p = 0; p < g.ncb; ++p) d.mask[p] = g.abit[p] >= 0 ? 1u << g.abit[p] : (1u << g.bbit[p]) << 16;
+    for (int j = 0; j < g.kbits; ++j) {
+      f |= 1u << g.ka[j] | (1u << g.kb[j]) << 16;
+      (j == 0 ? d.flip0 : j == 1 ? d.flip1 : d.flip[j - 2]) = f;
+    }
+    d.ctl = (uint32_t)g.ncb << 16 | (uint32_t)g.kbits << 20;
+    // An operand's LDS offset: its own, or the stage that the loading wave fills for this step.
+    auto operand = [&](int x, uint32_t second, uint32_t global, uint32_t &count) -> uint32_t {
+      if (slot[x] >= 0) return (uint32_t)slot[x];
+      if ((size_t)x < net.n_leaves && net.nodes[x].size <= kChainStage) {
+        count = (uint32_t)net.nodes[x].size;
+        return kChainLds + (uint32_t)(s & 1) * 2 * kChainStage + second * kChainStage;
+      }
+      d.ctl |= global;
+      return 0;
+    };
+    d.base = operand(st.a, 0, kChainGlobalA, d.na);
+    d.base |= operand(st.b, 1, kChainGlobalB, d.nb) << 16;
+    const uint64_t size = net.nodes[st.c].size;
+    d.ctl |= kChainStoreGlobal;
+    if (reader[st.c] < count) {
+      d.ctl |= kChainWait;
+      const uint64_t at = arena.alloc(size);
+      if (at + round16(size) <= kChainLds) {
+        slot[st.c] = (int64_t)at;
+        d.ctl = (d.ctl & ~(kChainStoreGlobal | kChainWait)) | kChainStoreLds | (uint32_t)at;
+      } else {
+        arena.release(at, size);
+      }
+    }
+    const uint32_t inside = kChainGlobalA | kChainGlobalB | kChainStoreGlobal;
+    if (!(d.ctl & inside) && g.ncb <= 8 && (g.kbits == 1 || g.kbits == 2)) d.ctl |= kChainSmall;
+    for (int x : {st.a, st.b})
+      if (slot[x] >= 0) arena.release((uint64_t)slot[x], net.nodes[x].size);
+  }
+}
+
+ChainStep make_chain_step(const qtnh_net_s &net, Where block, size_t s) {
+  const auto &st = net.steps[s];
+  ChainStep d = net.chain[s];
+  d.a = (const double2_t *)node_ptr(net, block, st.a);
+  d.b = (const double2_t *)node_ptr(net, block, st.b);
+  d.c = (double2_t *)node_ptr(net, block, st.c);
+  return d;
+}
+
 // The step's descriptor for one placement of the network.
 GDesc make_gdesc(const qtnh_net_s &net, Where block, size_t s, uint64_t first) {
   const auto &st = net.steps[s];
@@ -868,17 +1105,6 @@ bool grouped_step(const qtnh_net_s &n, int prec, size_t s, uint64_t sum) {
   if (s >= n.steps.size()) return false;
   const auto &st = n.steps[s];
   return st.groupable && step_precision(st, prec) == QTNH_PREC_FP64 && sum + st.ws64 <= kGroupWsTotal;
-}
-
-// Steps of a network's leading run of small direct contractions (operands and
-// result of at most 2^12 elements) run in its chain, one workgroup stepping
-// through them (chain_direct_kernel): measured on 256 grid-circuit networks,
-// 97% of the steps, in 217 instead of 609 step indices of grouped launches.
-constexpr uint64_t kChainMaxElems = 1ull << 12;
-bool chain_step(const qtnh_net_s &n, size_t s) {
-  const auto &st = n.steps[s];
-  return st.direct && st.binary && n.nodes[st.a].size <= kChainMaxElems && n.nodes[st.b].size <= kChainMaxElems &&
-         n.nodes[st.c].size <= kChainMaxElems;
 }
 
 // Device bytes of a wave (a consecutive run of networks), network by network:
@@ -931,11 +1157,14 @@ struct Wave {
   std::vector<uint32_t> dk;
   std::vector<size_t> dk_off;
   std::vector<uint64_t> dfirst;
-  // Network i's steps [0, chain_len[i]) run in chain_direct_kernel (chains: one
-  // per network with a chain, descriptors at the front of the list).
-  std::vector<size_t> chain_len;
+  // Network i's steps [0, nets[i]->chain.size()) run in chain_direct_kernel:
+  // one chain per network that has one, records network by network.
+  std::vector<size_t> chain_at;  // first record of network i
   std::vector<ChainDesc> chains;
+  size_t nchain = 0;
   ChainDesc *dchains = nullptr;
+  ChainStep *dcsteps = nullptr;
+  std::vector<ChainStep> csteps;  // host copy, when built in full (prepared batches)
   std::vector<Gather> gathers;
   c128 *base = nullptr, *res = nullptr;
   char *gws = nullptr;
@@ -994,19 +1223,16 @@ struct Wave {
       loff += round16(n->leaf_elems);
       aoff += round16(n->arena_elems);
     }
-    // Descriptor positions.  First each network's chain (its leading small
-    // direct steps, chain_direct_kernel), network by network; then, for every
-    // step index, that index's other direct steps in network order, each with
-    // its first block in the index's grouped launch (from the step templates'
-    // result sizes).
-    chain_len.assign(nets.size(), 0);
+    // Descriptor positions.  Each network's chain has its own records; then, for
+    // every step index, that index's other direct steps in network order, each
+    // with its first block in the index's grouped launch (from the step
+    // templates' result sizes).
+    chain_at.assign(nets.size(), 0);
     chains.clear();
-    size_t nchain = 0;
+    nchain = 0;
     for (size_t i = 0; i < nets.size(); ++i) {
-      const auto &n = *nets[i];
-      size_t c = 0;
-      while (c < n.steps.size() && chain_step(n, c)) ++c;
-      chain_len[i] = c;
+      chain_at[i] = nchain;
+      const size_t c = nets[i]->chain.size();
       if (c) chains.push_back({(uint32_t)nchain, (uint32_t)c});
       nchain += c;
     }
@@ -1017,24 +1243,18 @@ struct Wave {
       const auto *n = nets[i];
       dk_off[i] = ndk;
       ndk += n->steps.size();
-      for (size_t s = chain_len[i]; s < n->steps.size(); ++s) starts[s + 1] += n->steps[s].direct && n->steps[s].binary;
+      for (size_t s = n->chain.size(); s < n->steps.size(); ++s) starts[s + 1] += n->steps[s].direct && n->steps[s].binary;
     }
-    starts[0] = nchain;
     for (size_t s = 0; s < steps; ++s) starts[s + 1] += starts[s];
     ndesc = starts[steps];
     dk.assign(ndk, 0);
     dfirst.assign(ndesc, 0);
     {
       std::vector<size_t> next(starts.begin(), starts.end() - 1);
-      size_t kc = 0;
       for (size_t i = 0; i < nets.size(); ++i) {
         const auto *n = nets[i];
-        for (size_t s = 0; s < n->steps.size(); ++s) {
+        for (size_t s = n->chain.size(); s < n->steps.size(); ++s) {
           if (!n->steps[s].direct || !n->steps[s].binary) continue;
-          if (s < chain_len[i]) {
-            dk[dk_off[i] + s] = (uint32_t)kc++;  // first block unused (dfirst 0)
-            continue;
-          }
           const size_t k = next[s]++;
           dk[dk_off[i] + s] = (uint32_t)k;
           dfirst[k] = gdesc_blocks(n->gdesc[s]);  // block count; prefix sums below
@@ -1051,7 +1271,8 @@ struct Wave {
     }
     if (with_descs) {
       descs.resize(ndesc);
-      fill_descs(descs.data());
+      csteps.resize(nchain);
+      fill_descs(descs.data(), csteps.data());
       hdesc = descs.data();
     }
     layout_grouped();
@@ -1181,19 +1402,20 @@ struct Wave {
     }
   }
 
-  // Every direct-step descriptor (chains and step indices) into out[0 .. ndesc),
-  // network by network, networks split over up
+  // Every direct-step descriptor into out[0 .. ndesc) and every chain record
+  // into chain_out[0 .. nchain), network by network, networks split over up
   // to kPlanThreads host threads (measured: 8-13 ms for the 93k descriptors
   // of a 256-network batch when built step index by step index on one thread,
   // which touches every network per step index).
-  void fill_descs(GDesc *out) const {
+  void fill_descs(GDesc *out, ChainStep *chain_out) const {
     const int nt = (int)std::max<size_t>(1, std::min<size_t>({nets.size(), (size_t)kPlanThreads,
                                                                (size_t)std::max(1u, std::thread::hardware_concurrency()),
-                                                               (ndesc + 4095) / 4096}));
+                                                               (ndesc + nchain + 4095) / 4096}));
     auto work = [&](int t) {
       for (size_t i = t; i < nets.size(); i += nt) {
         const auto &n = *nets[i];
-        for (size_t s = 0; s < n.steps.size(); ++s) {
+        for (size_t s = 0; s < n.chain.size(); ++s) chain_out[chain_at[i] + s] = make_chain_step(n, blocks[i], s);
+        for (size_t s = n.chain.size(); s < n.steps.size(); ++s) {
           if (!n.steps[s].direct || !n.steps[s].binary) continue;
           const size_t k = dk[dk_off[i] + s];
           out[k] = make_gdesc(n, blocks[i], s, dfirst[k]);
@@ -1208,8 +1430,11 @@ struct Wave {
 
   static uint64_t pad256(uint64_t b) { return (b + 255) & ~255ull; }
 
+  // The per-step descriptors: direct steps, then chain records.
+  uint64_t head_bytes() const { return pad256(ndesc * sizeof(GDesc)) + pad256(nchain * sizeof(ChainStep)); }
+
   uint64_t desc_bytes() const {
-    return pad256(ndesc * sizeof(GDesc)) + pad256(gathers.size() * sizeof(Gather)) +
+    return head_bytes() + pad256(gathers.size() * sizeof(Gather)) +
            pad256(chains.size() * sizeof(ChainDesc)) +
            pad256(pin.size() * sizeof(PermDesc)) + pad256(pout.size() * sizeof(PermDesc)) +
            pad256(zg[0].size() * sizeof(ZGroupDesc)) + pad256(zg[1].size() * sizeof(ZGroupDesc)) +
@@ -1220,6 +1445,8 @@ struct Wave {
     char *p = (char *)mem;
     ddesc = (GDesc *)p;
     p += pad256(ndesc * sizeof(GDesc));
+    dcsteps = (ChainStep *)p;
+    p += pad256(nchain * sizeof(ChainStep));
     dgath = (Gather *)p;
     p += pad256(gathers.size() * sizeof(Gather));
     dchains = (ChainDesc *)p;
@@ -1239,7 +1466,7 @@ struct Wave {
 
   // Bytes from the gather table to the end of the descriptor region (laid out
   // as on the device): what upload_packed stages.
-  uint64_t tail_bytes() const { return desc_bytes() - pad256(ndesc * sizeof(GDesc)); }
+  uint64_t tail_bytes() const { return desc_bytes() - head_bytes(); }
 
   // The gather table and the grouped GEMM-route descriptors, packed into
   // pinned staging at their device layout and sent with one asynchronous copy
@@ -1285,6 +1512,7 @@ struct Wave {
                        "batch grouped descriptor upload");
     };
     put(dchains, chains.data(), chains.size() * sizeof(ChainDesc));
+    put(dcsteps, csteps.data(), csteps.size() * sizeof(ChainStep));
     put(d_pin, pin.data(), pin.size() * sizeof(PermDesc));
     put(d_pout, pout.data(), pout.size() * sizeof(PermDesc));
     put(d_zg[0], zg[0].data(), zg[0].size() * sizeof(ZGroupDesc));
@@ -1323,7 +1551,7 @@ struct Wave {
   // The kernels of step indices [s0, s1) (from index 0: the chains first).
   qtnh_status enqueue_steps(qtnh_ctx_t ctx, size_t s0, size_t s1) {
     if (s0 == 0 && !chains.empty()) {
-      hipLaunchKernelGGL(chain_direct_kernel, dim3((unsigned)chains.size()), dim3(kGThreads), 0, ctx->stream, ddesc,
+      hipLaunchKernelGGL(chain_direct_kernel, dim3((unsigned)chains.size()), dim3(kGThreads + 64), 0, ctx->stream, dcsteps,
                          dchains, (int)chains.size());
       qtnh_status st = check_hip(ctx, hipGetLastError(), "chain launch");
       if (st) return st;
@@ -1722,7 +1950,7 @@ qtnh_status qtnh_net_run_batch(qtnh_ctx_t ctx, int count, const qtnh_net_t *nets
     Wave w;
     w.layout(nets + w0, w1 - w0, (char *)wp, false, resident.data());
     // Pinned staging: the direct-step descriptors, then the other tables.
-    const uint64_t gbytes = ((std::max<size_t>(w.ndesc, 1) * sizeof(GDesc)) + 255) & ~255ull;
+    const uint64_t gbytes = w.head_bytes();
     st = grow_buffer(ctx, &ctx->desc, &ctx->desc_bytes, w.desc_bytes());
     if (!st) st = grow_pinned(ctx, gbytes + w.tail_bytes());
     if (st) return st;
@@ -1733,9 +1961,9 @@ qtnh_status qtnh_net_run_batch(qtnh_ctx_t ctx, int count, const qtnh_net_t *nets
     // by its copy before the wave's closing sync.
     GDesc *hp = (GDesc *)ctx->pinned;
     w.hdesc = hp;
-    if (!st && w.ndesc) {
-      w.fill_descs(hp);
-      st = check_hip(ctx, hipMemcpyAsync(w.ddesc, hp, w.ndesc * sizeof(GDesc), hipMemcpyHostToDevice, ctx->stream),
+    if (!st && gbytes) {
+      w.fill_descs(hp, (ChainStep *)((char *)hp + Wave::pad256(w.ndesc * sizeof(GDesc))));
+      st = check_hip(ctx, hipMemcpyAsync(w.ddesc, hp, gbytes, hipMemcpyHostToDevice, ctx->stream),
                      "batch descriptor upload");
     }
     if (!st) st = w.enqueue_steps(ctx, 0, w.steps);

@@ -268,3 +268,68 @@ def test_grouped_gemm_route_steps_bitwise(use_graph):
             assert same_bits(s, g), rep
         torch.cuda.synchronize()
     prepared.close()
+
+
+def _random_network(seed, leaves, closed, opened, bond_bits):
+    """A connected network of `leaves` tensors on a ring with `closed` further
+    bonds between random leaves, each bond of up to bond_bits binary axes, and
+    `opened` open axes; returns (net, labels and arrays of its leaves)."""
+    rng = np.random.default_rng(seed)
+    legs = [[] for _ in range(leaves)]
+    label = 0
+    pairs = [(i, (i + 1) % leaves) for i in range(leaves)]
+    pairs += [tuple(rng.choice(leaves, 2, replace=False)) for _ in range(closed)]
+    for i, j in pairs:
+        for _ in range(int(rng.integers(1, bond_bits + 1))):
+            legs[i].append(label)
+            legs[j].append(label)
+            label += 1
+    for _ in range(opened):
+        legs[int(rng.integers(0, leaves))].append(label)
+        label += 1
+    net, arrays = ops.Network(), []
+    for l in legs:
+        rng.shuffle(l)
+        arrays.append(rng.standard_normal(1 << len(l)) + 1j * rng.standard_normal(1 << len(l)))
+        net.add([2] * len(l), l, arrays[-1])
+    net.plan(seed, 26)
+    return net, legs, arrays
+
+
+@pytest.mark.parametrize("leaves,closed,opened,bond_bits", [
+    (2, 0, 0, 1),    # one step, one element
+    (3, 0, 3, 1),    # chains of one to four steps: the pipeline's prologue
+    (4, 1, 2, 2),
+    (5, 0, 9, 1),    # results past 256 elements
+    (4, 0, 11, 3),   # leaves past the staged size, read from global memory
+    (7, 8, 3, 2),    # intermediates beyond the LDS space, read back from global memory
+    (10, 10, 0, 2),
+    (9, 4, 0, 2),    # long sums
+    (40, 6, 6, 1),   # the ring of records wraps many times
+])
+def test_chains_of_small_steps_bitwise(leaves, closed, opened, bond_bits):
+    """Small direct steps run as a chain equal the same steps run one launch at
+    a time bit for bit, and numpy within 1e-12 relative (sums of at most a few
+    hundred terms per step, some eps each)."""
+    nets, want = [], []
+    for seed in range(6):
+        net, legs, arrays = _random_network(seed, leaves, closed, opened, bond_bits)
+        nets.append(net)
+        args = []
+        for l, x in zip(legs, arrays):
+            args += [x.reshape([2] * len(l)), l]
+        want.append((args, sorted(v for v in sum(legs, []) if sum(legs, []).count(v) == 1)))
+    solo = [n.run() for n in nets]
+    batch, _ = ops.run_networks(nets)
+    prepared = ops.NetworkBatch(nets, use_graph=True)
+    for _ in range(2):
+        for s, b, g in zip(solo, batch, prepared.run()):
+            assert same_bits(s, b)
+            assert same_bits(s, g)
+    prepared.close()
+    for s, (args, out) in zip(solo, want):
+        if len(set(sum(args[1::2], []))) > 50:
+            continue  # more labels than einsum has letters
+        ref = np.einsum(*args, out, optimize="greedy").reshape(-1)
+        for x, y in ((s.real, ref.real), (s.imag, ref.imag)):  # the plan's result axes are in an order of its own
+            assert np.linalg.norm(np.sort(x) - np.sort(y)) <= 1e-12 * np.linalg.norm(ref)
