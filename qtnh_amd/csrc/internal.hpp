@@ -83,6 +83,19 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Last of the nd entries of a launch's work list, whose first blocks ascend from
+// 0, that begins at or before blk: the lanes look at 64 entries at a time (a
+// binary search would wait for memory once a halving).  Every lane must be active.
+template <typename Desc>
+__device__ __forceinline__ int find_entry(const Desc *d, int nd, uint64_t blk) {
+  int n = 0;
+  for (int i = 0; i < nd; i += 64) {
+    const int j = i + (int)(threadIdx.x & 63);
+    n += __popcll(__ballot(j < nd && d[j].first <= blk));
+  }
+  return __builtin_amdgcn_readfirstlane(n - 1);
+}
+
 // Row-major size with overflow detection; false on overflow.
 bool checked_size(int rank, const uint64_t *dims, uint64_t *n);
 
@@ -206,14 +219,19 @@ struct SkDesc {
   uint64_t N, K, kc, S, MN;
   uint64_t first, first2;
 };
-// A bit permutation (every dim a power of two): element j of dst is element
-// sum_p bit_p(j) << sbit[p] of src; 1024 elements per block.
+// A bit permutation (every dim a power of two) in tiles of 2^tile elements, one
+// per block.  All entries are offsets that are XORed together: bit i of a tile's
+// element moves the source and the LDS slot in load order, the result and the
+// LDS slot in store order; bit i of the tile's index moves source and result.
+constexpr int kPermTileBits = 10, kPermMaxBits = 32;
 struct PermDesc {
   const c128 *src;
   c128 *dst;
-  uint64_t n, first;
-  int nb;
-  int8_t sbit[64];
+  uint64_t first;  // first block in the launch
+  uint32_t tile, blocks;
+  uint32_t load_src[kPermTileBits], load_lds[kPermTileBits];
+  uint32_t store_dst[kPermTileBits], store_lds[kPermTileBits];
+  uint32_t tile_src[kPermMaxBits - kPermTileBits], tile_dst[kPermMaxBits - kPermTileBits];
 };
 qtnh_status launch_zgemm_grouped(qtnh_ctx_t ctx, int tile, const ZGroupDesc *d, int nd, uint64_t total_blocks);
 qtnh_status launch_zgemm_grouped_sum(qtnh_ctx_t ctx, const ZSumDesc *d, int nd, uint64_t total_blocks);
@@ -226,9 +244,8 @@ int zgemm_group_tile(uint64_t M, uint64_t N);
 void zgemm_chunk_shape(uint64_t M, uint64_t N, uint64_t K, uint64_t *kc, uint64_t *nchunks);
 // Terms per chunk of the split-K route (a multiple of its workgroup size).
 uint64_t splitk_chunk_len(uint64_t K, uint64_t chunks);
-// Source bit of every result bit of a permutation of power-of-two dims
-// (false when a dim is not a power of two).
-bool permute_source_bits(int rank, const uint64_t *dims, const uint16_t *ptup, int *nb, int8_t *sbit);
+// The tiles of a permutation (false when a dim is no power of two or the tensor has more than 2^32 elements).
+bool plan_permute_tiles(int rank, const uint64_t *dims, const uint16_t *ptup, PermDesc *d);
 
 // Split-precision complex GEMM C[MxN] = A[MxK] * B (all contiguous, row-major)
 // on INT8 matrix cores, B given as B[KxN] (b_cols) or as Bt[NxK]; scratch of

@@ -1327,9 +1327,9 @@ struct Wave {
             R.split)
           continue;
         PermDesc pa, pb, pc;
-        if ((!R.idA && !permute_source_bits((int)A.dims.size(), A.dims.data(), R.pA.data(), &pa.nb, pa.sbit)) ||
-            (!R.idB && !permute_source_bits((int)B.dims.size(), B.dims.data(), R.pB.data(), &pb.nb, pb.sbit)) ||
-            (!R.idC && !permute_source_bits((int)Cn.dims.size(), R.dn.data(), R.pC.data(), &pc.nb, pc.sbit)))
+        if ((!R.idA && !plan_permute_tiles((int)A.dims.size(), A.dims.data(), R.pA.data(), &pa)) ||
+            (!R.idB && !plan_permute_tiles((int)B.dims.size(), B.dims.data(), R.pB.data(), &pb)) ||
+            (!R.idC && !plan_permute_tiles((int)Cn.dims.size(), R.dn.data(), R.pC.data(), &pc)))
           continue;
         grouped[i][s] = 1;
         const c128 *Ap = node_ptr(n, blocks[i], st.a), *Bp = node_ptr(n, blocks[i], st.b);
@@ -1337,18 +1337,16 @@ struct Wave {
         const c128 *Aw = R.idA ? Ap : (const c128 *)(w + R.offA);
         const c128 *Bw = R.idB ? Bp : (const c128 *)(w + R.offB);
         c128 *Cw = R.idC ? Cp : (c128 *)(w + R.offC);
-        auto add_perm = [](std::vector<PermDesc> &v, GRange &r, PermDesc d, const c128 *src, c128 *dst,
-                           uint64_t count) {
+        auto add_perm = [](std::vector<PermDesc> &v, GRange &r, PermDesc d, const c128 *src, c128 *dst) {
           d.src = src;
           d.dst = dst;
-          d.n = count;
           d.first = r.blocks;
-          r.blocks += (count + 1023) / 1024;
+          r.blocks += d.blocks;
           v.push_back(d);
           r.e = (uint32_t)v.size();
         };
-        if (!R.idA) add_perm(pin, r_pin[s], pa, Ap, (c128 *)Aw, R.M * R.K);
-        if (!R.idB) add_perm(pin, r_pin[s], pb, Bp, (c128 *)Bw, R.K * R.N);
+        if (!R.idA) add_perm(pin, r_pin[s], pa, Ap, (c128 *)Aw);
+        if (!R.idB) add_perm(pin, r_pin[s], pb, Bp, (c128 *)Bw);
         if (R.splitk) {
           SkDesc d;
           d.A = Aw;
@@ -1397,7 +1395,7 @@ struct Wave {
             r_zsum[s].e = (uint32_t)zsum.size();
           }
         }
-        if (!R.idC) add_perm(pout, r_pout[s], pc, Cw, Cp, R.nC);
+        if (!R.idC) add_perm(pout, r_pout[s], pc, Cw, Cp);
       }
     }
   }

@@ -1197,59 +1197,124 @@ qtnh_status launch_swap(qtnh_ctx_t ctx, c128 *buf, int rank, const uint64_t *dim
 
 
 namespace {
-// Many bit permutations in one launch (the small operand permutes of a
-// network batch's steps): block b of descriptor D moves dst elements
-// [1024 b, 1024 b + 1024) of D, thread t the elements 1024 b + t + 256 i,
-// so each store instruction writes 4 KiB of consecutive elements.  The source
-// offset of an element splits over its disjoint bits: that of the block's
-// base (bits 10 and up) OR that of t + 256 i (bits 0..9).
-__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd,
-                                                              uint64_t total) {
-  for (uint64_t blk = blockIdx.x; blk < total; blk += gridDim.x) {
-    int lo = 0, hi = nd - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (d[mid].first <= blk)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const PermDesc &D = d[lo];
-    const uint64_t base = (blk - D.first) << 10;
-    uint64_t sbase = 0;
-    for (int p = 10; p < D.nb; ++p)
-      if ((base >> p) & 1ull) sbase |= 1ull << D.sbit[p];
-    const int lowbits = D.nb < 10 ? D.nb : 10;
+// Many bit permutations in one launch (the operand permutes of a network
+// batch's steps), one tile per block: a tile holds the 32 elements that are
+// consecutive in the source and in the result around each of its elements, so
+// both sides move 512-byte runs, and turns its order round in LDS (memory is the
+// bound; 16 KB a block lets ten of them share a compute unit).  36 permutes of
+// 2^12 to 2^20 elements, 142 MB in all: 47 us, and 154 us with every element
+// gathered by a source offset put together from its result index.
+__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd) {
+  __shared__ double2_t tile[1 << kPermTileBits];
+  const PermDesc &D = d[find_entry(d, nd, blockIdx.x)];
+  const uint32_t t = blockIdx.x - (uint32_t)D.first, tid = threadIdx.x;
+  uint32_t so = 0, to = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t low = threadIdx.x + 256u * i;
-      const uint64_t j = base + low;
-      if (j >= D.n) continue;
-      uint64_t s = sbase;
-      for (int p = 0; p < lowbits; ++p)
-        if ((low >> p) & 1u) s |= 1ull << D.sbit[p];
-      D.dst[j] = D.src[s];
-    }
+  for (int p = 0; p < kPermMaxBits - kPermTileBits; ++p) {
+    const uint32_t on = 0u - ((t >> p) & 1u);
+    so ^= on & D.tile_src[p];
+    to ^= on & D.tile_dst[p];
+  }
+  uint32_t ls = 0, ll = 0, ss = 0, sl = 0;
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const uint32_t on = 0u - ((tid >> p) & 1u);
+    ls ^= on & D.load_src[p];
+    ll ^= on & D.load_lds[p];
+    ss ^= on & D.store_dst[p];
+    sl ^= on & D.store_lds[p];
+  }
+  const double2_t *src = reinterpret_cast<const double2_t *>(D.src);
+  double2_t *dst = reinterpret_cast<double2_t *>(D.dst);
+  if (D.tile == kPermTileBits) {
+    double2_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = src[so ^ ls ^ (i & 1 ? D.load_src[8] : 0u) ^ (i & 2 ? D.load_src[9] : 0u)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tile[ll ^ (i & 1 ? D.load_lds[8] : 0u) ^ (i & 2 ? D.load_lds[9] : 0u)] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      dst[to ^ ss ^ (i & 1 ? D.store_dst[8] : 0u) ^ (i & 2 ? D.store_dst[9] : 0u)] =
+          tile[sl ^ (i & 1 ? D.store_lds[8] : 0u) ^ (i & 2 ? D.store_lds[9] : 0u)];
+    return;
+  }
+  // A tensor of fewer elements than a tile.
+  for (uint32_t e = tid; e < (1u << D.tile); e += 256) {
+    const bool b8 = e & 256;
+    tile[ll ^ (b8 ? D.load_lds[8] : 0u)] = src[ls ^ (b8 ? D.load_src[8] : 0u)];
+  }
+  __syncthreads();
+  for (uint32_t e = tid; e < (1u << D.tile); e += 256) {
+    const bool b8 = e & 256;
+    dst[ss ^ (b8 ? D.store_dst[8] : 0u)] = tile[sl ^ (b8 ? D.store_lds[8] : 0u)];
   }
 }
 }  // namespace
 
-bool permute_source_bits(int rank, const uint64_t *dims, const uint16_t *ptup, int *nb, int8_t *sbit) {
+bool plan_permute_tiles(int rank, const uint64_t *dims, const uint16_t *ptup, PermDesc *d) {
   uint64_t nd[kMaxRank];
   for (int i = 0; i < rank; ++i) nd[ptup[i]] = dims[i];
   const BitLayout in = bit_layout(rank, dims);
   const BitLayout out = bit_layout(rank, nd);
-  if (!in.binary || !out.binary || in.nbits > 64) return false;
+  if (!in.binary || !out.binary || in.nbits > kPermMaxBits) return false;
+  const int nb = in.nbits;
+  int sbit[kPermMaxBits], rbit[kPermMaxBits];  // source bit of each result bit, and back
   for (int i = 0; i < rank; ++i)
-    for (int t = 0; t < in.width[i]; ++t) sbit[out.shift[ptup[i]] + t] = (int8_t)(in.shift[i] + t);
-  *nb = in.nbits;
+    for (int t = 0; t < in.width[i]; ++t) {
+      sbit[out.shift[ptup[i]] + t] = in.shift[i] + t;
+      rbit[in.shift[i] + t] = out.shift[ptup[i]] + t;
+    }
+  // The tile's result bits: the lowest of the result and of the source in turn.
+  const int tile = std::min(nb, kPermTileBits);
+  uint32_t in_tile = 0;
+  for (int i = 0; __builtin_popcount(in_tile) < tile; ++i) {
+    in_tile |= 1u << i;
+    if (__builtin_popcount(in_tile) < tile) in_tile |= 1u << rbit[i];
+  }
+  memset(d, 0, sizeof(*d));
+  d->tile = (uint32_t)tile;
+  d->blocks = 1u << (nb - tile);
+  int slot[kPermMaxBits];  // place of a result bit of the tile in store order
+  for (int p = 0, i = 0, h = 0; p < nb; ++p) {
+    if (in_tile >> p & 1) {
+      slot[p] = i;
+      d->store_dst[i] = 1u << p;
+      d->store_lds[i] = 1u << i;
+      ++i;
+    } else {
+      d->tile_dst[h] = 1u << p;
+      d->tile_src[h] = 1u << sbit[p];
+      ++h;
+    }
+  }
+  for (int q = 0, i = 0; q < nb; ++q)
+    if (in_tile >> rbit[q] & 1) {
+      d->load_src[i] = 1u << q;
+      d->load_lds[i] = 1u << slot[rbit[q]];
+      ++i;
+    }
+  // Eight consecutive lanes cover all LDS banks in store order.  So that they do
+  // in load order too, slot bits that its lowest three bits set above these
+  // three are added to the ones of the three that they leave out.
+  uint32_t free_bits = 7;
+  for (int i = 0; i < std::min(tile, 3); ++i) free_bits &= ~d->load_lds[i];
+  for (int i = 0; i < std::min(tile, 3); ++i) {
+    const uint32_t bit = d->load_lds[i];
+    if (bit < 8 || !free_bits) continue;
+    const uint32_t add = free_bits & (0u - free_bits);
+    free_bits ^= add;
+    for (int j = 0; j < tile; ++j)
+      if (d->store_lds[j] == bit) d->store_lds[j] |= add;
+    d->load_lds[i] |= add;
+  }
   return true;
 }
 
 qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, uint64_t total) {
   if (nd <= 0 || total == 0) return QTNH_OK;
-  const unsigned grid = (unsigned)std::min<uint64_t>(total, (uint64_t)ctx->num_cus * 16);
-  hipLaunchKernelGGL(permute_grouped_kernel, dim3(grid), dim3(256), 0, ctx->stream, d, nd, total);
+  hipLaunchKernelGGL(permute_grouped_kernel, dim3((unsigned)total), dim3(256), 0, ctx->stream, d, nd);
   return check_hip(ctx, hipGetLastError(), "grouped permute launch");
 }
 

@@ -333,3 +333,32 @@ def test_chains_of_small_steps_bitwise(leaves, closed, opened, bond_bits):
         ref = np.einsum(*args, out, optimize="greedy").reshape(-1)
         for x, y in ((s.real, ref.real), (s.imag, ref.imag)):  # the plan's result axes are in an order of its own
             assert np.linalg.norm(np.sort(x) - np.sort(y)) <= 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (2, 14, 5),   # an operand of 2^7 elements
+    (12, 2, 7),   # 2^9
+    (11, 2, 8),   # one tile, 2^10
+    (4, 7, 10),
+    (4, 5, 12),
+    (3, 3, 14),
+])
+def test_grouped_permutes_of_any_axis_order_bitwise(m, n, k):
+    """The operand permutes of grouped steps (tensors smaller than, as large as
+    and larger than a tile; shuffled axes) equal the ungrouped ones bit for bit."""
+    nets = []
+    for seed in range(4):
+        rng = np.random.default_rng(seed)
+        net = ops.Network()
+        for l in (list(range(m)) + list(range(m + n, m + n + k)), list(range(m, m + n + k))):
+            rng.shuffle(l)
+            net.add([2] * len(l), l, rng.standard_normal(1 << len(l)) + 1j * rng.standard_normal(1 << len(l)))
+        nets.append(net.plan(0, 64))
+    solo = [x.run() for x in nets]
+    batch, _ = ops.run_networks(nets)
+    prepared = ops.NetworkBatch(nets, use_graph=False)
+    assert prepared.stats()["grouped_gemm"] == 4
+    for s, b, g in zip(solo, batch, prepared.run()):
+        assert same_bits(s, b)
+        assert same_bits(s, g)
+    prepared.close()
