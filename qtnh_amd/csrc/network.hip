@@ -34,79 +34,199 @@ namespace qtnh_hip {
 namespace {
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
+// A pointer read from memory has no known address space: accesses through it
+// would be flat ones, which count as LDS accesses too.
+using GlobalIn = const __attribute__((address_space(1))) double2_t *;
+using GlobalOut = __attribute__((address_space(1))) double2_t *;
 
 constexpr int kGThreads = 256;
 constexpr int kGMaxBits = 32;
 
-// A small contraction over binary (dim 2) axes, as bit maps.
-struct GDesc {
-  const double2_t *A;
-  const double2_t *B;
-  double2_t *C;
-  uint64_t first;  // first block of this contraction in the launch
-  uint64_t nC;
-  int ncb;         // result bits
-  int kbits;       // closed bits
+// A contraction over binary (dim 2) axes, as bit maps.
+struct StepBits {
+  int ncb, kbits;          // result bits, closed bits
   int8_t abit[kGMaxBits];  // A bit feeding result bit p (-1: from B)
   int8_t bbit[kGMaxBits];
   int8_t ka[kGMaxBits];    // A bit of closed bit j (j = 0: last wire in the sum order)
   int8_t kb[kGMaxBits];
 };
 
-__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd,
-                                                                   uint64_t total_blocks) {
-  // Counting the closed tuple t up by one flips its bits 0 .. ctz(t + 1): the
-  // A / B offset changes by the prefix masks below (one XOR per term).
-  __shared__ uint64_t flip_a[64], flip_b[64];
-  for (uint64_t blk = blockIdx.x; blk < total_blocks; blk += gridDim.x) {
-    int lo = 0, hi = nd - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (descs[mid].first <= blk)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const GDesc &D = descs[lo];
-    __syncthreads();  // the previous block's readers are done with the masks
-    if ((int)threadIdx.x < D.kbits) {
-      uint64_t fa = 0, fb = 0;
-      for (int j = 0; j <= (int)threadIdx.x; ++j) {
-        fa |= 1ull << D.ka[j];
-        fb |= 1ull << D.kb[j];
+// A direct contraction in a grouped launch.  All tables hold offsets that are
+// XORed together: result bits that number the threads move A or B, and C; the
+// register bits number the 2^ta x 2^tb results of a thread; counting the closed
+// tuple t up by one flips entry ctz(t + 1).
+constexpr int kGMaxTerms = 12;  // log2 of the terms (direct contractions have at most 2^10)
+enum : uint32_t { kGWide = 16 };
+// One wave per result from 2^6 terms and up to 2^8 results: 18 contractions of
+// 2^6 results with 2^7 to 2^9 terms took 74 us with a thread each, 9 us so; seven of 2^12
+// results with 2^7 terms 21 us with a thread each, 46 us with a wave.  Register
+// tiles of 4 and 16 results where enough threads remain: 22 contractions of 2^12
+// to 2^18 results took 70 us without, 27 us with (two more or fewer bits at either
+// line: no difference).
+constexpr int kGWideMinBits = 6, kGWideMaxResult = 8, kGTile4 = 14, kGTile16 = 18;
+struct GDesc {
+  const double2_t *A;
+  const double2_t *B;
+  double2_t *C;
+  uint64_t first;          // first block of this contraction in the launch
+  uint32_t blocks;
+  uint32_t kind;           // ta | tb << 2, or kGWide: one wave per result
+  uint32_t nb, kbits;      // log2 of the threads' results outside the register tile, of the terms
+  uint32_t reg_a[2], reg_b[2];    // register bits: offset in A, in B
+  uint32_t reg_ca[2], reg_cb[2];  // ... and in C
+  uint32_t flip_a[kGMaxTerms], flip_b[kGMaxTerms];
+  uint32_t a[kGMaxBits], b[kGMaxBits], c[kGMaxBits];
+};
+
+__device__ __forceinline__ void product_add(double &ar, double &ai, double2_t a, double2_t b) {
+  double pr, pi;
+  cmul_parts(a.x, a.y, b.x, b.y, &pr, &pi);
+  ar = ar + pr;
+  ai = ai + pi;
+}
+
+// The results of one thread.  The operands of TU terms are requested before
+// their products are added, in the order of the closed tuples.
+template <int TA, int TB>
+__device__ __forceinline__ void direct_tile(const GDesc &D, uint32_t x, uint32_t y, uint32_t z) {
+  constexpr int NA = 1 << TA, NB = 1 << TB, TU = NA * NB > 4 ? 2 : 4;
+  GlobalIn pa[NA], pb[NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) pa[i] = (GlobalIn)D.A + ((i & 1 ? D.reg_a[0] : 0u) | (i & 2 ? D.reg_a[1] : 0u));
+#pragma unroll
+  for (int i = 0; i < NB; ++i) pb[i] = (GlobalIn)D.B + ((i & 1 ? D.reg_b[0] : 0u) | (i & 2 ? D.reg_b[1] : 0u));
+  double re[NA][NB], im[NA][NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) re[i][j] = im[i][j] = 0.0;
+  const uint32_t K = 1u << D.kbits, f0 = D.flip_a[0], g0 = D.flip_b[0], f1 = D.flip_a[1], g1 = D.flip_b[1];
+  double2_t va[TU][NA], vb[TU][NB];
+  auto get = [&](int u, uint32_t xa, uint32_t xb) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) va[u][i] = pa[i][xa];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) vb[u][j] = pb[j][xb];
+  };
+  auto mac = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) product_add(re[i][j], im[i][j], va[u][i], vb[u][j]);
+  };
+  if (K < TU) {
+    get(0, x, y);
+    if (K == 2) get(1, x ^ f0, y ^ g0);
+    mac(0);
+    if (K == 2) mac(1);
+  } else {
+    for (uint32_t t = 0;;) {
+      get(0, x, y);
+      get(1, x ^= f0, y ^= g0);
+      if constexpr (TU == 4) {
+        get(2, x ^= f1, y ^= g1);
+        get(3, x ^= f0, y ^= g0);
       }
-      flip_a[threadIdx.x] = fa;
-      flip_b[threadIdx.x] = fb;
+#pragma unroll
+      for (int u = 0; u < TU; ++u) mac(u);
+      t += TU;
+      if (t == K) break;
+      const int c = __builtin_ctz(t);
+      x ^= D.flip_a[c];
+      y ^= D.flip_b[c];
     }
-    __syncthreads();
-    const uint64_t e = (blk - D.first) * kGThreads + threadIdx.x;
-    if (e >= D.nC) continue;
-    uint64_t oa = 0, ob = 0;
-    for (int p = 0; p < D.ncb; ++p) {
-      if (!((e >> p) & 1ull)) continue;
-      if (D.abit[p] >= 0)
-        oa |= 1ull << D.abit[p];
-      else
-        ob |= 1ull << D.bbit[p];
+  }
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      ((GlobalOut)D.C)[z ^ (i & 1 ? D.reg_ca[0] : 0u) ^ (i & 2 ? D.reg_ca[1] : 0u) ^ (j & 1 ? D.reg_cb[0] : 0u) ^
+          (j & 2 ? D.reg_cb[1] : 0u)] = double2_t{re[i][j], im[i][j]};
+}
+
+// Direct contractions of many networks' steps in one launch.  Loads bound them:
+// of the two a product takes, a thread of 2^ta x 2^tb results shares each among
+// as many products.  Sums of few results and 64 terms or more (closing steps)
+// are a chain of dependent loads and additions for a thread: there each wave
+// takes one result, its lanes form the products of 64 terms at a time, and only
+// the additions follow one another.
+__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd) {
+  __shared__ double2_t prod[kGThreads];
+  const GDesc &D = descs[find_entry(descs, nd, blockIdx.x)];
+  const uint32_t tid = threadIdx.x, kind = D.kind, nb = D.nb;
+  const uint32_t wide = kind == kGWide;
+  // Thread's number among the results: low part from the lane, the rest (hi) of the block.
+  const uint32_t block = blockIdx.x - (uint32_t)D.first;
+  const uint32_t low = wide ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)) | (block << 2 & 255u) : tid;
+  const uint32_t hi = wide ? block >> 6 : block;
+  if (low >= (nb < 8 ? 1u << nb : 256u)) return;
+  uint32_t x = 0, y = 0, z = 0;
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const uint32_t on = 0u - (hi >> p & 1u);
+    x ^= on & D.a[8 + p];
+    y ^= on & D.b[8 + p];
+    z ^= on & D.c[8 + p];
+  }
+  if (nb > 16) {
+#pragma unroll
+    for (int p = 8; p < kGMaxBits - 8; ++p) {
+      const uint32_t on = 0u - (hi >> p & 1u);
+      x ^= on & D.a[8 + p];
+      y ^= on & D.b[8 + p];
+      z ^= on & D.c[8 + p];
     }
-    // Closed tuples in the reference order: the tuple index counts up with the
-    // last wire fastest (bit 0).
-    double ar = 0.0, ai = 0.0;
-    const uint64_t K = 1ull << D.kbits;
-    uint64_t xa = oa, xb = ob;
-    for (uint64_t t = 0; t < K; ++t) {
-      const double2_t a = D.A[xa], b = D.B[xb];
+  }
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const uint32_t on = 0u - (low >> p & 1u);
+    x ^= on & D.a[p];
+    y ^= on & D.b[p];
+    z ^= on & D.c[p];
+  }
+  if (wide) {
+    const uint32_t lane = tid & 63, K = 1u << D.kbits;
+    double2_t *mine = prod + (tid & ~63u);
+    uint32_t xl = x, yl = y;
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+      const uint32_t on = 0u - (lane >> p & 1u);
+      xl ^= on & (D.flip_a[p] ^ (p ? D.flip_a[p - 1] : 0u));
+      yl ^= on & (D.flip_b[p] ^ (p ? D.flip_b[p - 1] : 0u));
+    }
+    double sum = 0.0;  // lane 0: real part, lane 1: imaginary part
+    double2_t a = ((GlobalIn)D.A)[xl], b = ((GlobalIn)D.B)[yl];
+    for (uint32_t t = 64;; t += 64) {
       double pr, pi;
       cmul_parts(a.x, a.y, b.x, b.y, &pr, &pi);
-      ar = ar + pr;
-      ai = ai + pi;
-      if (t + 1 < K) {
-        const int c = __builtin_ctzll(t + 1);
-        xa ^= flip_a[c];
-        xb ^= flip_b[c];
+      mine[lane] = double2_t{pr, pi};
+      if (t < K) {  // the next terms' operands arrive during the additions
+        const int c = __builtin_ctz(t);
+        xl ^= D.flip_a[c] ^ D.flip_a[5];
+        yl ^= D.flip_b[c] ^ D.flip_b[5];
+        a = ((GlobalIn)D.A)[xl];
+        b = ((GlobalIn)D.B)[yl];
       }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const double *part = reinterpret_cast<const double *>(mine) + (lane & 1);
+#pragma unroll 16
+      for (int i = 0; i < 64; ++i) sum = sum + part[2 * i];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (t >= K) break;
     }
-    D.C[e] = double2_t{ar, ai};
+    if (lane < 2) ((__attribute__((address_space(1))) double *)(D.C + z))[lane] = sum;
+    return;
+  }
+  switch (kind) {
+    case 0: direct_tile<0, 0>(D, x, y, z); break;
+    case 1 | 1 << 2: direct_tile<1, 1>(D, x, y, z); break;
+    case 2 | 2 << 2: direct_tile<2, 2>(D, x, y, z); break;
+    case 2: direct_tile<2, 0>(D, x, y, z); break;
+    default: direct_tile<0, 2>(D, x, y, z); break;
   }
 }
 
@@ -145,19 +265,7 @@ struct ChainDesc {
   uint32_t first, count;
 };
 
-// A pointer read from LDS has no known address space: accesses through it would
-// be flat ones, which the LDS barrier waits for.
-using GlobalIn = const __attribute__((address_space(1))) double2_t *;
-using GlobalOut = __attribute__((address_space(1))) double2_t *;
-
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-
-__device__ __forceinline__ void chain_mac(double &ar, double &ai, double2_t a, double2_t b) {
-  double pr, pi;
-  cmul_parts(a.x, a.y, b.x, b.y, &pr, &pi);
-  ar = ar + pr;
-  ai = ai + pi;
-}
 
 // Chains, one workgroup each.  What bounds them is latency, step after step:
 // so intermediates stay in LDS where they fit (a step's result goes to global
@@ -185,18 +293,18 @@ __device__ __forceinline__ void chain_step_elements(const ChainStep &D, double2_
     for (int p = 8; p < kChainBits; ++p) x ^= (0u - ((e >> p) & 1u)) & D.mask[p];
     double ar = 0.0, ai = 0.0;
     if (K < 4) {
-      chain_mac(ar, ai, get_a(x), get_b(x));
-      if (K == 2) chain_mac(ar, ai, get_a(x ^ f0), get_b(x ^ f0));
+      product_add(ar, ai, get_a(x), get_b(x));
+      if (K == 2) product_add(ar, ai, get_a(x ^ f0), get_b(x ^ f0));
     } else {
       // Four terms' operands are requested before their products are added, in order.
       for (uint32_t t = 0;;) {
         const uint32_t x1 = x ^ f0, x2 = x1 ^ f1, x3 = x2 ^ f0;
         const double2_t a0 = get_a(x), a1 = get_a(x1), a2 = get_a(x2), a3 = get_a(x3);
         const double2_t b0 = get_b(x), b1 = get_b(x1), b2 = get_b(x2), b3 = get_b(x3);
-        chain_mac(ar, ai, a0, b0);
-        chain_mac(ar, ai, a1, b1);
-        chain_mac(ar, ai, a2, b2);
-        chain_mac(ar, ai, a3, b3);
+        product_add(ar, ai, a0, b0);
+        product_add(ar, ai, a1, b1);
+        product_add(ar, ai, a2, b2);
+        product_add(ar, ai, a3, b3);
         t += 4;
         if (t == K) break;
         x = x3 ^ D.flip[__builtin_ctz(t) - 2];
@@ -302,14 +410,14 @@ __global__ void __launch_bounds__(kGThreads + 64) chain_direct_kernel(const Chai
               const uint32_t x2 = x ^ h.z ^ h.w, p2 = h.x + x2, p3 = h.x + (x2 ^ h.z);
               const double2_t a2 = lds[p2 & 0xffffu], b2 = lds[p2 >> 16], a3 = lds[p3 & 0xffffu], b3 = lds[p3 >> 16];
               head(k + 1, hn, xn);
-              chain_mac(ar, ai, a0, b0);
-              chain_mac(ar, ai, a1, b1);
-              chain_mac(ar, ai, a2, b2);
-              chain_mac(ar, ai, a3, b3);
+              product_add(ar, ai, a0, b0);
+              product_add(ar, ai, a1, b1);
+              product_add(ar, ai, a2, b2);
+              product_add(ar, ai, a3, b3);
             } else {
               head(k + 1, hn, xn);
-              chain_mac(ar, ai, a0, b0);
-              chain_mac(ar, ai, a1, b1);
+              product_add(ar, ai, a0, b0);
+              product_add(ar, ai, a1, b1);
             }
             if ((uint32_t)tid < n) lds[(ctl & 0xffffu) + tid] = double2_t{ar, ai};
           } else {
@@ -401,7 +509,7 @@ struct qtnh_net_s {
   double cost = 0;  // planning objective: flops + kElemCost x elements read and written per step
   // Grouped-launch descriptor of each direct power-of-two step, without its
   // device pointers and launch position (filled in per batch placement).
-  std::vector<GDesc> gdesc;
+  std::vector<GDesc> gdesc;  // of step chain.size() + i
   // Records of the steps of the network's chain, without device pointers.
   std::vector<ChainStep> chain;
   // Device copy of leaf_data: uploaded by the first blocking run on a device
@@ -419,8 +527,7 @@ namespace {
 
 uint64_t block_elems(const qtnh_net_s &n) { return round16(n.leaf_elems) + round16(n.arena_elems); }
 
-GDesc gdesc_template(const qtnh_net_s &net, size_t s);
-void plan_chain(qtnh_net_s &net);
+void plan_direct(qtnh_net_s &net);
 
 // A network in split precision uses the split GEMM only for steps where it
 // is the faster: 128 x 128 output tiles over M x 2N (the embedded real
@@ -570,10 +677,7 @@ void finish_plan(qtnh_net_s &net) {
   }
   net.arena_elems = hw;
   net.result = net.steps.empty() ? 0 : net.steps.back().c;
-  net.gdesc.assign(net.steps.size(), GDesc{});
-  for (size_t s = 0; s < net.steps.size(); ++s)
-    if (net.steps[s].direct && net.steps[s].binary) net.gdesc[s] = gdesc_template(net, s);
-  plan_chain(net);
+  plan_direct(net);
   net.planned = true;
 }
 
@@ -969,17 +1073,12 @@ qtnh_status run_step(qtnh_ctx_t ctx, const qtnh_net_s &net, Where block, size_t 
                          node_ptr(net, block, st.c), step_precision(st, precision), nullptr, ws, ws_bytes);
 }
 
-GDesc gdesc_template(const qtnh_net_s &net, size_t s) {
+StepBits step_bits(const qtnh_net_s &net, size_t s) {
   const auto &st = net.steps[s];
   const auto &A = net.nodes[st.a], &B = net.nodes[st.b], &C = net.nodes[st.c];
   const int rA = (int)A.dims.size(), rB = (int)B.dims.size(), rC = (int)C.dims.size();
-  GDesc d;
+  StepBits d;
   memset(&d, -1, sizeof(d));
-  d.A = nullptr;
-  d.B = nullptr;
-  d.C = nullptr;
-  d.first = 0;
-  d.nC = C.size;
   d.ncb = rC;
   const int nw = (int)st.wires.size() / 2;
   d.kbits = nw;
@@ -1012,18 +1111,66 @@ GDesc gdesc_template(const qtnh_net_s &net, size_t s) {
   return d;
 }
 
-// The network's chain: records of its leading small direct steps.  Their
-// intermediates get LDS offsets by first fit over their lifetimes; one that
+// Descriptor of a direct step in grouped launches, without pointers.
+GDesc plan_grouped(const StepBits &g) {
+  GDesc d = {};
+  d.kbits = (uint32_t)g.kbits;
+  for (int j = 0; j < g.kbits; ++j) {
+    d.flip_a[j] = (j ? d.flip_a[j - 1] : 0u) | 1u << g.ka[j];
+    d.flip_b[j] = (j ? d.flip_b[j - 1] : 0u) | 1u << g.kb[j];
+  }
+  // Register bits: the highest result bits of A and of B, so that the lanes
+  // keep the lowest, whose elements are consecutive.
+  std::vector<int> from_a, from_b;
+  for (int p = g.ncb - 1; p >= 0; --p) (g.abit[p] >= 0 ? from_a : from_b).push_back(p);
+  size_t ta = 0, tb = 0;
+  d.kind = kGWide;
+  if (g.kbits < kGWideMinBits || g.ncb > kGWideMaxResult) {
+    if (g.ncb >= kGTile4 && !from_a.empty() && !from_b.empty()) ta = tb = 1;
+    if (g.ncb >= kGTile16 && from_a.size() > 1 && from_b.size() > 1) ta = tb = 2;
+    if (g.ncb >= kGTile4 && from_a.empty()) tb = 2;
+    if (g.ncb >= kGTile4 && from_b.empty()) ta = 2;
+    d.kind = (uint32_t)(ta | tb << 2);
+  }
+  uint64_t in_regs = 0;
+  for (size_t i = 0; i < ta; ++i) {
+    in_regs |= 1ull << from_a[i];
+    d.reg_a[i] = 1u << g.abit[from_a[i]];
+    d.reg_ca[i] = 1u << from_a[i];
+  }
+  for (size_t i = 0; i < tb; ++i) {
+    in_regs |= 1ull << from_b[i];
+    d.reg_b[i] = 1u << g.bbit[from_b[i]];
+    d.reg_cb[i] = 1u << from_b[i];
+  }
+  for (int p = 0; p < g.ncb; ++p) {
+    if (in_regs >> p & 1) continue;
+    if (g.abit[p] >= 0)
+      d.a[d.nb] = 1u << g.abit[p];
+    else
+      d.b[d.nb] = 1u << g.bbit[p];
+    d.c[d.nb++] = 1u << p;
+  }
+  const uint32_t per_block = d.kind == kGWide ? 2 : 8;  // log2 of the threads' results a block takes
+  d.blocks = d.nb > per_block ? 1u << (d.nb - per_block) : 1u;
+  return d;
+}
+
+// The network's direct steps: records of its chain, descriptors of the others.
+// The chain's intermediates get LDS offsets by first fit over their lifetimes; one that
 // does not fit, or that a step outside the chain reads, goes to its arena place.
-void plan_chain(qtnh_net_s &net) {
+void plan_direct(qtnh_net_s &net) {
   auto small = [&](int x) { return net.nodes[x].size <= kChainMaxElems; };
   size_t count = 0;
   while (count < net.steps.size()) {
     const auto &st = net.steps[count];
     if (!st.direct || !st.binary || !small(st.a) || !small(st.b) || !small(st.c)) break;
-    if (net.nodes[st.c].size << net.gdesc[count].kbits > kChainMaxProducts) break;
+    if (net.nodes[st.c].size << st.wires.size() / 2 > kChainMaxProducts) break;
     ++count;
   }
+  net.gdesc.assign(net.steps.size() - count, GDesc{});
+  for (size_t s = count; s < net.steps.size(); ++s)
+    if (net.steps[s].direct && net.steps[s].binary) net.gdesc[s - count] = plan_grouped(step_bits(net, s));
   std::vector<size_t> reader(net.nodes.size(), net.steps.size());  // step that reads a node
   for (size_t s = 0; s < net.steps.size(); ++s) reader[net.steps[s].a] = reader[net.steps[s].b] = s;
   std::vector<int64_t> slot(net.nodes.size(), -1);
@@ -1031,7 +1178,7 @@ void plan_chain(qtnh_net_s &net) {
   net.chain.assign(count, ChainStep{});
   for (size_t s = 0; s < count; ++s) {
     const auto &st = net.steps[s];
-    const GDesc &g = net.gdesc[s];
+    const StepBits g = step_bits(net, s);
     ChainStep &d = net.chain[s];
     uint32_t f = 0;
     for (int p = 0; p < g.ncb; ++p) d.mask[p] = g.abit[p] >= 0 ? 1u << g.abit[p] : (1u << g.bbit[p]) << 16;
@@ -1083,15 +1230,13 @@ ChainStep make_chain_step(const qtnh_net_s &net, Where block, size_t s) {
 // The step's descriptor for one placement of the network.
 GDesc make_gdesc(const qtnh_net_s &net, Where block, size_t s, uint64_t first) {
   const auto &st = net.steps[s];
-  GDesc d = net.gdesc[s];
+  GDesc d = net.gdesc[s - net.chain.size()];
   d.A = (const double2_t *)node_ptr(net, block, st.a);
   d.B = (const double2_t *)node_ptr(net, block, st.b);
   d.C = (double2_t *)node_ptr(net, block, st.c);
   d.first = first;
   return d;
 }
-
-uint64_t gdesc_blocks(const GDesc &d) { return (d.nC + kGThreads - 1) / kGThreads; }
 
 }  // namespace
 }  // namespace qtnh_hip
@@ -1257,7 +1402,7 @@ struct Wave {
           if (!n->steps[s].direct || !n->steps[s].binary) continue;
           const size_t k = next[s]++;
           dk[dk_off[i] + s] = (uint32_t)k;
-          dfirst[k] = gdesc_blocks(n->gdesc[s]);  // block count; prefix sums below
+          dfirst[k] = n->gdesc[s - n->chain.size()].blocks;  // block count; prefix sums below
         }
       }
       for (size_t s = 0; s < steps; ++s) {
@@ -1557,10 +1702,9 @@ struct Wave {
     for (size_t s = s0; s < s1; ++s) {
       const size_t b = starts[s], e = starts[s + 1];
       if (e > b) {
-        const uint64_t tb = hdesc[e - 1].first + gdesc_blocks(hdesc[e - 1]);
-        const unsigned grid = (unsigned)std::min<uint64_t>(tb, (uint64_t)ctx->num_cus * 16);
-        hipLaunchKernelGGL(grouped_direct_kernel, dim3(grid), dim3(kGThreads), 0, ctx->stream, ddesc + b, (int)(e - b),
-                           tb);
+        const uint64_t grid = hdesc[e - 1].first + hdesc[e - 1].blocks;
+        hipLaunchKernelGGL(grouped_direct_kernel, dim3((unsigned)grid), dim3(kGThreads), 0, ctx->stream, ddesc + b,
+                           (int)(e - b));
         qtnh_status st = check_hip(ctx, hipGetLastError(), "grouped contraction launch");
         if (st) return st;
       }

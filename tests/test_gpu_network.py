@@ -362,3 +362,32 @@ def test_grouped_permutes_of_any_axis_order_bitwise(m, n, k):
         assert same_bits(s, b)
         assert same_bits(s, g)
     prepared.close()
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (0, 15, 3), (16, 0, 4), (14, 1, 2), (1, 13, 4),    # register tiles along one operand, across both
+    (9, 9, 4), (10, 11, 1), (2, 17, 0),                # 16 results a thread; 2 terms, 1 term
+    (5, 8, 3), (2, 10, 4), (12, 1, 1),                 # one result a thread
+    (3, 3, 10), (4, 4, 9), (0, 0, 10), (1, 7, 6),      # long sums of few results
+    (5, 4, 10), (6, 6, 7),                             # ... and of more
+])
+def test_grouped_direct_steps_bitwise(m, n, k):
+    """Direct steps of several networks in one launch equal the same steps run
+    one at a time bit for bit, for shuffled axes."""
+    nets = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        net = ops.Network()
+        for l in (list(range(m)) + list(range(m + n, m + n + k)), list(range(m, m + n + k))):
+            rng.shuffle(l)
+            net.add([2] * len(l), l, rng.standard_normal(1 << len(l)) + 1j * rng.standard_normal(1 << len(l)))
+        nets.append(net.plan(0, 64))
+    solo = [x.run() for x in nets]
+    batch, _ = ops.run_networks(nets)
+    prepared = ops.NetworkBatch(nets, use_graph=True)
+    assert prepared.stats()["grouped_direct"] == 3
+    for _ in range(2):
+        for s, b, g in zip(solo, batch, prepared.run()):
+            assert same_bits(s, b)
+            assert same_bits(s, g)
+    prepared.close()
