@@ -44,8 +44,12 @@ struct GateArgs {
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
 
-// U groups per thread and iteration, all loaded before any is stored: more
-// memory requests in flight per thread.  NT: non-temporal loads and stores,
+// One group per thread: memory bounds these gates, and the state streams best
+// when the requests in flight cover few contiguous stretches.  At 2^28 and 2^26
+// elements, mean over bits 6 to 27 against two groups per thread half the state
+// apart: 1-qubit gates 1.43 -> 1.36 ms and 0.377 -> 0.337 ms, 2-qubit gates
+// 1.52 -> 1.48 ms and 0.399 -> 0.367 ms, with few_workgroups() below.
+// NT: non-temporal loads and stores,
 // used when the lowest gate bit is >= 3, so that the 64 lanes of each load
 // cover whole 128-byte lines (with lower gate bits the lanes of one load are
 // strided inside lines, and the next load of the same lines must hit in cache).
@@ -60,46 +64,36 @@ template <int KB, bool NT>
 __global__ void __launch_bounds__(kGateThreads) gate_bits_kernel(c128 *__restrict__ psi, GateArgs<KB> args,
                                                                  uint64_t n_groups) {
   constexpr int K = 1 << KB;
-  constexpr int U = KB <= 2 ? 2 : 1;
   double2_t *p2 = reinterpret_cast<double2_t *>(psi);
   const uint64_t stride = (uint64_t)gridDim.x * kGateThreads;
-  for (uint64_t g0 = (uint64_t)blockIdx.x * kGateThreads + threadIdx.x; g0 < n_groups; g0 += stride * U) {
-    uint64_t base[U];
-    double2_t in[U][K];
+  for (uint64_t g = (uint64_t)blockIdx.x * kGateThreads + threadIdx.x; g < n_groups; g += stride) {
+    uint64_t base = g;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t g = g0 + u * stride;
-      uint64_t b = g < n_groups ? g : g0;
-#pragma unroll
-      for (int j = 0; j < KB; ++j) {
-        const int p = args.zpos[j];
-        b = ((b >> p) << (p + 1)) | (b & ((1ull << p) - 1));
-      }
-      base[u] = b;
-#pragma unroll
-      for (int c = 0; c < K; ++c) in[u][c] = NT ? __builtin_nontemporal_load(p2 + b + args.comb[c]) : p2[b + args.comb[c]];
+    for (int j = 0; j < KB; ++j) {
+      const int p = args.zpos[j];
+      base = ((base >> p) << (p + 1)) | (base & ((1ull << p) - 1));
     }
+    double2_t in[K];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (g0 + u * stride >= n_groups) continue;
+    for (int c = 0; c < K; ++c)
+      in[c] = NT ? __builtin_nontemporal_load(p2 + base + args.comb[c]) : p2[base + args.comb[c]];
 #pragma unroll
-      for (int o = 0; o < K; ++o) {
-        int oc = o;
-        if (KB == 3) asm volatile("" : "+s"(oc));
-        double ar = 0.0, ai = 0.0;
+    for (int o = 0; o < K; ++o) {
+      int oc = o;
+      if (KB == 3) asm volatile("" : "+s"(oc));
+      double ar = 0.0, ai = 0.0;
 #pragma unroll
-        for (int i = 0; i < K; ++i) {
-          const c128 x = {in[u][i].x, in[u][i].y};
-          const c128 gg = KB == 3 ? args.g[K * oc + i] : args.g[i * K + o];
-          const c128 pr = cmul(x, gg);
-          ar = ar + pr.re;
-          ai = ai + pr.im;
-        }
-        if (NT)
-          __builtin_nontemporal_store(double2_t{ar, ai}, p2 + base[u] + args.comb[o]);
-        else
-          p2[base[u] + args.comb[o]] = double2_t{ar, ai};
+      for (int i = 0; i < K; ++i) {
+        const c128 x = {in[i].x, in[i].y};
+        const c128 gg = KB == 3 ? args.g[K * oc + i] : args.g[i * K + o];
+        const c128 pr = cmul(x, gg);
+        ar = ar + pr.re;
+        ai = ai + pr.im;
       }
+      if (NT)
+        __builtin_nontemporal_store(double2_t{ar, ai}, p2 + base + args.comb[o]);
+      else
+        p2[base + args.comb[o]] = double2_t{ar, ai};
     }
   }
 }
@@ -474,6 +468,19 @@ qtnh_status launch_gate_lanes(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *
   return check_hip(ctx, hipGetLastError(), "gate launch");
 }
 
+// LDS asked for (and not used) so that three workgroups share a compute unit's 160 KB.
+constexpr unsigned kGateLds = 53000;
+
+// Whether a compute unit takes three workgroups instead of the seven or eight that
+// fit: 1-qubit gates on bits 6 to 23 of 2^28 elements take 1.26 to 1.48 ms
+// so and 1.28 to 1.56 with all (bits 25 to 27: within 2%), 2-qubit gates 2% less
+// on average unless both bits are high (25 and 20: 1.83 against 1.75 ms, 21 and 20:
+// 1.87 against 1.75), 3-qubit gates 3% more as often as less.
+template <int KB>
+bool few_workgroups(const int *ascending_bits) {
+  return KB == 1 || (KB == 2 && ascending_bits[0] < 19);
+}
+
 template <int KB>
 qtnh_status launch_gate_bits(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *msb_bits, const double *G) {
   constexpr int K = 1 << KB;
@@ -502,12 +509,13 @@ qtnh_status launch_gate_bits(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *m
     return launch_gate_lanes<KB, (KB >= 3 ? 2 : 0)>(ctx, psi, n, msb_bits, G);
   }
   const uint64_t groups = n >> KB;
-  constexpr int U = KB <= 2 ? 2 : 1;
-  unsigned blocks = grid_for((groups + U - 1) / U, kGateThreads, g_stream_blocks);
+  const unsigned blocks = grid_for(groups, kGateThreads, g_stream_blocks);
+  const unsigned lds = few_workgroups<KB>(args.zpos) ? kGateLds : 0;
   if (args.zpos[0] >= 3)
-    hipLaunchKernelGGL((gate_bits_kernel<KB, true>), dim3(blocks), dim3(kGateThreads), 0, ctx->stream, psi, args, groups);
+    hipLaunchKernelGGL((gate_bits_kernel<KB, true>), dim3(blocks), dim3(kGateThreads), lds, ctx->stream, psi, args,
+                       groups);
   else
-    hipLaunchKernelGGL((gate_bits_kernel<KB, false>), dim3(blocks), dim3(kGateThreads), 0, ctx->stream, psi, args,
+    hipLaunchKernelGGL((gate_bits_kernel<KB, false>), dim3(blocks), dim3(kGateThreads), lds, ctx->stream, psi, args,
                        groups);
   return check_hip(ctx, hipGetLastError(), "gate launch");
 }
