@@ -106,66 +106,25 @@ struct DiagArgs {
   int kb;
 };
 
-// Tables of up to 4 entries: the entries are read once per thread with
-// uniform (scalar) loads and chosen per element by selects in registers.  An
-// index into the argument block that varies per lane compiles to a vector
-// memory load per element, which queues behind the stream's own loads (a
-// diagonal on the two lowest bits measured 1.07 TB/s that way on one box).
+// Memory bounds a diagonal: one element per thread, and the table is read from
+// LDS, where each workgroup copies it (indexing the argument block per lane would
+// issue a memory load per element, which waits behind the stream's own loads).
+// 2^28 elements take 1.28 ms, 6.7 TB/s; tables of 2 and 4 entries took 1.32 ms with
+// their entries held in registers and chosen by selects.
 __global__ void __launch_bounds__(kGateThreads) diag_bits_kernel(c128 *__restrict__ psi, DiagArgs args, uint64_t n) {
-  constexpr int U = 4;
-  const c128 t0 = args.d[0], t1 = args.d[1], t2 = args.d[2], t3 = args.d[3];
-  double2_t *p2 = reinterpret_cast<double2_t *>(psi);
-  const uint64_t stride = (uint64_t)gridDim.x * kGateThreads;
-  for (uint64_t e0 = (uint64_t)blockIdx.x * kGateThreads + threadIdx.x; e0 < n; e0 += stride * U) {
-    double2_t v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t e = e0 + u * stride;
-      v[u] = e < n ? __builtin_nontemporal_load(p2 + e) : double2_t{0.0, 0.0};
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t e = e0 + u * stride;
-      if (e >= n) continue;
-      uint32_t c = 0;
-      for (int j = 0; j < args.kb; ++j) c = (c << 1) | (uint32_t)((e >> args.bitpos[j]) & 1ull);
-      const c128 lo = (c & 1) ? t1 : t0, hi = (c & 1) ? t3 : t2;
-      const c128 r = cmul(c128{v[u].x, v[u].y}, (c & 2) ? hi : lo);
-      __builtin_nontemporal_store(double2_t{r.re, r.im}, p2 + e);
-    }
-  }
-}
-
-// As diag_bits_kernel, for tables of more than 4 entries: the table is copied
-// into LDS once per workgroup and read from there per element (indexing the
-// argument block per lane would issue a memory load per element, which waits
-// behind the stream's own loads).  Same arithmetic as diag_bits_kernel.
-__global__ void __launch_bounds__(kGateThreads) diag_bits_lds_kernel(c128 *__restrict__ psi, DiagArgs args,
-                                                                     uint64_t n) {
-  constexpr int U = 4;
   __shared__ double2_t tab[kMaxDiag];
   const int K = 1 << args.kb;
   for (int i = threadIdx.x; i < K; i += kGateThreads) tab[i] = double2_t{args.d[i].re, args.d[i].im};
   __syncthreads();
   double2_t *p2 = reinterpret_cast<double2_t *>(psi);
   const uint64_t stride = (uint64_t)gridDim.x * kGateThreads;
-  for (uint64_t e0 = (uint64_t)blockIdx.x * kGateThreads + threadIdx.x; e0 < n; e0 += stride * U) {
-    double2_t v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t e = e0 + u * stride;
-      v[u] = e < n ? __builtin_nontemporal_load(p2 + e) : double2_t{0.0, 0.0};
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t e = e0 + u * stride;
-      if (e >= n) continue;
-      uint32_t c = 0;
-      for (int j = 0; j < args.kb; ++j) c = (c << 1) | (uint32_t)((e >> args.bitpos[j]) & 1ull);
-      const double2_t dc = tab[c];
-      const c128 r = cmul(c128{v[u].x, v[u].y}, c128{dc.x, dc.y});
-      __builtin_nontemporal_store(double2_t{r.re, r.im}, p2 + e);
-    }
+  for (uint64_t e = (uint64_t)blockIdx.x * kGateThreads + threadIdx.x; e < n; e += stride) {
+    const double2_t v = __builtin_nontemporal_load(p2 + e);
+    uint32_t c = 0;
+    for (int j = 0; j < args.kb; ++j) c = (c << 1) | (uint32_t)((e >> args.bitpos[j]) & 1ull);
+    const double2_t dc = tab[c];
+    const c128 r = cmul(c128{v.x, v.y}, c128{dc.x, dc.y});
+    __builtin_nontemporal_store(double2_t{r.re, r.im}, p2 + e);
   }
 }
 
@@ -594,10 +553,7 @@ qtnh_status launch_diag(qtnh_ctx_t ctx, c128 *state, int rank, const uint64_t *d
     // contiguous stretch of the state (81% of HBM peak at 2^28 and 2^30
     // elements, against 68-76% with four elements per thread 2^26+ apart).
     unsigned blocks = grid_for(n, kGateThreads, kMaxStreamBlocks);
-    if (K > 4)
-      hipLaunchKernelGGL(diag_bits_lds_kernel, dim3(blocks), dim3(kGateThreads), 0, ctx->stream, state, args, n);
-    else
-      hipLaunchKernelGGL(diag_bits_kernel, dim3(blocks), dim3(kGateThreads), 0, ctx->stream, state, args, n);
+    hipLaunchKernelGGL(diag_bits_kernel, dim3(blocks), dim3(kGateThreads), 0, ctx->stream, state, args, n);
     return check_hip(ctx, hipGetLastError(), "diag launch");
   }
   DiagGenArgs args;
