@@ -319,7 +319,7 @@ qtnh_status qtnh_ctx_create(int device, void *stream, qtnh_ctx_t *out) {
   if (st == QTNH_OK) st = check_hip(ctx, hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking), "side stream");
   if (st == QTNH_OK) st = check_hip(ctx, hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming), "event");
   if (st == QTNH_OK) st = check_hip(ctx, hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming), "event");
-  if (st == QTNH_OK) st = check_hip(ctx, hipHostMalloc((void **)&ctx->host_scalar, 64), "hipHostMalloc");
+  if (st == QTNH_OK) st = check_hip(ctx, hipHostMalloc((void **)&ctx->host_scalar, kHostScalars * sizeof(double)), "hipHostMalloc");
   if (st == QTNH_OK) st = check_hip(ctx, hipMalloc((void **)&ctx->dev_scalar, 2048 * sizeof(double)), "hipMalloc scalar");
   // Device address of the no-allocation entry point's scratch array (once per device).
   if (st == QTNH_OK) st = noalloc_setup(ctx);

@@ -884,70 +884,101 @@ __global__ void __launch_bounds__(256, MINW)
 // ---- <Z_q> for a list of qubits --------------------------------------------
 // Chunks of 2^kChunkBits consecutive amplitudes.  Per chunk: the total
 // probability and, for each of the chunk's own index bits, the probability
-// with that bit set.  Bits above the chunk are constant inside it.
+// with that bit set (slot s of chunk c at part[s nchunks + c]).  Bits above the
+// chunk are constant inside it.
 constexpr int kChunkBits = 12;
 constexpr int kZThreads = 256;
 constexpr int kZSlots = 1 + kChunkBits;
 
-__global__ void __launch_bounds__(kZThreads) zchunk_kernel(const double2_t *__restrict__ psi, uint64_t n, int cb,
+// Memory bounds it: a thread's 16 amplitudes are requested together, and of the
+// 13 sums over the threads those of the low eight bits are taken from the same
+// totals as the chunk's own, a quarter of them by each wave, with one barrier a
+// chunk.  2^20 amplitudes: 4.8 us, and 13.7 with a tree of eight barriers for every
+// sum; 2^28: 720 us and 890.  FULL: the chunk has 2^kChunkBits amplitudes.  NT:
+// non-temporal loads, for states beyond the 256 MB cache (2^26 amplitudes: 203 us a
+// call, 219 without; 2^24: 67 us a call, 62.6 without).
+template <bool FULL, bool NT>
+__global__ void __launch_bounds__(kZThreads) zchunk_kernel(const double2_t *__restrict__ psi, int cb,
                                                            double *__restrict__ part, uint64_t nchunks) {
-  __shared__ double red[kZThreads];
-  for (uint64_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    // Thread t owns chunk elements t + kZThreads j: bits 0..7 of the element are t's bits.
-    double tot = 0.0, hib[kChunkBits];
+  constexpr int kEach = (1 << kChunkBits) / kZThreads, kHigh = kChunkBits - 8;
+  __shared__ double red[1 + kHigh][kZThreads];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t ch = blockIdx.x;
+  // Thread t owns chunk elements t + kZThreads j: bits 0..7 of the element are t's bits.
+  double2_t v[kEach];
 #pragma unroll
-    for (int b = 0; b < kChunkBits; ++b) hib[b] = 0.0;
-    const uint64_t e0 = ch << cb;
-    const int csize = 1 << cb;
-    for (int l = threadIdx.x; l < csize; l += kZThreads) {
-      const uint64_t e = e0 + l;
-      double p = 0.0;
-      if (e < n) {
-        const double2_t v = psi[e];
-        p = v.x * v.x;
-        p = p + v.y * v.y;
-      }
-      tot = tot + p;
+  for (int j = 0; j < kEach; ++j) {
+    const int l = tid + kZThreads * j;
+    const double2_t *p = psi + (ch << cb) + l;
+    v[j] = double2_t{0.0, 0.0};
+    if (FULL || l < 1 << cb) v[j] = NT ? __builtin_nontemporal_load(p) : *p;
+  }
+  double tot = 0.0, hib[kHigh] = {};
 #pragma unroll
-      for (int b = 8; b < kChunkBits; ++b)
-        if ((l >> b) & 1) hib[b] = hib[b] + p;
+  for (int j = 0; j < kEach; ++j) {
+    double p = v[j].x * v[j].x;
+    p = p + v[j].y * v[j].y;
+    tot = tot + p;
+#pragma unroll
+    for (int b = 0; b < kHigh; ++b)
+      if (j >> b & 1) hib[b] = hib[b] + p;
+  }
+  red[0][tid] = tot;
+#pragma unroll
+  for (int b = 0; b < kHigh; ++b) red[1 + b][tid] = hib[b];
+  __syncthreads();
+  // slot 0: total; slot 1 + b: probability with bit b set.
+#pragma unroll
+  for (int i = 0; i < (kZSlots + 3) / 4; ++i) {
+    const int s = wave + 4 * i, b = s - 1;
+    if (s >= kZSlots) break;
+    const double *r = red[s > 8 ? s - 8 : 0];
+    double x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double y = r[64 * k + lane];
+      x[k] = s == 0 || s > 8 || (64 * k + lane) >> b & 1 ? y : 0.0;
     }
-    // slot 0: total; slot 1 + b: probability with bit b set.
+    double sum = (x[0] + x[2]) + (x[1] + x[3]);
 #pragma unroll
-    for (int s = 0; s < kZSlots; ++s) {
-      double v;
-      if (s == 0)
-        v = tot;
-      else if (s - 1 < 8)
-        v = ((threadIdx.x >> (s - 1)) & 1) ? tot : 0.0;
-      else
-        v = hib[s - 1];
-      red[threadIdx.x] = v;
-      __syncthreads();
-      for (int w = kZThreads / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
-        __syncthreads();
-      }
-      if (threadIdx.x == 0) part[ch * kZSlots + s] = red[0];
-      __syncthreads();
-    }
+    for (int w = 32; w > 0; w >>= 1) sum = sum + __shfl_down(sum, w, 64);
+    if (lane == 0) part[(uint64_t)s * nchunks + ch] = sum;
   }
 }
 
-// One workgroup per requested qubit: <Z_b> = sum over chunks of (total - 2 set_b).
+struct ZQubits {
+  uint8_t bit[kHostScalars];
+};
+
+// One workgroup per requested qubit: <Z_b> = sum over chunks of (total - 2 set_b),
+// eight of a thread's chunks read at a time (2^16 chunks: 41 us, 138 one at a time
+// from a table of 13 slots a chunk).
 __global__ void __launch_bounds__(kZThreads) zfinal_kernel(const double *__restrict__ part, uint64_t nchunks, int cb,
-                                                           const int *__restrict__ bits, double *__restrict__ out) {
+                                                           ZQubits qubits, double *__restrict__ out) {
   __shared__ double red[kZThreads];
-  const int b = bits[blockIdx.x];
+  const int b = qubits.bit[blockIdx.x];
+  const bool inside = b < cb;
+  const double *set = part + (inside ? (uint64_t)(1 + b) * nchunks : 0);
   double s = 0.0;
-  for (uint64_t ch = threadIdx.x; ch < nchunks; ch += kZThreads) {
-    const double tot = part[ch * kZSlots];
-    double v;
-    if (b < cb)
-      v = tot - 2.0 * part[ch * kZSlots + 1 + b];
-    else
-      v = (((ch << cb) >> b) & 1) ? -tot : tot;
-    s = s + v;
+  for (uint64_t c0 = threadIdx.x; c0 < nchunks; c0 += 8 * kZThreads) {
+    double tot[8], on[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint64_t ch = c0 + j * kZThreads < nchunks ? c0 + j * kZThreads : c0;
+      tot[j] = part[ch];
+      on[j] = set[ch];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint64_t ch = c0 + j * kZThreads;
+      if (ch >= nchunks) break;
+      double v;
+      if (inside)
+        v = tot[j] - 2.0 * on[j];
+      else
+        v = (((ch << cb) >> b) & 1) ? -tot[j] : tot[j];
+      s = s + v;
+    }
   }
   red[threadIdx.x] = s;
   __syncthreads();
@@ -2080,36 +2111,40 @@ qtnh_status qtnh_expect_z_c128(qtnh_ctx_t ctx, const void *state, int n_qubits, 
                                double *out) {
   qtnh_status st = enter_ctx(ctx);
   if (st) return st;
-  if (!state || !out || n_qubits < 1 || n_qubits > 62 || nq < 1 || nq > 1024 || !qubits)
+  if (!state || !out || n_qubits < 1 || n_qubits > 62 || nq < 1 || nq > kHostScalars || !qubits)
     return set_error(ctx, QTNH_EINVAL, "expect_z: bad arguments");
   for (int j = 0; j < nq; ++j)
     if (qubits[j] >= n_qubits) return set_error(ctx, QTNH_EINVAL, "expect_z: qubit %d out of range", qubits[j]);
   const uint64_t n = 1ull << n_qubits;
   const int cb = std::min(n_qubits, kChunkBits);
   const uint64_t nchunks = n >> cb;
-  const uint64_t part_bytes = ((nchunks * kZSlots * sizeof(double)) + 255) & ~255ull;
-  st = grow_buffer(ctx, &ctx->red, &ctx->red_bytes, part_bytes + (uint64_t)nq * (sizeof(int) + sizeof(double)) + 512);
+  st = grow_buffer(ctx, &ctx->red, &ctx->red_bytes, nchunks * kZSlots * sizeof(double));
   if (st) return st;
   double *part = (double *)ctx->red;
-  int *bits = (int *)((char *)ctx->red + part_bytes);
-  double *dout = (double *)((char *)ctx->red + part_bytes + (((uint64_t)nq * sizeof(int) + 255) & ~255ull));
-  std::vector<int> hb(nq);
-  for (int j = 0; j < nq; ++j) hb[j] = n_qubits - 1 - qubits[j];
-  st = check_hip(ctx, hipMemcpyAsync(bits, hb.data(), nq * sizeof(int), hipMemcpyHostToDevice, ctx->stream),
-                 "expect_z upload");
-  if (st) return st;
-  const unsigned blocks = (unsigned)std::min<uint64_t>(nchunks, (uint64_t)ctx->num_cus * 8);
-  hipLaunchKernelGGL(zchunk_kernel, dim3(blocks), dim3(kZThreads), 0, ctx->stream, (const double2_t *)state, n, cb,
-                     part, nchunks);
+  ZQubits bits;
+  for (int j = 0; j < nq; ++j) bits.bit[j] = (uint8_t)(n_qubits - 1 - qubits[j]);
+  const unsigned blocks = (unsigned)nchunks;
+  const auto *psi = (const double2_t *)state;
+  if (n_qubits > 24)
+    hipLaunchKernelGGL((zchunk_kernel<true, true>), dim3(blocks), dim3(kZThreads), 0, ctx->stream, psi, cb, part,
+                       nchunks);
+  else if (cb == kChunkBits)
+    hipLaunchKernelGGL((zchunk_kernel<true, false>), dim3(blocks), dim3(kZThreads), 0, ctx->stream, psi, cb, part,
+                       nchunks);
+  else
+    hipLaunchKernelGGL((zchunk_kernel<false, false>), dim3(blocks), dim3(kZThreads), 0, ctx->stream, psi, cb, part,
+                       nchunks);
   st = check_hip(ctx, hipGetLastError(), "expect_z launch");
   if (st) return st;
-  hipLaunchKernelGGL(zfinal_kernel, dim3(nq), dim3(kZThreads), 0, ctx->stream, part, nchunks, cb, bits, dout);
+  // The results go to pinned host memory from the kernel.
+  hipLaunchKernelGGL(zfinal_kernel, dim3(nq), dim3(kZThreads), 0, ctx->stream, part, nchunks, cb, bits,
+                     ctx->host_scalar);
   st = check_hip(ctx, hipGetLastError(), "expect_z final launch");
   if (st) return st;
-  st = check_hip(ctx, hipMemcpyAsync(out, dout, nq * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-                 "expect_z copy");
+  st = check_hip(ctx, hipStreamSynchronize(ctx->stream), "expect_z sync");
   if (st) return st;
-  return check_hip(ctx, hipStreamSynchronize(ctx->stream), "expect_z sync");
+  memcpy(out, ctx->host_scalar, nq * sizeof(double));
+  return QTNH_OK;
 }
 
 }  // extern "C"

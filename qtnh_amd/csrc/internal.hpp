@@ -18,7 +18,7 @@ struct qtnh_ctx_s {
   // Growable device workspace for permute-to-matrix temporaries.
   void *ws = nullptr;
   uint64_t ws_bytes = 0;
-  // Small pinned host buffer + device buffer for reduction results.
+  // Small pinned host buffer (kHostScalars) + device buffer for reduction results.
   double *host_scalar = nullptr;
   double *dev_scalar = nullptr;
   // Growable device buffer for launch descriptors (circuit runs, batches).
@@ -51,6 +51,7 @@ struct c128 {
 };
 
 constexpr int kMaxRank = QTNH_MAX_RANK;
+constexpr int kHostScalars = 1024;
 
 qtnh_status set_error(qtnh_ctx_t ctx, qtnh_status st, const char *fmt, ...);
 qtnh_status check_hip(qtnh_ctx_t ctx, hipError_t e, const char *what);
