@@ -10,6 +10,7 @@ Placement arguments follow reference src/tensor/contract.cpp: repl1/repl2
 give each open axis its position in the result (X for wired axes).
 """
 import ctypes
+from array import array
 
 import numpy as np
 import torch
@@ -43,18 +44,30 @@ def trim(device=None, stream=None):
     check(lib().qtnh_ctx_trim(ctx), ctx)
 
 
+# Lists of dims, axes and wires as C arrays: a call of the small contractions
+# converts several, and one through numpy takes 3.6 us, through array 0.9 us.
+# What array does not take (floats, nested lists, values out of range) goes
+# through numpy.
 def _u64(v):
-    a = np.ascontiguousarray(np.asarray(list(v), dtype=np.uint64))
-    if a.size == 0:
-        a = np.zeros(1, dtype=np.uint64)
-    return a, a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64))
+    v = list(v) or [0]
+    try:
+        a = array("Q", v)
+    except (TypeError, OverflowError):
+        a = np.ascontiguousarray(np.asarray(v, dtype=np.uint64))
+        return a, a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64))
+    return a, (ctypes.c_uint64 * len(a)).from_buffer(a)
 
 
 def _u16(v):
-    a = np.ascontiguousarray(np.asarray(list(v), dtype=np.uint16).reshape(-1))
-    if a.size == 0:
-        a = np.zeros(1, dtype=np.uint16)
-    return a, a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16))
+    v = list(v) or [0]
+    try:
+        a = array("H", v)
+    except (TypeError, OverflowError):
+        a = np.ascontiguousarray(np.asarray(v, dtype=np.uint16).reshape(-1))
+        if a.size == 0:
+            a = np.zeros(1, dtype=np.uint16)
+        return a, a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16))
+    return a, (ctypes.c_uint16 * len(a)).from_buffer(a)
 
 
 def _c128_host(v):
@@ -168,12 +181,10 @@ def diag_apply_(x, dims, axes, dvals):
 
 def default_repls(r1, ndis1, r2, ndis2, wires):
     w, wp = _u16([v for pair in wires for v in pair])
-    o1 = np.zeros(max(r1, 1), dtype=np.uint16)
-    o2 = np.zeros(max(r2, 1), dtype=np.uint16)
-    check(lib().qtnh_default_repls(r1, ndis1, r2, ndis2, len(wires), wp,
-                                   o1.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16)),
-                                   o2.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16))))
-    return [int(v) for v in o1[:r1]], [int(v) for v in o2[:r2]]
+    o1 = (ctypes.c_uint16 * max(r1, 1))()
+    o2 = (ctypes.c_uint16 * max(r2, 1))()
+    check(lib().qtnh_default_repls(r1, ndis1, r2, ndis2, len(wires), wp, o1, o2))
+    return o1[:r1], o2[:r2]
 
 
 def symm_repls(r1, nd2, nl2, n_dis_in, wires):
@@ -196,11 +207,14 @@ def contract_dims(dA, dB, wires, repl1, repl2):
     w, wp = _u16([v for pair in wires for v in pair])
     r1, r1p = _u16(repl1)
     r2, r2p = _u16(repl2)
+    return _contract_dims(len(dA), ap, len(dB), bp, len(wires), wp, r1p, r2p)
+
+
+def _contract_dims(*args):
     rc = ctypes.c_int(0)
-    out = np.zeros(64, dtype=np.uint64)
-    check(lib().qtnh_contract_dims(len(dA), ap, len(dB), bp, len(wires), wp, r1p, r2p, ctypes.byref(rc),
-                                   out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64))))
-    return [int(v) for v in out[:rc.value]]
+    out = (ctypes.c_uint64 * 64)()
+    check(lib().qtnh_contract_dims(*args, ctypes.byref(rc), out))
+    return out[:rc.value]
 
 
 def contract(A, dA, B, dB, wires, repl1=None, repl2=None, precision=PREC_FP64, out=None):
@@ -210,7 +224,13 @@ def contract(A, dA, B, dB, wires, repl1=None, repl2=None, precision=PREC_FP64, o
     _check_len(B, dB)
     if repl1 is None or repl2 is None:
         repl1, repl2 = default_repls(len(dA), 0, len(dB), 0, wires)
-    dC = contract_dims(dA, dB, wires, repl1, repl2)
+    a, ap = _u64(dA)
+    b, bp = _u64(dB)
+    w, wp = _u16([v for pair in wires for v in pair])
+    r1, r1p = _u16(repl1)
+    r2, r2p = _u16(repl2)
+    shape = (len(dA), ap, len(dB), bp, len(wires), wp, r1p, r2p)
+    dC = _contract_dims(*shape)
     if B.device != A.device:
         raise ValueError("A is on %s, B on %s" % (A.device, B.device))
     if out is None:
@@ -218,14 +238,9 @@ def contract(A, dA, B, dB, wires, repl1=None, repl2=None, precision=PREC_FP64, o
     else:
         _check_out(out, A, dC)
     ctx = context(A.device.index)
-    a, ap = _u64(dA)
-    b, bp = _u64(dB)
-    w, wp = _u16([v for pair in wires for v in pair])
-    r1, r1p = _u16(repl1)
-    r2, r2p = _u16(repl2)
     err = ctypes.c_double(0.0)
-    check(lib().qtnh_contract_c128(ctx, _ptr(A), len(dA), ap, _ptr(B), len(dB), bp, len(wires), wp, r1p, r2p,
-                                   _ptr(out), precision, ctypes.byref(err)), ctx)
+    check(lib().qtnh_contract_c128(ctx, _ptr(A), *shape[:2], _ptr(B), *shape[2:], _ptr(out), precision,
+                                   ctypes.byref(err)), ctx)
     return out, dC, err.value
 
 
@@ -508,9 +523,9 @@ class Network:
 
     def result_dims(self):
         r = ctypes.c_int(0)
-        d = np.zeros(64, dtype=np.uint64)
-        check(lib().qtnh_net_result_dims(self._h, ctypes.byref(r), d.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64))))
-        return [int(v) for v in d[:r.value]]
+        d = (ctypes.c_uint64 * 64)()
+        check(lib().qtnh_net_result_dims(self._h, ctypes.byref(r), d))
+        return d[:r.value]
 
     def run(self, device=None):
         n = _size(self.result_dims())
@@ -555,25 +570,29 @@ class NetworkBatch:
         return {"grouped_direct": v[0].value, "grouped_gemm": v[1].value, "single": v[2].value}
 
     def run(self):
-        outs = [np.zeros(max(_size(n.result_dims()), 1), dtype=np.complex128) for n in self.nets]
-        ps = (ctypes.POINTER(ctypes.c_double) * len(outs))(*[o.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-                                                              for o in outs])
+        sizes, outs, ps = _result_buffers(self.nets)
         check(lib().qtnh_net_batch_run(self._ctx, self._h, ps), self._ctx)
-        return [o[:_size(n.result_dims())] for o, n in zip(outs, self.nets)]
+        return [o[:n] for o, n in zip(outs, sizes)]
+
+
+def _result_buffers(nets):
+    """The networks' result sizes, a host buffer for each and the table of their addresses."""
+    sizes = [_size(n.result_dims()) for n in nets]
+    outs = [np.zeros(max(n, 1), dtype=np.complex128) for n in sizes]
+    ps = (ctypes.c_void_p * len(outs))(*[o.__array_interface__["data"][0] for o in outs])
+    return sizes, outs, ctypes.cast(ps, ctypes.POINTER(ctypes.POINTER(ctypes.c_double)))
 
 
 def run_networks(nets, budget_bytes=1 << 40, device=None):
     """Contract planned networks as one batch; returns (results, waves)."""
-    outs = [np.zeros(max(_size(n.result_dims()), 1), dtype=np.complex128) for n in nets]
+    sizes, outs, ps = _result_buffers(nets)
     if not nets:
         return outs, 0
     ctx = context(device)
     hs = (ctypes.c_void_p * len(nets))(*[n.handle.value for n in nets])
-    ps = (ctypes.POINTER(ctypes.c_double) * len(nets))(*[o.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-                                                          for o in outs])
     waves = ctypes.c_int(0)
     check(lib().qtnh_net_run_batch(ctx, len(nets), hs, ps, budget_bytes, ctypes.byref(waves)), ctx)
-    return [o[:_size(n.result_dims())] for o, n in zip(outs, nets)], waves.value
+    return [o[:n] for o, n in zip(outs, sizes)], waves.value
 
 
 def serve(queries, budget_bytes, policy=_lib.SERVE_BATCHED, device=None):
