@@ -379,69 +379,122 @@ __device__ __forceinline__ OzTile oz_tile(const OzArgs &a, int BM, int BN) {
   return r;
 }
 
-// Recombines one output of part t from its S diagonal sums (row scale
-// 2^er fr, column scale 2^ec fc) and stores it.
-template <int S>
-__device__ __forceinline__ void oz_store(const OzArgs &a, int t, uint64_t gm, uint64_t gn, const int *accd, double fr,
-                                         int er, double fc, int ec) {
+// One output from its S diagonal sums, up to the power of two of its scales.
+// The weights are powers of two, so each fma rounds as the addition of the
+// scaled term does.
+template <int S, typename Acc>
+__device__ __forceinline__ double oz_combine(const Acc &accd, double scale) {
   double sum = 0.0;
 #pragma unroll
-  for (int d = S - 1; d >= 0; --d) sum += ldexp((double)accd[d], 8 * (2 * S - 2 - d));
-  const double v = ldexp(sum * (fr * fc), er + ec);
-  const uint64_t MN = a.M * a.N, e = gm * a.N + gn;
-  if (t == 2 && a.combine) {
-    double t3 = v;
-    if (a.accumulate) t3 += a.T[2 * MN + e];  // T3 exists when the depth takes several chunks
-    const double t1 = a.T[e], t2 = a.T[MN + e];
-    a.C[e] = double2_t{t1 - t2, (t3 - t1) - t2};
-  } else {
-    double *dst = a.T + (uint64_t)t * MN + e;
-    *dst = a.accumulate ? *dst + v : v;
-  }
+  for (int d = S - 1; d >= 0; --d) sum = __builtin_fma((double)accd(d), ldexp(1.0, 8 * (2 * S - 2 - d)), sum);
+  return sum * scale;
 }
 
-// 16x16 i32 result layout: lane l holds column l % 16 of rows 4 (l / 16) + v.
-// The scales of the lane's 4 FA rows and FB columns are read once (the
-// stores in between would otherwise make the compiler reload them per
-// output: 4 scattered loads per output).
-template <int S, int FA, int FB>
-__device__ __forceinline__ void oz_epilogue(const OzArgs &a, const OzTile &tl, int wm, int wn, int lane,
-                                            const int4_t (&acc)[S][FA][FB]) {
+// Recombines and stores a wave's outputs (row scale 2^er fr, column scale
+// 2^ec fc).  16x16 i32 result layout: lane l holds column l % 16 of rows
+// 4 (l / 16) + v.  One workgroup has the compute unit, so nothing overlaps this
+// but its own two waves per SIMD: as few instructions per output as it takes
+// (14 for S = 5 and the stores, where a scaling per term, bounds checks and
+// addresses per output made it about 90), and the loads of four rows of FB columns
+// together: the matrix cores' share of T3 with the final combination, 4096^3, went
+// from 66% to 72%.  WHOLE: the tile is within M x N.
+template <int S, int FA, int FB, bool WHOLE>
+__device__ __forceinline__ void oz_finish(const OzArgs &a, const OzTile &tl, int wm, int wn, int lane,
+                                          const int4_t (&acc)[S][FA][FB]) {
   const int t = tl.part;
-  double fr[FA][4], fc[FB];
-  int er[FA][4], ec[FB];
-#pragma unroll
-  for (int i = 0; i < FA; ++i)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const uint64_t gm = tl.m0 + wm + 16 * i + 4 * (lane >> 4) + v;
-      const uint64_t r = (uint64_t)t * a.M + (gm < a.M ? gm : 0);
-      fr[i][v] = a.fa[r];
-      er[i][v] = a.ea[r];
-    }
+  const uint64_t MN = a.M * a.N, gn0 = tl.n0 + wn + (lane & 15);
+  double fc[FB];
+  int ec[FB];
+  bool col[FB];
 #pragma unroll
   for (int j = 0; j < FB; ++j) {
-    const uint64_t gn = tl.n0 + wn + 16 * j + (lane & 15);
-    const uint64_t c = (uint64_t)t * a.N + (gn < a.N ? gn : 0);
+    col[j] = WHOLE || gn0 + 16 * j < a.N;
+    const uint64_t c = (uint64_t)t * a.N + (col[j] ? gn0 + 16 * j : 0);
     fc[j] = a.fb[c];
     ec[j] = a.eb[c];
   }
 #pragma unroll
-  for (int i = 0; i < FA; ++i)
+  for (int i = 0; i < FA; ++i) {
+    const uint64_t gm0 = tl.m0 + wm + 16 * i + 4 * (lane >> 4);
+    double fr[4];
+    int er[4];
+    bool row[4];
 #pragma unroll
-    for (int j = 0; j < FB; ++j)
+    for (int v = 0; v < 4; ++v) {
+      row[v] = WHOLE || gm0 + v < a.M;
+      const uint64_t r = (uint64_t)t * a.M + (row[v] ? gm0 + v : 0);
+      fr[v] = a.fa[r];
+      er[v] = a.ea[r];
+    }
+    double out[4][FB];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const uint64_t gm = tl.m0 + wm + 16 * i + 4 * (lane >> 4) + v;
-        const uint64_t gn = tl.n0 + wn + 16 * j + (lane & 15);
-        if (gm < a.M && gn < a.N) {
-          int accd[S];
+    for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int d = 0; d < S; ++d) accd[d] = acc[d][i][j][v];
-          oz_store<S>(a, t, gm, gn, accd, fr[i][v], er[i][v], fc[j], ec[j]);
-        }
-      }
+      for (int j = 0; j < FB; ++j)
+        out[v][j] = ldexp(oz_combine<S>([&](int d) { return acc[d][i][j][v]; }, fr[v] * fc[j]), er[v] + ec[j]);
+    const uint64_t e0 = gm0 * a.N + gn0;
+    auto each = [&](auto &&f) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < FB; ++j)
+          if (WHOLE || (row[v] && col[j])) f(v, j, e0 + v * a.N + 16 * j);
+    };
+    const bool last = t == 2 && a.combine;
+    double *T = a.T + (uint64_t)t * MN;
+    if (a.accumulate) {  // the depth takes several chunks
+      double old[4][FB];
+      each([&](int v, int j, uint64_t e) { old[v][j] = T[e]; });
+      each([&](int v, int j, uint64_t) { out[v][j] = old[v][j] + out[v][j]; });
+    }
+    if (last) {
+      double t1[4][FB], t2[4][FB];
+      each([&](int v, int j, uint64_t e) {
+        t1[v][j] = a.T[e];
+        t2[v][j] = a.T[MN + e];
+      });
+      each([&](int v, int j, uint64_t e) {
+        a.C[e] = double2_t{t1[v][j] - t2[v][j], (out[v][j] - t1[v][j]) - t2[v][j]};
+      });
+    } else {
+      each([&](int v, int j, uint64_t e) { T[e] = out[v][j]; });
+    }
+  }
 }
+
+template <int S, int FA, int FB>
+__device__ __forceinline__ void oz_epilogue(const OzArgs &a, const OzTile &tl, int BM, int BN, int wm, int wn,
+                                            int lane, const int4_t (&acc)[S][FA][FB]) {
+  if (tl.m0 + BM <= a.M && tl.n0 + BN <= a.N)
+    oz_finish<S, FA, FB, true>(a, tl, wm, wn, lane, acc);
+  else
+    oz_finish<S, FA, FB, false>(a, tl, wm, wn, lane, acc);
+}
+
+// One operand's chunks of a wave: chunk wv + NW i of the S planes' ROWS / 16 row
+// groups, i ascending.
+template <int S, int ROWS, int NW>
+struct OzFeed {
+  static constexpr int G = ROWS / 16, N = (S * G + NW - 1) / NW;
+  const int8_t *src[N];
+  int last;  // planes past the last chunk's (0 or less: the wave has none)
+  // panel: the rows' first chunk; a plane and a row group further on.
+  __device__ __forceinline__ void set(const int8_t *panel, uint64_t plane, uint64_t group, int wv) {
+    const int8_t *first = panel + (NW >= G ? (wv / G) * plane + (wv % G) * group : wv * group);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      src[i] = first + (NW >= G ? i * (NW / G) * plane : (i * NW / G) * plane + (i * NW % G) * group);
+    last = S - (wv + NW * (N - 1)) / G;
+  }
+  __device__ __forceinline__ void issue(int4_t *lds, uint32_t off, int wv) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (S * G % NW == 0 || i + 1 < N || last > 0)
+        __builtin_amdgcn_global_load_lds((const void *)(src[i] + off),
+                                         (void __attribute__((address_space(3))) *)(lds + (wv + NW * i) * 64), 16, 0,
+                                         0);
+  }
+};
 
 template <int S, int WM, int WN, int WGM, int WGN, int MINW>
 __global__ void __launch_bounds__(64 * WGM * WGN, MINW) ozaki_gemm_kernel(OzArgs a) {
@@ -466,28 +519,22 @@ __global__ void __launch_bounds__(64 * WGM * WGN, MINW) ozaki_gemm_kernel(OzArgs
   // A chunk of the tiled planes is one wave instruction: lane i copies its
   // 16-byte slot i into LDS slot i.  The planes hold whole tiles of rows (the
   // rows past M or N are padding whose products land only in outputs that are
-  // not stored), so no row is clamped: a chunk's address is a wave-uniform base
-  // plus the lane's 16 i, and issuing a chunk costs no per-lane arithmetic.
+  // not stored), so no row is clamped.  The wave's chunks keep their places from
+  // one depth step to the next, 1 KiB on: their addresses stay in scalar
+  // registers and a step adds the lane's offset to them.  (Worked out anew each
+  // step, some 300 scalar instructions, they kept the matrix cores idle a third of
+  // the time: 65% busy, 76% so, T1 and T2 of 4096^3 1598 -> 1350 us.  At that
+  // load the clock falls to 1.6 to 1.9 GHz, so what is left of the issue time
+  // gives less than its share.)
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  const uint32_t off = 16 * lane;
-  // Row groups of 16 rows are lda / 64 chunks of 1 KiB apart; depth step kt is
-  // chunk kt of its row group.
+  OzFeed<S, BM, Z::NW> feedA;
+  OzFeed<S, BN, Z::NW> feedB;
+  feedA.set(As + (m0 >> 4) * (a.lda << 4), a.a_plane, a.lda << 4, wv);
+  feedB.set(Bs + (n0 >> 4) * (a.ldb << 4), a.b_plane, a.ldb << 4, wv);
   auto issue = [&](int st, uint64_t kt) {
-#pragma unroll
-    for (int i = 0; i < (Z::CA + Z::CB + Z::NW - 1) / Z::NW; ++i) {
-      const int c = wv + Z::NW * i;
-      if (c < Z::CA + Z::CB) {
-        const bool isA = c < Z::CA;
-        const int cc = isA ? c : c - Z::CA;
-        const int rows = isA ? BM : BN;
-        const int p = cc / (rows / 16), g = cc % (rows / 16);
-        const int8_t *base = isA ? As + p * a.a_plane + ((m0 >> 4) + g) * (a.lda << 4) + (kt << 10)
-                                 : Bs + p * a.b_plane + ((n0 >> 4) + g) * (a.ldb << 4) + (kt << 10);
-        int4_t *dst = isA ? &sA[st][(p * rows + g * 16) * 4] : &sB[st][(p * rows + g * 16) * 4];
-        __builtin_amdgcn_global_load_lds((const void *)(base + off), (void __attribute__((address_space(3))) *)dst, 16,
-                                         0, 0);
-      }
-    }
+    const uint32_t off = 16 * lane + ((uint32_t)kt << 10);
+    feedA.issue(sA[st], off, wv);
+    feedB.issue(sB[st], off, wv);
   };
 
   // The caller pads the depth to a multiple of BK with zeros.
@@ -527,7 +574,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, MINW) ozaki_gemm_kernel(OzArgs
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
-  oz_epilogue<S, Z::FA, Z::FB>(a, tl, wm, wn, lane, acc);
+  oz_epilogue<S, Z::FA, Z::FB>(a, tl, BM, BN, wm, wn, lane, acc);
 }
 
 // Register-staged variant for S >= 6 (128 x 64 tiles, 8 waves of 32 x 32):
@@ -621,7 +668,7 @@ __global__ void __launch_bounds__(512) ozaki_gemm_staged(OzArgs a) {
       }
     }
   }
-  oz_epilogue<S, 2, 2>(a, tl, wm, wn, lane, acc);
+  oz_epilogue<S, 2, 2>(a, tl, BM, BN, wm, wn, lane, acc);
 }
 
 // Tile shapes of ozaki_gemm_kernel (wave tile WM x WN, WGM x WGN waves, MINW

@@ -232,3 +232,16 @@ def test_split_b_by_rows_and_by_columns_bitwise(m, k, n):
     C = g1.reshape(m, n)
     assert np.all(C[:, 5] == 0)
     check_bound(A, B, C, A @ B, eta, k)
+
+
+@pytest.mark.parametrize("slices", [5, 6])
+@pytest.mark.parametrize("m,k,n", [(128, 8192, 128), (256, 8200, 128), (130, 8260, 129), (17, 16500, 200)])
+def test_split_depth_chunks_and_partial_tiles(slices, m, k, n):
+    """Whole and partial result tiles, one and several depth chunks (2^13 terms
+    each): normwise error <= 1e-10 as everywhere at five slices or more."""
+    A, B = rnd((m, k), 1), rnd((k, n), 2)
+    ops.tune_split(slices)
+    C = host(ops.contract(dev(A), [m, k], dev(B), [k, n], [(1, 0)], precision=SPLIT)[0]).reshape(m, n)
+    ops.tune_split(5)
+    ref = A @ B
+    assert np.linalg.norm(C - ref) <= 1e-10 * np.linalg.norm(ref)
