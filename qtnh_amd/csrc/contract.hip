@@ -728,6 +728,8 @@ ContractRoute contract_route(int rA, const uint64_t *dA, int rB, const uint64_t 
   return R;
 }
 
+constexpr uint64_t kPairMaxElems = 1ull << 22;
+
 qtnh_status launch_contract(qtnh_ctx_t ctx, const c128 *A, int rA, const uint64_t *dA, const c128 *B, int rB,
                             const uint64_t *dB, int nw, const uint16_t *wires, const uint16_t *r1, const uint16_t *r2,
                             c128 *C, int precision, double *err_out, void *ext_ws, uint64_t ext_ws_bytes) {
@@ -755,15 +757,24 @@ qtnh_status launch_contract(qtnh_ctx_t ctx, const c128 *A, int rA, const uint64_
   const c128 *Ap = L.idA ? A : (const c128 *)(ws + L.offA);
   const c128 *Bp = L.idB ? B : (const c128 *)(ws + L.offB);
   c128 *Cn = L.idC ? C : (c128 *)(ws + L.offC);
-  if (!L.idA) {
-    qtnh_status st = launch_permute(ctx, A, (c128 *)Ap, rA, dA, L.pA.data());
-    if (st) return st;
+  qtnh_status st = QTNH_OK;
+  PermDesc pa, pb;
+  // Both operands of a contraction over power-of-two dims go in one launch while
+  // neither is large: 2^19 elements each take 7 us so and 18 in two launches of
+  // the tuned kernel, a contraction with an operand of 2^22 elements 48 us and
+  // 54; with one of 2^24, which fills the chip by itself, 181 us and 178.
+  if (!L.idA && !L.idB && std::max(P.M, P.N) * P.K <= kPairMaxElems && plan_permute_tiles(rA, dA, L.pA.data(), &pa) &&
+      plan_permute_tiles(rB, dB, L.pB.data(), &pb)) {
+    pa.src = A;
+    pa.dst = (c128 *)Ap;
+    pb.src = B;
+    pb.dst = (c128 *)Bp;
+    st = launch_permute_pair(ctx, pa, pb);
+  } else {
+    if (!L.idA) st = launch_permute(ctx, A, (c128 *)Ap, rA, dA, L.pA.data());
+    if (!st && !L.idB) st = launch_permute(ctx, B, (c128 *)Bp, rB, dB, L.pB.data());
   }
-  if (!L.idB) {
-    qtnh_status st = launch_permute(ctx, B, (c128 *)Bp, rB, dB, L.pB.data());
-    if (st) return st;
-  }
-  qtnh_status st;
+  if (st) return st;
   if (L.splitk) {
     st = launch_zgemm_splitk(ctx, Ap, Bp, Cn, P.M, P.N, P.K, L.kchunks, (c128 *)(ws + L.offS));
     if (err_out) *err_out = 0.0;

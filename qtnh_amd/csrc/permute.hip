@@ -1204,10 +1204,9 @@ namespace {
 // bound; 16 KB a block lets ten of them share a compute unit).  36 permutes of
 // 2^12 to 2^20 elements, 142 MB in all: 47 us, and 154 us with every element
 // gathered by a source offset put together from its result index.
-__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd) {
+__device__ __forceinline__ void permute_tile(const PermDesc &D, uint32_t t) {
   __shared__ double2_t tile[1 << kPermTileBits];
-  const PermDesc &D = d[find_entry(d, nd, blockIdx.x)];
-  const uint32_t t = blockIdx.x - (uint32_t)D.first, tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x;
   uint32_t so = 0, to = 0;
 #pragma unroll
   for (int p = 0; p < kPermMaxBits - kPermTileBits; ++p) {
@@ -1250,6 +1249,19 @@ __global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__
     const bool b8 = e & 256;
     dst[ss ^ (b8 ? D.store_dst[8] : 0u)] = tile[sl ^ (b8 ? D.store_lds[8] : 0u)];
   }
+}
+
+__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd) {
+  const PermDesc &D = d[find_entry(d, nd, blockIdx.x)];
+  permute_tile(D, blockIdx.x - (uint32_t)D.first);
+}
+
+struct PermPair {
+  PermDesc d[2];
+};
+__global__ void __launch_bounds__(256) permute_pair_kernel(PermPair p) {
+  const int i = blockIdx.x >= p.d[1].first;
+  permute_tile(p.d[i], blockIdx.x - (uint32_t)p.d[i].first);
 }
 }  // namespace
 
@@ -1316,6 +1328,14 @@ qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, ui
   if (nd <= 0 || total == 0) return QTNH_OK;
   hipLaunchKernelGGL(permute_grouped_kernel, dim3((unsigned)total), dim3(256), 0, ctx->stream, d, nd);
   return check_hip(ctx, hipGetLastError(), "grouped permute launch");
+}
+
+qtnh_status launch_permute_pair(qtnh_ctx_t ctx, const PermDesc &a, const PermDesc &b) {
+  PermPair p = {{a, b}};
+  p.d[0].first = 0;
+  p.d[1].first = a.blocks;
+  hipLaunchKernelGGL(permute_pair_kernel, dim3(a.blocks + b.blocks), dim3(256), 0, ctx->stream, p);
+  return check_hip(ctx, hipGetLastError(), "permute pair launch");
 }
 
 }  // namespace qtnh_hip

@@ -541,3 +541,41 @@ def test_contract_gemm_every_tile_and_depth(m, n, k):
     assert np.isnan(got[-1]).all() and not np.isfinite(got[:, -1]).any()
     inner = np.linalg.norm(got[:-1, :-1] - ref[:-1, :-1])
     assert inner <= 1e-12 * max(np.linalg.norm(ref[:-1, :-1]), 1e-300)
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 14, 5), (12, 2, 8), (9, 10, 6), (8, 8, 9), (3, 17, 5), (3, 18, 5)])
+@pytest.mark.parametrize("form", ["bits", "wider"])
+def test_contract_permutes_both_operands_bitwise(m, n, k, form):
+    """A contraction whose operands both have to be permuted (operands below a
+    tile, at and above the size that goes in one launch, axes of one and more
+    bits) equals the one whose operands lie in order, bit for bit."""
+    rng = np.random.default_rng(m + 100 * n)
+    def split(bits):
+        dims = []
+        while bits:
+            b = 1 if form == "bits" else min(bits, int(rng.integers(1, 4)))
+            dims.append(1 << b)
+            bits -= b
+        return dims
+    dm, dn, dk = split(m), split(n), split(k)
+    A = rng.standard_normal(dm + dk) + 1j * rng.standard_normal(dm + dk)
+    B = rng.standard_normal(dk + dn) + 1j * rng.standard_normal(dk + dn)
+    a, b, c = len(dm), len(dn), len(dk)
+    want = host(ops.contract(dev(A.reshape(-1)), dm + dk, dev(B.reshape(-1)), dk + dn, [(a + i, i) for i in range(c)])[0])
+    # Open axes keep their order among themselves; the wired ones go anywhere, and
+    # the wires are taken in the order of B's.
+    def shuffled(no, wired):
+        labels = ["o%d" % i for i in range(no)] + wired
+        places = sorted(rng.choice(no + c, no, replace=False))
+        out, o, w = [], iter(labels[:no]), iter(wired)
+        for i in range(no + c):
+            out.append(next(o) if i in places else next(w))
+        return out
+    wired = ["k%d" % i for i in range(c)]
+    la, lb = shuffled(a, list(rng.permutation(wired))), shuffled(b, wired)
+    pa = [["o%d" % i for i in range(a)].index(v) if v[0] == "o" else a + int(v[1:]) for v in la]
+    pb = [c + int(v[1:]) if v[0] == "o" else int(v[1:]) for v in lb]
+    At, Bt = np.ascontiguousarray(A.transpose(pa)), np.ascontiguousarray(B.transpose(pb))
+    wires = [(la.index(w), lb.index(w)) for w in wired]
+    got = host(ops.contract(dev(At.reshape(-1)), At.shape, dev(Bt.reshape(-1)), Bt.shape, wires)[0])
+    assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
