@@ -98,8 +98,9 @@ __global__ void __launch_bounds__(kDirThreads) contract_direct_general(const c12
   }
 }
 
-// Power-of-two result dims: C index bit p comes from A bit abit[p] or B bit
-// bbit[p] (-1 when from the other side).  A block handles 256 consecutive
+// Power-of-two dims of tensors beyond 2^32 elements (smaller ones: launch_direct):
+// C index bit p comes from A bit abit[p] or B bit bbit[p] (-1 when from the other
+// side).  A block handles 256 consecutive
 // result elements per step; the low 8 bits are per-thread constants.
 struct OutBits {
   int8_t abit[64];
@@ -576,6 +577,21 @@ qtnh_status launch_contract_direct(qtnh_ctx_t ctx, const c128 *A, int rA, const 
         default: launch_rows_kb<4, 1>(cb.kbits, g, ctx->stream, A, B, C, ob, cb, nrows); break;
       }
       return check_hip(ctx, hipGetLastError(), "contract_direct_rows launch");
+    }
+    // Tensors of up to 2^32 elements: the tiled form, whose offsets have 32 bits.
+    if (std::max({LA.nbits, LB.nbits, LC.nbits}) <= kGMaxBits && cb.kbits <= kGMaxTerms) {
+      StepBits bits;
+      bits.ncb = LC.nbits;
+      bits.kbits = cb.kbits;
+      for (int p = 0; p < LC.nbits; ++p) {
+        bits.abit[p] = ob.abit[p];
+        bits.bbit[p] = ob.bbit[p];
+      }
+      for (int j = 0; j < cb.kbits; ++j) {
+        bits.ka[j] = (int8_t)__builtin_ctzll(cb.fa[j] ^ (j ? cb.fa[j - 1] : 0ull));
+        bits.kb[j] = (int8_t)__builtin_ctzll(cb.fb[j] ^ (j ? cb.fb[j - 1] : 0ull));
+      }
+      return launch_direct(ctx, bits, A, B, C);
     }
     const int lowbits = std::min(LC.nbits, 8);
     const uint64_t nhi = P.nC >> lowbits;

@@ -220,6 +220,16 @@ struct SkDesc {
   uint64_t N, K, kc, S, MN;
   uint64_t first, first2;
 };
+// A contraction over power-of-two dims by direct sums, as bit maps (at most 2^10 terms).
+constexpr int kGMaxBits = 32, kGMaxTerms = 12;
+struct StepBits {
+  int ncb, kbits;          // result bits, closed bits
+  int8_t abit[kGMaxBits];  // A bit feeding result bit p (-1: from B)
+  int8_t bbit[kGMaxBits];
+  int8_t ka[kGMaxTerms];   // A bit of closed bit j (j = 0: last wire in the sum order)
+  int8_t kb[kGMaxTerms];
+};
+qtnh_status launch_direct(qtnh_ctx_t ctx, const StepBits &bits, const c128 *A, const c128 *B, c128 *C);
 // A bit permutation (every dim a power of two) in tiles of 2^tile elements, one
 // per block.  All entries are offsets that are XORed together: bit i of a tile's
 // element moves the source and the LDS slot in load order, the result and the

@@ -40,30 +40,19 @@ using GlobalIn = const __attribute__((address_space(1))) double2_t *;
 using GlobalOut = __attribute__((address_space(1))) double2_t *;
 
 constexpr int kGThreads = 256;
-constexpr int kGMaxBits = 32;
-
-// A contraction over binary (dim 2) axes, as bit maps.
-struct StepBits {
-  int ncb, kbits;          // result bits, closed bits
-  int8_t abit[kGMaxBits];  // A bit feeding result bit p (-1: from B)
-  int8_t bbit[kGMaxBits];
-  int8_t ka[kGMaxBits];    // A bit of closed bit j (j = 0: last wire in the sum order)
-  int8_t kb[kGMaxBits];
-};
 
 // A direct contraction in a grouped launch.  All tables hold offsets that are
 // XORed together: result bits that number the threads move A or B, and C; the
 // register bits number the 2^ta x 2^tb results of a thread; counting the closed
 // tuple t up by one flips entry ctz(t + 1).
-constexpr int kGMaxTerms = 12;  // log2 of the terms (direct contractions have at most 2^10)
 enum : uint32_t { kGWide = 16 };
-// One wave per result from 2^6 terms and up to 2^8 results: 18 contractions of
-// 2^6 results with 2^7 to 2^9 terms took 74 us with a thread each, 9 us so; seven of 2^12
-// results with 2^7 terms 21 us with a thread each, 46 us with a wave.  Register
-// tiles of 4 and 16 results where enough threads remain: 22 contractions of 2^12
-// to 2^18 results took 70 us without, 27 us with (two more or fewer bits at either
-// line: no difference).
-constexpr int kGWideMinBits = 6, kGWideMaxResult = 8, kGTile4 = 14, kGTile16 = 18;
+// One wave per result from 2^6 terms and up to 2^10 results: 2^6 results of 2^10
+// terms take 11 us so and 95 with a thread each, 2^12 results of 2^7 terms in seven
+// contractions at once 46 us so and 21 with a thread each.  Register tiles of 4
+// and 16 results where enough threads remain: 22 contractions of 2^12 to 2^18
+// results took 70 us without, 27 us with (two more or fewer bits at either line: no
+// difference).
+constexpr int kGWideMinBits = 6, kGWideMaxResult = 10, kGTile4 = 14, kGTile16 = 18;
 struct GDesc {
   const double2_t *A;
   const double2_t *B;
@@ -149,14 +138,13 @@ __device__ __forceinline__ void direct_tile(const GDesc &D, uint32_t x, uint32_t
 // as many products.  Sums of few results and 64 terms or more (closing steps)
 // are a chain of dependent loads and additions for a thread: there each wave
 // takes one result, its lanes form the products of 64 terms at a time, and only
-// the additions follow one another.
-__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd) {
+// the additions follow one another.  Alone: 2^12 x 2^12 results of 2^4 terms
+// 100 us and 269 with a result per thread, 2^13 x 2^12 of 2^2 terms 87 and 194.
+__device__ __forceinline__ void direct_block(const GDesc &D, uint32_t block) {
   __shared__ double2_t prod[kGThreads];
-  const GDesc &D = descs[find_entry(descs, nd, blockIdx.x)];
   const uint32_t tid = threadIdx.x, kind = D.kind, nb = D.nb;
   const uint32_t wide = kind == kGWide;
   // Thread's number among the results: low part from the lane, the rest (hi) of the block.
-  const uint32_t block = blockIdx.x - (uint32_t)D.first;
   const uint32_t low = wide ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)) | (block << 2 & 255u) : tid;
   const uint32_t hi = wide ? block >> 6 : block;
   if (low >= (nb < 8 ? 1u << nb : 256u)) return;
@@ -229,6 +217,13 @@ __global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *
     default: direct_tile<0, 2>(D, x, y, z); break;
   }
 }
+
+__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd) {
+  const GDesc &D = descs[find_entry(descs, nd, blockIdx.x)];
+  direct_block(D, blockIdx.x - (uint32_t)D.first);
+}
+
+__global__ void __launch_bounds__(kGThreads) direct_kernel(GDesc D) { direct_block(D, blockIdx.x); }
 
 // Steps of a network's leading run of small direct contractions (operands and
 // result of at most 2^12 elements) run in its chain: one workgroup steps
@@ -1121,24 +1116,27 @@ GDesc plan_grouped(const StepBits &g) {
   }
   // Register bits: the highest result bits of A and of B, so that the lanes
   // keep the lowest, whose elements are consecutive.
-  std::vector<int> from_a, from_b;
-  for (int p = g.ncb - 1; p >= 0; --p) (g.abit[p] >= 0 ? from_a : from_b).push_back(p);
-  size_t ta = 0, tb = 0;
+  int from_a[2], from_b[2], na = 0, nb = 0, ta = 0, tb = 0;
+  for (int p = g.ncb - 1; p >= 0 && (na < 2 || nb < 2); --p) {
+    if (g.abit[p] >= 0) {
+      if (na < 2) from_a[na++] = p;
+    } else if (nb < 2) {
+      from_b[nb++] = p;
+    }
+  }
   d.kind = kGWide;
   if (g.kbits < kGWideMinBits || g.ncb > kGWideMaxResult) {
-    if (g.ncb >= kGTile4 && !from_a.empty() && !from_b.empty()) ta = tb = 1;
-    if (g.ncb >= kGTile16 && from_a.size() > 1 && from_b.size() > 1) ta = tb = 2;
-    if (g.ncb >= kGTile4 && from_a.empty()) tb = 2;
-    if (g.ncb >= kGTile4 && from_b.empty()) ta = 2;
+    if (g.ncb >= kGTile4) ta = nb ? (na ? 1 : 0) : 2, tb = na ? (nb ? 1 : 0) : 2;
+    if (g.ncb >= kGTile16 && na > 1 && nb > 1) ta = tb = 2;
     d.kind = (uint32_t)(ta | tb << 2);
   }
   uint64_t in_regs = 0;
-  for (size_t i = 0; i < ta; ++i) {
+  for (int i = 0; i < ta; ++i) {
     in_regs |= 1ull << from_a[i];
     d.reg_a[i] = 1u << g.abit[from_a[i]];
     d.reg_ca[i] = 1u << from_a[i];
   }
-  for (size_t i = 0; i < tb; ++i) {
+  for (int i = 0; i < tb; ++i) {
     in_regs |= 1ull << from_b[i];
     d.reg_b[i] = 1u << g.bbit[from_b[i]];
     d.reg_cb[i] = 1u << from_b[i];
@@ -1156,6 +1154,18 @@ GDesc plan_grouped(const StepBits &g) {
   return d;
 }
 
+}  // namespace
+
+qtnh_status launch_direct(qtnh_ctx_t ctx, const StepBits &bits, const c128 *A, const c128 *B, c128 *C) {
+  GDesc d = plan_grouped(bits);
+  d.A = (const double2_t *)A;
+  d.B = (const double2_t *)B;
+  d.C = (double2_t *)C;
+  hipLaunchKernelGGL(direct_kernel, dim3(d.blocks), dim3(kGThreads), 0, ctx->stream, d);
+  return check_hip(ctx, hipGetLastError(), "direct contraction launch");
+}
+
+namespace {
 // The network's direct steps: records of its chain, descriptors of the others.
 // The chain's intermediates get LDS offsets by first fit over their lifetimes; one that
 // does not fit, or that a step outside the chain reads, goes to its arena place.

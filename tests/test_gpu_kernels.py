@@ -579,3 +579,37 @@ def test_contract_permutes_both_operands_bitwise(m, n, k, form):
     wires = [(la.index(w), lb.index(w)) for w in wired]
     got = host(ops.contract(dev(At.reshape(-1)), At.shape, dev(Bt.reshape(-1)), Bt.shape, wires)[0])
     assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (0, 15, 3), (16, 0, 4), (14, 1, 2), (1, 13, 4), (9, 9, 4), (10, 9, 1), (2, 17, 0),  # register tiles
+    (5, 8, 3), (2, 10, 4), (12, 1, 1), (0, 0, 0), (1, 0, 3),                             # one result a thread
+    (3, 3, 10), (4, 4, 9), (0, 0, 10), (1, 7, 6), (5, 5, 8), (5, 6, 9), (6, 6, 5),        # long sums
+])
+@pytest.mark.parametrize("widest", [1, 3])
+def test_contract_direct_matches_oracle_bitwise(m, n, k, widest):
+    """Direct contractions over power-of-two dims, with shuffled axes, wires and
+    result placement, at the edges of the kernel's forms."""
+    rng = np.random.default_rng(1000 * m + 100 * n + k)
+    def split(bits):
+        dims = []
+        while bits:
+            b = min(bits, int(rng.integers(1, widest + 1)))
+            dims.append(1 << b)
+            bits -= b
+        return dims
+    dm, dn, dk = split(m), split(n), split(k)
+    a = [("m", i) for i in range(len(dm))] + [("k", i) for i in range(len(dk))]
+    b = [("n", i) for i in range(len(dn))] + [("k", i) for i in range(len(dk))]
+    rng.shuffle(a), rng.shuffle(b)
+    a, b = [(x, int(i)) for x, i in a], [(x, int(i)) for x, i in b]
+    size = {"m": dm, "n": dn, "k": dk}
+    da, db = [size[x][i] for x, i in a], [size[x][i] for x, i in b]
+    wires = [(a.index(("k", i)), b.index(("k", i))) for i in rng.permutation(len(dk))]
+    place = iter(int(v) for v in rng.permutation(len(dm) + len(dn)))
+    r1 = [X if x == "k" else next(place) for x, _ in a]
+    r2 = [X if x == "k" else next(place) for x, _ in b]
+    A, B = rnd(1 << (m + k), 1), rnd(1 << (n + k), 2)
+    want, _ = oracle.contract(A, da, B, db, wires, r1, r2)
+    got, _, _ = ops.contract(dev(A), da, dev(B), db, wires, r1, r2)
+    assert same_bits(host(got), want)
