@@ -81,6 +81,7 @@ struct OutGen {
   int rc;
 };
 
+// Tensors beyond 2^32 elements.
 __global__ void __launch_bounds__(kDirThreads) contract_direct_general(const c128 *__restrict__ A,
                                                                        const c128 *__restrict__ B,
                                                                        c128 *__restrict__ C, OutGen out, Closed cl,
@@ -95,6 +96,103 @@ __global__ void __launch_bounds__(kDirThreads) contract_direct_general(const c12
       ob += i * out.cb[p];
     }
     C[e] = closed_sum(A, B, oa, ob, cl);
+  }
+}
+
+// Any dims, tensors of up to 2^32 elements and sums of up to kTermTable terms.
+struct DirectArgs {
+  uint32_t cd[kMaxOut], ca[kMaxOut], cb[kMaxOut];           // as OutGen
+  uint32_t kd[kMaxClosed], ka[kMaxClosed], kb[kMaxClosed];  // as Closed
+  int rc, nw;
+  uint32_t nC, K;
+};
+constexpr uint32_t kTermTable = 1024;
+
+// What bounds it is latency: each workgroup first lists the A and B offsets of
+// the closed tuples in LDS, so that a sum's loads do not wait for an odometer, and
+// four terms are requested together.  Sums of 64 terms or more with few results
+// are taken a wave each (WIDE): its lanes form the products of 64 terms at a time,
+// only the additions, in order, follow one another.  3 x 3 x 1000 x 7 (63 results
+// of 1000 terms): 17 us a call, 208 with an odometer per result; 1000 x 1000 results of
+// 12 terms 19 and 31.
+template <bool WIDE>
+__global__ void __launch_bounds__(kDirThreads) contract_direct_table(const c128 *__restrict__ A,
+                                                                     const c128 *__restrict__ B, c128 *__restrict__ C,
+                                                                     DirectArgs g) {
+  __shared__ uint2 term[kTermTable];
+  __shared__ c128 prod[WIDE ? kDirThreads : 1];
+  const uint32_t tid = threadIdx.x, K = g.K;
+  for (uint32_t t = tid; t < K; t += kDirThreads) {
+    uint32_t rest = t, oa = 0, ob = 0;
+    for (int w = g.nw - 1; w >= 0; --w) {
+      const uint32_t d = g.kd[w], i = rest % d;
+      rest /= d;
+      oa += i * g.ka[w];
+      ob += i * g.kb[w];
+    }
+    term[t] = uint2{oa, ob};
+  }
+  __syncthreads();
+  const uint32_t per_block = WIDE ? kDirThreads / 64 : kDirThreads;
+  const uint32_t mine = WIDE ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)) : tid;
+  for (uint64_t e64 = (uint64_t)blockIdx.x * per_block + mine; e64 < g.nC; e64 += (uint64_t)gridDim.x * per_block) {
+    uint32_t rest = (uint32_t)e64, oa = 0, ob = 0;
+    for (int p = g.rc - 1; p >= 0; --p) {
+      const uint32_t d = g.cd[p], i = rest % d;
+      rest /= d;
+      oa += i * g.ca[p];
+      ob += i * g.cb[p];
+    }
+    const c128 *pa = A + oa, *pb = B + ob;
+    if constexpr (WIDE) {
+      const uint32_t lane = tid & 63;
+      c128 *slot = prod + (tid & ~63u);
+      auto get = [&](uint32_t t, c128 &a, c128 &b) {  // past the last term: the last one, not added
+        const uint2 o = term[t < K ? t : K - 1];
+        a = pa[o.x];
+        b = pb[o.y];
+      };
+      double sum = 0.0;  // lane 0: real part, lane 1: imaginary part
+      c128 a, b;
+      get(lane, a, b);
+      for (uint32_t r = 0; r < K; r += 64) {
+        slot[lane] = c128{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+        get(r + 64 + lane, a, b);  // arrives during the additions
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double *part = reinterpret_cast<const double *>(slot) + (lane & 1);
+        if (r + 64 <= K) {
+#pragma unroll 16
+          for (int i = 0; i < 64; ++i) sum = sum + part[2 * i];
+        } else {
+          for (uint32_t i = 0; i < K - r; ++i) sum = sum + part[2 * i];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      if (lane < 2) reinterpret_cast<double *>(C + e64)[lane] = sum;
+    } else {
+      double ar = 0.0, ai = 0.0;
+      uint32_t t = 0;
+      for (; t + 4 <= K; t += 4) {
+        c128 a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint2 o = term[t + u];
+          a[u] = pa[o.x];
+          b[u] = pb[o.y];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) cmac(ar, ai, a[u], b[u]);
+      }
+      for (; t < K; ++t) {
+        const uint2 o = term[t];
+        cmac(ar, ai, pa[o.x], pb[o.y]);
+      }
+      C[e64] = c128{ar, ai};
+    }
   }
 }
 
@@ -599,6 +697,35 @@ qtnh_status launch_contract_direct(qtnh_ctx_t ctx, const c128 *A, int rA, const 
     unsigned blocks = (unsigned)std::min<uint64_t>(nhi, cap);
     hipLaunchKernelGGL(contract_direct_bits, dim3(blocks), dim3(kDirThreads), 0, ctx->stream, A, B, C, ob, cb, P.nC);
     return check_hip(ctx, hipGetLastError(), "contract_direct_bits launch");
+  }
+  uint64_t nA = 1, nB = 1;
+  for (int i = 0; i < rA; ++i) nA *= dA[i];
+  for (int i = 0; i < rB; ++i) nB *= dB[i];
+  if (std::max({nA, nB, P.nC}) < (1ull << 32) && P.K <= kTermTable) {
+    DirectArgs g;
+    g.rc = P.rC;
+    g.nw = P.nw;
+    g.nC = (uint32_t)P.nC;
+    g.K = (uint32_t)P.K;
+    for (int p = 0; p < P.rC; ++p) {
+      const int q = inv[p];
+      g.cd[p] = (uint32_t)P.dC[p];
+      g.ca[p] = q < n1 ? (uint32_t)stA[P.open1[q]] : 0u;
+      g.cb[p] = q < n1 ? 0u : (uint32_t)stB[P.open2[q - n1]];
+    }
+    for (int w = 0; w < P.nw; ++w) {
+      g.kd[w] = (uint32_t)cl.kd[w];
+      g.ka[w] = (uint32_t)cl.ka[w];
+      g.kb[w] = (uint32_t)cl.kb[w];
+    }
+    // A wave per result from 64 terms and up to 2^10 results, as in launch_direct.
+    const bool wide = P.K >= 64 && P.nC <= 1024;
+    const unsigned blocks = grid_for(P.nC, wide ? kDirThreads / 64 : kDirThreads, 1u << 20);
+    if (wide)
+      hipLaunchKernelGGL((contract_direct_table<true>), dim3(blocks), dim3(kDirThreads), 0, ctx->stream, A, B, C, g);
+    else
+      hipLaunchKernelGGL((contract_direct_table<false>), dim3(blocks), dim3(kDirThreads), 0, ctx->stream, A, B, C, g);
+    return check_hip(ctx, hipGetLastError(), "contract_direct_table launch");
   }
   OutGen og;
   memset(&og, 0, sizeof(og));

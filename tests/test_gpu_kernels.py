@@ -613,3 +613,28 @@ def test_contract_direct_matches_oracle_bitwise(m, n, k, widest):
     want, _ = oracle.contract(A, da, B, db, wires, r1, r2)
     got, _, _ = ops.contract(dev(A), da, dev(B), db, wires, r1, r2)
     assert same_bits(host(got), want)
+
+
+@pytest.mark.parametrize("dm,dn,dk", [
+    ([3], [5], [3]), ([7, 3], [2, 2], [4]), ([5], [1], [5, 3]), ([], [], [7]),
+    ([3], [3], [9, 7]), ([3, 2], [3], [64]), ([1], [3, 1], [5, 13]), ([3], [1], [10, 10]),  # 63, 64, 65, 100 terms
+    ([31], [33], [2, 32, 3]), ([5, 5], [41], [3, 43]), ([3], [21], [8, 125]),                # to and past 2^10 results
+    ([], [3], [1023]), ([3], [], [2, 512]), ([50, 20], [61], [3, 5]), ([600], [700], [3]),
+])
+def test_contract_direct_ragged_matches_oracle_bitwise(dm, dn, dk):
+    """Direct contractions over any dims, with shuffled axes, wires and result
+    placement: remainders of four and of 64 terms, the lines between the forms."""
+    rng = np.random.default_rng(len(dm) + 10 * len(dn) + 100 * sum(dk))
+    a = [("m", i) for i in range(len(dm))] + [("k", i) for i in range(len(dk))]
+    b = [("n", i) for i in range(len(dn))] + [("k", i) for i in range(len(dk))]
+    a, b = [a[i] for i in rng.permutation(len(a))], [b[i] for i in rng.permutation(len(b))]
+    size = {"m": dm, "n": dn, "k": dk}
+    da, db = [size[x][i] for x, i in a], [size[x][i] for x, i in b]
+    wires = [(a.index(("k", i)), b.index(("k", i))) for i in rng.permutation(len(dk))]
+    place = iter(int(v) for v in rng.permutation(len(dm) + len(dn)))
+    r1 = [X if x == "k" else next(place) for x, _ in a]
+    r2 = [X if x == "k" else next(place) for x, _ in b]
+    A, B = rnd(int(np.prod(da)), 1), rnd(int(np.prod(db)), 2)
+    want, _ = oracle.contract(A, da, B, db, wires, r1, r2)
+    got, _, _ = ops.contract(dev(A), da, dev(B), db, wires, r1, r2)
+    assert same_bits(host(got), want)
