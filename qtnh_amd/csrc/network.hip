@@ -1552,6 +1552,19 @@ struct Wave {
         }
         if (!R.idC) add_perm(pout, r_pout[s], pc, Cw, Cp);
       }
+      // The deepest tiles of a launch start first: left to the end, they would run
+      // on alone.
+      for (int bi = 0; bi < 2; ++bi) {
+        const auto b = zg[bi].begin() + r_zg[bi][s].b, e = zg[bi].begin() + std::max(r_zg[bi][s].b, r_zg[bi][s].e);
+        std::stable_sort(b, e, [](const ZGroupDesc &x, const ZGroupDesc &y) {
+          return std::min(x.kc, x.K) > std::min(y.kc, y.K);
+        });
+        uint64_t first = 0;
+        for (auto d = b; d != e; ++d) {
+          d->first = first;
+          first += d->tiles * ((d->K + d->kc - 1) / d->kc);
+        }
+      }
     }
   }
 
