@@ -387,7 +387,7 @@ qtnh_status qtnh_expect_z_c128(qtnh_ctx_t ctx, const void *state, int n_qubits, 
  * depend on them.  Setting them turns per-permutation tuning off. */
 void qtnh_tune_permute(int a, int b, int u_target, int order, int nt, int blocks_per_cu);
 /* Per-permutation tuning of the power-of-two permute (on by default): the
- * first permute of >= 2^23 elements with a new bit permutation on a device
+ * first permute of >= 2^24 elements with a new bit permutation on a device
  * times a few tile shapes on the caller's buffers (one stream synchronisation;
  * skipped while the stream is being captured) and keeps the fastest.  on = 1
  * restores the default tile and clears the tuned shapes; 0 uses the set tile

@@ -249,7 +249,8 @@ qtnh_status launch_zgemm_grouped_sum(qtnh_ctx_t ctx, const ZSumDesc *d, int nd, 
 qtnh_status launch_splitk_grouped(qtnh_ctx_t ctx, const SkDesc *d, int nd, uint64_t total_partial,
                                   uint64_t total_final);
 qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, uint64_t total_blocks);
-// Two of them in one launch, descriptors by value.
+// One of them, and two in one launch, descriptors by value.
+qtnh_status launch_permute_tiles(qtnh_ctx_t ctx, const PermDesc &d);
 qtnh_status launch_permute_pair(qtnh_ctx_t ctx, const PermDesc &a, const PermDesc &b);
 // Tile edge (32 or 64) of a shape in grouped launches, and the depth chunks
 // (length on BK steps, count) of launch_zgemm_f64, which they share.

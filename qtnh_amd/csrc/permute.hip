@@ -489,7 +489,7 @@ static PermTune g_perm;
 // tiles, gives 5.9-6.0 on some permutations and 4.7 on others; where the
 // natural tile is short, filling it with outer bits near 2^10 gives 6.0-6.2
 // against 5.4-5.7 for longer runs), and every shape writes the same bits.  So the first permute of a
-// large state (>= 2^23 elements) with a new (bit count, bit permutation)
+// large state (>= 2^24 elements; dense gates in its tiles: >= 2^23) with a new (bit count, bit permutation)
 // signature on a device times each candidate below on the caller's buffers
 // and keeps the fastest for that signature.  The timing synchronises the
 // stream once; it is skipped (defaults used, nothing cached) while the stream
@@ -1116,6 +1116,8 @@ qtnh_status launch_permute_box(qtnh_ctx_t ctx, const c128 *src, c128 *dst, uint6
 }
 }  // namespace
 
+constexpr int kPermTileMaxBits = 23;
+
 qtnh_status launch_permute(qtnh_ctx_t ctx, const c128 *src, c128 *dst, int rank, const uint64_t *dims,
                            const uint16_t *ptup) {
   uint64_t n;
@@ -1136,8 +1138,16 @@ qtnh_status launch_permute(qtnh_ctx_t ctx, const c128 *src, c128 *dst, int rank,
     for (int i = 0; i < rank; ++i)
       for (int t = 0; t < in.width[i]; ++t) sigma[in.shift[i] + t] = out.shift[ptup[i]] + t;
     for (int p = 0; p < nb; ++p) inv[sigma[p]] = p;
+    // Up to 2^23 elements one block per tile is the faster: 2.6 us against 3.9 at
+    // 2^12 elements, 3.6 against 6.0 at 2^18, 6 against 8.5 at 2^20, 39 against 46 to
+    // 55 at 2^23; at 2^24 the tuned kernel takes 86 to 119 us and this one 91 to 118.
+    PermDesc d;
+    if (g_perm_auto && nb <= kPermTileMaxBits && plan_permute_tiles(rank, dims, ptup, &d)) {
+      d.src = src;
+      d.dst = dst;
+      return launch_permute_tiles(ctx, d);
+    }
     PermTune cfg = g_perm;
-    if (g_perm_auto && n < kStreamMin) cfg.nt = 0;
     if (g_perm_auto && n >= kPermAutoMin) {
       std::string key((const char *)&ctx->device, sizeof(int));
       for (int p = 0; p < nb; ++p) key.push_back((char)sigma[p]);
@@ -1256,6 +1266,8 @@ __global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__
   permute_tile(D, blockIdx.x - (uint32_t)D.first);
 }
 
+__global__ void __launch_bounds__(256) permute_one_kernel(PermDesc d) { permute_tile(d, blockIdx.x); }
+
 struct PermPair {
   PermDesc d[2];
 };
@@ -1328,6 +1340,11 @@ qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, ui
   if (nd <= 0 || total == 0) return QTNH_OK;
   hipLaunchKernelGGL(permute_grouped_kernel, dim3((unsigned)total), dim3(256), 0, ctx->stream, d, nd);
   return check_hip(ctx, hipGetLastError(), "grouped permute launch");
+}
+
+qtnh_status launch_permute_tiles(qtnh_ctx_t ctx, const PermDesc &d) {
+  hipLaunchKernelGGL(permute_one_kernel, dim3(d.blocks), dim3(256), 0, ctx->stream, d);
+  return check_hip(ctx, hipGetLastError(), "permute launch");
 }
 
 qtnh_status launch_permute_pair(qtnh_ctx_t ctx, const PermDesc &a, const PermDesc &b) {

@@ -638,3 +638,23 @@ def test_contract_direct_ragged_matches_oracle_bitwise(dm, dn, dk):
     want, _ = oracle.contract(A, da, B, db, wires, r1, r2)
     got, _, _ = ops.contract(dev(A), da, dev(B), db, wires, r1, r2)
     assert same_bits(host(got), want)
+
+
+@pytest.mark.parametrize("dims", [[2] * 3, [2] * 9, [2] * 10, [2] * 11, [4, 2, 8, 2, 4], [1, 16, 1, 64, 2], [2] * 16,
+                                  [2] * 23, [2] * 24, [8, 4, 16, 2, 2, 32, 64, 8]])
+def test_permute_tiles_bitwise(dims):
+    """Power-of-two dims below, at and above a tile and on both sides of the
+    largest tensor that is moved a tile per block."""
+    x = ops.fill_(ops.empty(int(np.prod(dims))), 3)
+    rng = np.random.default_rng(len(dims))
+    n = len(dims)
+    for p in (rng.permutation(n), rng.permutation(n), np.arange(n)[::-1], np.roll(np.arange(n), 1)):
+        p = [int(v) for v in p]
+        # Source index of every result element, axis by axis from the last of the result.
+        left, source = torch.arange(x.numel(), device="cuda"), torch.zeros(x.numel(), dtype=torch.int64, device="cuda")
+        for i in reversed([p.index(k) for k in range(n)]):
+            source += left % dims[i] * int(np.prod(dims[i + 1:]))
+            left = left // dims[i]
+        got = ops.permute(x, dims, p)
+        assert torch.equal(torch.view_as_real(got).view(torch.int64),
+                           torch.view_as_real(x[source]).view(torch.int64)), p
