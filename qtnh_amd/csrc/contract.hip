@@ -903,7 +903,7 @@ qtnh_status launch_contract(qtnh_ctx_t ctx, const c128 *A, int rA, const uint64_
   qtnh_status st = QTNH_OK;
   PermDesc pa, pb;
   // Both operands of a contraction over power-of-two dims go in one launch while
-  // neither is large: 2^19 elements each take 7 us so and 18 in two launches of
+  // neither is large: 2^19 elements each take 10 us so and 18 in two launches of
   // the tuned kernel, a contraction with an operand of 2^22 elements 48 us and
   // 54; with one of 2^24, which fills the chip by itself, 181 us and 178.
   if (!L.idA && !L.idB && std::max(P.M, P.N) * P.K <= kPairMaxElems && plan_permute_tiles(rA, dA, L.pA.data(), &pa) &&
