@@ -414,8 +414,9 @@ uint64_t zgemm_chunks_large(uint64_t M, uint64_t N, uint64_t K) {
 // 32 x 64 tile 0.96, of a 32 x 32 tile 0.5 (1.0 and 0.6 where a compute unit
 // has only one); the second kernel that sums depth chunks 5.5 us and its
 // traffic.  A launch takes as long as the fullest of 256 compute units.
-// Depends on the shape only: the network planner sizes workspaces with it, and
-// every caller of a shape runs the same chunks.  (64 x 64 tiles or 64 x 128
+// The chunks depend on the shape only, also where the tiles are set: the network
+// planner sizes workspaces with them, and every caller of a shape runs the same
+// ones.  (64 x 64 tiles or 64 x 128
 // ones alone, the rule before: 512^3 92 us, now 25 with 32 x 32 tiles; 256 x
 // 512 x 256 85 and 14; 700^3 107 and 57; 4096^3 8.10 and 7.74 ms.)
 struct ZShape {
@@ -434,7 +435,6 @@ static ZShape zgemm_shape(uint64_t M, uint64_t N, uint64_t K) {
   ZShape best{64, 64, K, 1};
   double t_best = 0.0;
   for (const Tile &t : kTiles) {
-    if (g_zgemm_bn && t.bm != 64) continue;
     const uint64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     uint64_t last = 0;
     for (uint64_t want = 1; want <= 64; want += want < 4 ? 1 : want / 2) {
@@ -453,6 +453,7 @@ static ZShape zgemm_shape(uint64_t M, uint64_t N, uint64_t K) {
       }
     }
   }
+  if (g_zgemm_bn) best.bm = best.bn = 64;
   return best;
 }
 

@@ -391,3 +391,25 @@ def test_grouped_direct_steps_bitwise(m, n, k):
             assert same_bits(s, b)
             assert same_bits(s, g)
     prepared.close()
+
+
+@pytest.mark.parametrize("m,n,k", [(10, 8, 9), (9, 9, 9)])
+def test_gemm_tile_setting_after_planning(m, n, k):
+    """Batches of networks planned before the GEMM's tiles were set: the same
+    depth chunks, the same bits."""
+    nets = []
+    for seed in range(2):
+        rng = np.random.default_rng(seed)
+        net = ops.Network()
+        for l in (range(m + k), range(m, m + k + n)):
+            net.add([2] * len(l), l, rng.standard_normal(1 << len(l)) + 1j * rng.standard_normal(1 << len(l)))
+        nets.append(net.plan(0, 64))
+    want = [x.run() for x in nets]
+    ops.tune_zgemm(64)
+    try:
+        got, _ = ops.run_networks(nets)
+        solo = [x.run() for x in nets]
+    finally:
+        ops.tune_zgemm(0)
+    for w, g, s in zip(want, got, solo):
+        assert same_bits(w, g) and same_bits(w, s)

@@ -260,3 +260,22 @@ def test_plan_best_rank_cap():
     with pytest.raises(_lib.QtnhError) as e:
         ops.Network.amplitude(c).plan_best(0, 6, 16)
     assert e.value.status == _lib.QTNH_EUNSUPPORTED
+
+
+@pytest.mark.parametrize("m,n,k", [(10, 8, 9), (9, 9, 9), (8, 9, 8)])
+def test_gemm_tile_setting_leaves_the_workspace_alone(m, n, k):
+    """A plan's workspace and its batch run's layout use the same depth chunks
+    whatever tiles are set in between."""
+    def device_bytes():
+        net = ops.Network()
+        net.add([2] * (m + k), range(m + k), np.zeros(1 << (m + k)))
+        net.add([2] * (k + n), range(m, m + k + n), np.zeros(1 << (k + n)))
+        return net.plan(0, 64).info()["device_bytes"]
+
+    by_size = device_bytes()
+    try:
+        for bn in (64, 128):
+            ops.tune_zgemm(bn)
+            assert device_bytes() == by_size, bn
+    finally:
+        ops.tune_zgemm(0)
