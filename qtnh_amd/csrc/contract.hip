@@ -580,6 +580,8 @@ qtnh_status launch_contract_direct(qtnh_ctx_t ctx, const c128 *A, int rA, const 
                                    const uint64_t *dB, int nw, const uint16_t *wires, const uint16_t *r1,
                                    const uint16_t *r2, c128 *C) {
   Plan P = make_plan(rA, dA, rB, dB, nw, wires, r1, r2);
+  // Empty sums: the result is zero.
+  if (P.K == 0) return launch_zero(ctx, C, P.nC * sizeof(c128));
   if (P.nw > kMaxClosed || P.rC > kMaxOut)
     return set_error(ctx, QTNH_EUNSUPPORTED, "contract: %d closed / %d result axes exceed the direct kernel", P.nw,
                      P.rC);
@@ -593,10 +595,6 @@ qtnh_status launch_contract_direct(qtnh_ctx_t ctx, const c128 *A, int rA, const 
     cl.kd[w] = dA[P.cA[w]];
     cl.ka[w] = stA[P.cA[w]];
     cl.kb[w] = stB[P.cB[w]];
-  }
-  if (P.K == 0) {
-    // Empty sums: the result is zero.
-    return launch_zero(ctx, C, P.nC * sizeof(c128));
   }
   // Natural axis q -> source stride (A or B); result axis p holds natural axis inv[p].
   const int n1 = (int)P.open1.size();
@@ -745,8 +743,10 @@ qtnh_status launch_contract_direct(qtnh_ctx_t ctx, const c128 *A, int rA, const 
 
 // Route choice: the direct kernel sums K operand pairs per result element in
 // one thread, with no reuse, which is cheap while the sums are short (gates)
-// or the whole contraction is small and its sums stay short.
+// or the whole contraction is small and its sums stay short.  Empty sums need no
+// kernel of either route.
 static bool use_direct(const Plan &P) {
+  if (P.K == 0) return true;
   if (P.nw > kMaxClosed || P.rC > kMaxOut) return false;
   return P.K <= 16 || (P.M * P.N * P.K <= (1ull << 20) && P.K <= 1024);
 }

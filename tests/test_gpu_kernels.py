@@ -5,6 +5,7 @@ gates (the kernels keep the reference's summation order and separate
 rounding), and for small contractions (direct route).  The GEMM route is
 checked at relative error <= 1e-12 (the FP64 target).
 """
+import ctypes
 import math
 import random
 
@@ -658,3 +659,31 @@ def test_permute_tiles_bitwise(dims):
         got = ops.permute(x, dims, p)
         assert torch.equal(torch.view_as_real(got).view(torch.int64),
                            torch.view_as_real(x[source]).view(torch.int64)), p
+
+
+@pytest.mark.parametrize("precision", [_lib.PREC_FP64, _lib.PREC_SPLIT])
+@pytest.mark.parametrize("opened,closed", [
+    ([9], [0]), ([2] * 3, [0, 3]),                   # few axes
+    ([9], [1] * 30 + [0]), ([2] * 4, [0] + [2] * 25),  # more wires than the direct kernels take
+    ([3] * 2 + [1] * 26, [5, 0]),                    # more result axes than they take
+])
+def test_contract_empty_sums(opened, closed, precision):
+    """A closed dim of 0: every result is zero, whatever the axes."""
+    da, db = opened + closed, closed + opened
+    wires = [(len(opened) + i, i) for i in range(len(closed))]
+    empty = torch.empty(0, dtype=torch.complex128, device="cuda")
+    n = int(np.prod(opened)) ** 2
+    out = torch.full((n,), float("nan"), dtype=torch.complex128, device="cuda")
+    got, dc, err = ops.contract(empty, da, empty, db, wires, precision=precision, out=out)
+    assert dc == opened + opened and err == 0.0
+    assert np.array_equal(host(got).view(np.uint64), np.zeros(2 * n, dtype=np.uint64))
+    out.fill_(float("nan"))
+    u64, u16 = ops._u64, ops._u16
+    r1, r2 = ops.default_repls(len(da), 0, len(db), 0, wires)
+    args = [u64(da), u64(db), u16([v for w in wires for v in w]), u16(r1), u16(r2)]
+    eta = ctypes.c_double(-1.0)
+    _lib.check(_lib.lib().qtnh_contract_c128_noalloc(
+        ops.context(), None, len(da), args[0][1], None, len(db), args[1][1], len(wires), args[2][1], args[3][1],
+        args[4][1], ctypes.c_void_p(out.data_ptr()), precision, ctypes.byref(eta)), ops.context())
+    assert eta.value == 0.0
+    assert np.array_equal(host(out).view(np.uint64), np.zeros(2 * n, dtype=np.uint64))
