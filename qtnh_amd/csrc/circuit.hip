@@ -1540,11 +1540,15 @@ void add_group(const std::vector<RunRef> &refs, std::vector<RunDesc> &descs, std
 }
 
 // One workgroup per tile (a grid of resident workgroups walking the tiles ran
-// 10% longer at 28 qubits: its workgroups stay in step, all loading at a time).
+// 10% longer at 28 qubits: its workgroups stay in step, all loading at a time),
+// up to a grid whose threads stay below 2^32; beyond it, which takes states of
+// at least 24 qubits more than their tiles have, workgroups walk several.
+constexpr uint64_t kRegMaxBlocks = 1u << 23;
+
 template <int R, int KD, int MINW>
 void launch_reg(qtnh_ctx_t ctx, const RunDesc *d, int nr, uint64_t total, int tb) {
   const unsigned threads = std::max(64, 1 << (tb - R));
-  const unsigned blocks = (unsigned)std::min<uint64_t>(total, 1u << 30);
+  const unsigned blocks = (unsigned)std::min(total, kRegMaxBlocks);
   const size_t lds = (sizeof(double) << tb) + kRegCoef * sizeof(double2_t) + (kRegOps + 2) * sizeof(RegOp);
   hipLaunchKernelGGL((circuit_reg_kernel<R, KD, MINW>), dim3(blocks), dim3(threads), lds, ctx->stream, d, nr, total, tb);
 }

@@ -273,3 +273,28 @@ def test_register_runs_of_several_widths_in_one_launch(dense3):
     ops.run_batch(cs, states)
     for n, s, ref in zip(sizes, states, refs):
         assert same_bits(host(s), ref), n
+
+
+@pytest.mark.parametrize("dense3", [False, True])
+@pytest.mark.parametrize("sizes", [[28], [27, 26, 20]])
+def test_register_runs_walk_several_tiles(sizes, dense3):
+    """4-bit tiles of large states: more tiles than a launch has workgroups, so
+    a workgroup takes several, of one run and of several in turn, with more ops
+    than one staged chunk holds."""
+    ops.tune_circuit(4, 1)
+    try:
+        cs = []
+        for n in sizes:
+            c = _mixed_circuit(n, 20, dense3, n)
+            for i in range(60):  # one run, two chunks of ops
+                c.diag([i % n, (i + 5) % n], np.exp(1j * np.arange(4)))
+            cs.append(c)
+        got = [ops.fill_(ops.empty(1 << n), n) for n in sizes]
+        want = [ops.fill_(ops.empty(1 << n), n) for n in sizes]
+        ops.run_batch(cs, got)
+        for c, w in zip(cs, want):
+            c.run(w, _lib.RUN_PER_GATE)
+        for g, w in zip(got, want):
+            assert torch.equal(torch.view_as_real(g).view(torch.int64), torch.view_as_real(w).view(torch.int64))
+    finally:
+        ops.tune_circuit(12)
