@@ -25,8 +25,9 @@ constexpr int kGateThreads = 256;
 // Most workgroups of the streaming gate and diagonal kernels (they loop over
 // the rest): enough to keep many requests in flight on every CU.
 unsigned g_stream_blocks = 1u << 20;
-// Grid limit of the kernels sized to one element (or row) per thread.
-constexpr unsigned kMaxStreamBlocks = 1u << 30;
+// Grid limit of the kernels sized to one element (or row) per thread: a launch
+// takes fewer than 2^32 threads.  They loop over the rest, too.
+constexpr unsigned kMaxStreamBlocks = 1u << 23;
 
 __device__ inline c128 cmul(c128 a, c128 b) {
   c128 r;

@@ -687,3 +687,20 @@ def test_contract_empty_sums(opened, closed, precision):
         args[4][1], ctypes.c_void_p(out.data_ptr()), precision, ctypes.byref(eta)), ops.context())
     assert eta.value == 0.0
     assert np.array_equal(host(out).view(np.uint64), np.zeros(2 * n, dtype=np.uint64))
+
+
+def test_gates_beyond_one_launch_of_threads():
+    """32 qubits (64 GiB), an element or a row for each of 2^32 threads: a gate
+    on the lowest bit and a diagonal, on stretches over the whole state."""
+    n = 32
+    x = ops.fill_(ops.empty(1 << n), 5)
+    at = [0, (1 << 31) - (1 << 12), 1 << 31, 3 << 30, (1 << n) - (1 << 12)]
+    before = [host(x[i:i + (1 << 12)]) for i in at]
+    g = rnd(4, 1)
+    d = rnd(2, 2)
+    ops.gate_apply_(x, [2] * n, [n - 1], g)
+    ops.diag_apply_(x, [2] * n, [0], d)
+    for i, b in zip(at, before):
+        want = oracle.gate_apply(b, [2] * 12, [11], g)
+        want = oracle.diag_apply(want, [2] * 12, [0], [d[i >> 31]] * 2)
+        assert same_bits(host(x[i:i + (1 << 12)]), want), i
