@@ -1079,7 +1079,14 @@ qtnh_status launch_permute_box(qtnh_ctx_t ctx, const c128 *src, c128 *dst, uint6
   // elements; of 10: 400 against 351 for 60M).  And for small tensors, which
   // the caches hold: a tile's setup costs more than the scattered reads (90000
   // elements 3.7 us against 4.6; 360000: 9.2 against 5.6).
-  if (n < (1ull << 18) || (S.res[S.rank - 1] == S.rank - 1 && S.d[S.rank - 1] >= 16)) {
+  // And where the tiles' 32-bit counts do not take the shape (an axis of 2^32
+  // elements or more that a tile cuts).
+  BoxArgs A;
+  uint64_t n_tiles;
+  size_t lds_elems;
+  bool cut;
+  if (n < (1ull << 18) || (S.res[S.rank - 1] == S.rank - 1 && S.d[S.rank - 1] >= 16) ||
+      !plan_box(S, n, A, &n_tiles, &lds_elems, &cut)) {
     PermGenArgs g;
     memset(&g, 0, sizeof(g));
     g.rank = S.rank;
@@ -1091,12 +1098,6 @@ qtnh_status launch_permute_box(qtnh_ctx_t ctx, const c128 *src, c128 *dst, uint6
     hipLaunchKernelGGL(permute_general_kernel, dim3(blocks), dim3(256), 0, ctx->stream, src, dst, g, n);
     return check_hip(ctx, hipGetLastError(), "permute_general launch");
   }
-  BoxArgs A;
-  uint64_t n_tiles;
-  size_t lds_elems;
-  bool cut;
-  if (!plan_box(S, n, A, &n_tiles, &lds_elems, &cut))
-    return set_error(ctx, QTNH_EINVAL, "permute: no tile for this shape");
   const size_t lds = lds_elems * sizeof(c128);
   const bool wide = n > 0xffffffffull, stream = n >= kStreamMin;
   // The resident workgroups of a 64 KiB tile, each walking its share.

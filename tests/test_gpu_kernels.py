@@ -704,3 +704,22 @@ def test_gates_beyond_one_launch_of_threads():
         want = oracle.gate_apply(b, [2] * 12, [11], g)
         want = oracle.diag_apply(want, [2] * 12, [0], [d[i >> 31]] * 2)
         assert same_bits(host(x[i:i + (1 << 12)]), want), i
+
+
+@pytest.mark.parametrize("short_first", [False, True])
+def test_permute_axis_beyond_32_bits(short_first):
+    """An axis of more than 2^32 elements beside one of 2 (128 GiB a side)."""
+    d = (1 << 32) + 7
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 260 << 30:
+        pytest.skip("needs 256 GiB of free device memory")
+    dims = [2, d] if short_first else [d, 2]
+    x = ops.fill_(ops.empty(2 * d), 3)
+    y = ops.permute(x, dims, [1, 0])
+    a, b = x.view(dims), y.view(dims[::-1])
+    for i in (0, (1 << 31) - 512, (1 << 32) - 512, d - 1024):
+        for j in range(2):
+            s, t = (a[j, i:i + 1024], b[i:i + 1024, j]) if short_first else (a[i:i + 1024, j], b[j, i:i + 1024])
+            assert torch.equal(s, t), (i, j)
+    del x, y, a, b, s, t
+    torch.cuda.empty_cache()
