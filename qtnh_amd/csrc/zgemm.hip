@@ -26,6 +26,8 @@ constexpr int kThreads = 256;
 
 constexpr int kFold = 256;  // terms per accumulator set
 
+constexpr uint64_t kMaxTiles = (1ull << 32) / kThreads - 1;  // a launch takes fewer than 2^32 threads
+
 template <int BM, int BN>
 struct ZTile {
   static constexpr int LDA = BK + 1;  // padded LDS rows (complex elements)
@@ -443,6 +445,7 @@ static ZShape zgemm_shape(uint64_t M, uint64_t N, uint64_t K) {
       const uint64_t chunks = (K + kc - 1) / kc;
       if (chunks > 1 && (kc < 64 || chunks == last)) continue;
       if (chunks > large && own + chunks * M * N > room) continue;
+      if (tiles > kMaxTiles / chunks) continue;
       last = chunks;
       const double per = (double)((tiles * chunks + 255) / 256), stages = (double)((kc + BK - 1) / BK);
       double us = 5.0 + stages * (per * t.stage + (per > 1 ? 0.0 : t.alone));
@@ -480,7 +483,7 @@ qtnh_status launch_zgemm_f64(qtnh_ctx_t ctx, const c128 *A, const c128 *B, c128 
                              uint64_t lda, uint64_t ldb, uint64_t ldc, c128 *partials) {
   const ZShape z = zgemm_shape(M, N, K);
   const uint64_t tiles = ((N + z.bn - 1) / z.bn) * ((M + z.bm - 1) / z.bm);
-  if (tiles > 0x7fffffffull / z.chunks) return set_error(ctx, QTNH_EUNSUPPORTED, "zgemm: grid too large");
+  if (tiles > kMaxTiles / z.chunks) return set_error(ctx, QTNH_EUNSUPPORTED, "zgemm: grid too large");
   if (z.chunks > 1 && !partials) return set_error(ctx, QTNH_EINVAL, "zgemm: depth chunks need a partial buffer");
   c128 *out = z.chunks > 1 ? partials : C;
   const uint64_t ld = z.chunks > 1 ? N : ldc, cstride = z.chunks > 1 ? M * N : 0;

@@ -723,3 +723,21 @@ def test_permute_axis_beyond_32_bits(short_first):
             assert torch.equal(s, t), (i, j)
     del x, y, a, b, s, t
     torch.cuda.empty_cache()
+
+
+def test_contract_gemm_more_small_tiles_than_a_launch_takes():
+    """2^29 rows and few columns: 32 x 32 tiles would be 2^24 workgroups of 256
+    threads (a 136 GiB operand, the shortest depth of this route)."""
+    m, n, k = (1 << 29) + 3, 2, 17
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 170 << 30:
+        pytest.skip("needs 160 GiB of free device memory")
+    a = ops.fill_(ops.empty(m * k), 7)
+    b = rnd(k * n, 8)
+    got, _, _ = ops.contract(a, [m, k], dev(b), [k, n], [(1, 0)])
+    rows = a.view(m, k)
+    for i in (0, (1 << 28) - 32, m // 2, m - 64):
+        want = host(rows[i:i + 64]) @ b.reshape(k, n)
+        assert np.linalg.norm(host(got.view(m, n)[i:i + 64]) - want) <= 1e-12 * np.linalg.norm(want), i
+    del a, got, rows
+    torch.cuda.empty_cache()
