@@ -285,6 +285,11 @@ qtnh_status symm_repls(int r1, int nd2, int nl2, int n_dis_in, int nw, const uin
 qtnh_status contract_dims(int rA, const uint64_t *dA, int rB, const uint64_t *dB, int nw, const uint16_t *wires,
                           const uint16_t *repl1, const uint16_t *repl2, int *rC, uint64_t *dC);
 
+// Most workgroups of one launch of a kernel whose grid has a block per piece of
+// work (up to 256 threads each): the runtime counts a launch's threads in 32
+// bits and wraps past them.
+constexpr uint64_t kMaxGridBlocks = 1ull << 23;
+
 // Grid helper: at most `cap` blocks of `threads`, enough for `work` items.
 inline unsigned grid_for(uint64_t work, unsigned threads, unsigned cap) {
   uint64_t b = (work + threads - 1) / threads;

@@ -218,9 +218,11 @@ __device__ __forceinline__ void direct_block(const GDesc &D, uint32_t block) {
   }
 }
 
-__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd) {
-  const GDesc &D = descs[find_entry(descs, nd, blockIdx.x)];
-  direct_block(D, blockIdx.x - (uint32_t)D.first);
+__global__ void __launch_bounds__(kGThreads) grouped_direct_kernel(const GDesc *__restrict__ descs, int nd,
+                                                                   uint64_t from) {
+  const uint64_t block = from + blockIdx.x;
+  const GDesc &D = descs[find_entry(descs, nd, block)];
+  direct_block(D, (uint32_t)(block - D.first));
 }
 
 __global__ void __launch_bounds__(kGThreads) direct_kernel(GDesc D) { direct_block(D, blockIdx.x); }
@@ -1725,11 +1727,13 @@ struct Wave {
     for (size_t s = s0; s < s1; ++s) {
       const size_t b = starts[s], e = starts[s + 1];
       if (e > b) {
-        const uint64_t grid = hdesc[e - 1].first + hdesc[e - 1].blocks;
-        hipLaunchKernelGGL(grouped_direct_kernel, dim3((unsigned)grid), dim3(kGThreads), 0, ctx->stream, ddesc + b,
-                           (int)(e - b));
-        qtnh_status st = check_hip(ctx, hipGetLastError(), "grouped contraction launch");
-        if (st) return st;
+        const uint64_t total = hdesc[e - 1].first + hdesc[e - 1].blocks;
+        for (uint64_t from = 0; from < total; from += kMaxGridBlocks) {
+          hipLaunchKernelGGL(grouped_direct_kernel, dim3((unsigned)std::min(total - from, kMaxGridBlocks)),
+                             dim3(kGThreads), 0, ctx->stream, ddesc + b, (int)(e - b), from);
+          qtnh_status st = check_hip(ctx, hipGetLastError(), "grouped contraction launch");
+          if (st) return st;
+        }
       }
       qtnh_status st = enqueue_grouped(ctx, s);
       if (st) return st;

@@ -1262,9 +1262,10 @@ __device__ __forceinline__ void permute_tile(const PermDesc &D, uint32_t t) {
   }
 }
 
-__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd) {
-  const PermDesc &D = d[find_entry(d, nd, blockIdx.x)];
-  permute_tile(D, blockIdx.x - (uint32_t)D.first);
+__global__ void __launch_bounds__(256) permute_grouped_kernel(const PermDesc *__restrict__ d, int nd, uint64_t from) {
+  const uint64_t block = from + blockIdx.x;
+  const PermDesc &D = d[find_entry(d, nd, block)];
+  permute_tile(D, (uint32_t)(block - D.first));
 }
 
 __global__ void __launch_bounds__(256) permute_one_kernel(PermDesc d) { permute_tile(d, blockIdx.x); }
@@ -1338,9 +1339,13 @@ bool plan_permute_tiles(int rank, const uint64_t *dims, const uint16_t *ptup, Pe
 }
 
 qtnh_status launch_permute_grouped(qtnh_ctx_t ctx, const PermDesc *d, int nd, uint64_t total) {
-  if (nd <= 0 || total == 0) return QTNH_OK;
-  hipLaunchKernelGGL(permute_grouped_kernel, dim3((unsigned)total), dim3(256), 0, ctx->stream, d, nd);
-  return check_hip(ctx, hipGetLastError(), "grouped permute launch");
+  qtnh_status st = QTNH_OK;
+  for (uint64_t from = 0; from < total && nd > 0 && !st; from += kMaxGridBlocks) {
+    hipLaunchKernelGGL(permute_grouped_kernel, dim3((unsigned)std::min(total - from, kMaxGridBlocks)), dim3(256), 0,
+                       ctx->stream, d, nd, from);
+    st = check_hip(ctx, hipGetLastError(), "grouped permute launch");
+  }
+  return st;
 }
 
 qtnh_status launch_permute_tiles(qtnh_ctx_t ctx, const PermDesc &d) {

@@ -413,3 +413,17 @@ def test_gemm_tile_setting_after_planning(m, n, k):
         ops.tune_zgemm(0)
     for w, g, s in zip(want, got, solo):
         assert same_bits(w, g) and same_bits(w, s)
+
+
+def test_direct_steps_beyond_one_launch_of_threads():
+    """A step index whose grouped contractions take more than 2^24 workgroups of
+    256 threads: every network's result, the last ones included."""
+    rng = np.random.default_rng(1)
+    net = ops.Network()
+    for l in (range(11), range(5, 16)):
+        net.add([2] * 11, l, rng.standard_normal(1 << 11) + 1j * rng.standard_normal(1 << 11))
+    net.plan(0, 64)
+    want = net.run()
+    got, waves = ops.run_networks([net] * 66000)  # 256 workgroups each
+    assert waves == 1
+    assert all(same_bits(want, g) for g in got)
