@@ -141,10 +141,11 @@ __device__ __forceinline__ uint32_t row_slot(uint32_t k) { return k ^ ((k >> 4) 
 template <int S>
 __global__ void __launch_bounds__(kThreads) split_rows_kernel(const c128 *__restrict__ X, uint64_t rows, uint64_t K,
                                                               int8_t *__restrict__ out, uint64_t plane,
-                                                              uint64_t part_bytes, uint64_t Kp, ScaleOut sc_out) {
+                                                              uint64_t part_bytes, uint64_t Kp, ScaleOut sc_out,
+                                                              uint64_t first) {
   __shared__ c128 tile[kRowTile];
   __shared__ double red[kParts][kThreads / 64];
-  const uint64_t row = blockIdx.x;
+  const uint64_t row = first + blockIdx.x;
   if (row >= rows) return;  // uniform per block
   const c128 *x = X + row * K;
   const bool one_tile = K <= (uint64_t)kRowTile;
@@ -717,8 +718,13 @@ hipError_t split_planes(hipStream_t stream, hipStream_t side, hipEvent_t fork, h
   hipError_t e = hipEventRecord(fork, stream);
   if (e == hipSuccess) e = hipStreamWaitEvent(side, fork, 0);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((split_rows_kernel<S>), dim3((unsigned)M), dim3(kThreads), 0, stream, A, M, K, As, a_plane,
-                     (uint64_t)S * a_plane, Kp, sa);
+  // One block per row.
+  auto split_rows = [&](hipStream_t on, const c128 *X, uint64_t rows, int8_t *out, uint64_t plane, ScaleOut sc) {
+    for (uint64_t first = 0; first < rows; first += kMaxGridBlocks)
+      hipLaunchKernelGGL((split_rows_kernel<S>), dim3((unsigned)std::min(rows - first, kMaxGridBlocks)),
+                         dim3(kThreads), 0, on, X, rows, K, out, plane, (uint64_t)S * plane, Kp, sc, first);
+  };
+  split_rows(stream, A, M, As, a_plane, sa);
   if (b_cols) {
     // B as K x N: the columns' maxima, then digits read in place.
     hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)std::min<uint64_t>((kParts * N + 255) / 256, 65536)), dim3(256),
@@ -729,9 +735,7 @@ hipError_t split_planes(hipStream_t stream, hipStream_t side, hipEvent_t fork, h
     hipLaunchKernelGGL((split_cols_kernel<S>), dim3((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64)),
                        dim3(kThreads), 0, side, B, K, N, cmax, Bs, b_plane, (uint64_t)S * b_plane, Kp, sb);
   } else {
-    // B^T as N x K: one block per row.
-    hipLaunchKernelGGL((split_rows_kernel<S>), dim3((unsigned)N), dim3(kThreads), 0, side, B, N, K, Bs, b_plane,
-                       (uint64_t)S * b_plane, Kp, sb);
+    split_rows(side, B, N, Bs, b_plane, sb);  // B^T as N x K
   }
   e = hipGetLastError();
   if (e == hipSuccess) e = hipEventRecord(join, side);

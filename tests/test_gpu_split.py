@@ -245,3 +245,21 @@ def test_split_depth_chunks_and_partial_tiles(slices, m, k, n):
     ops.tune_split(5)
     ref = A @ B
     assert np.linalg.norm(C - ref) <= 1e-10 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("side", ["A", "B by rows", "B by columns"])
+def test_split_more_rows_than_a_launch_takes(side):
+    """2^24 rows and more of one operand, whose digits take a workgroup of 256
+    threads a row: sampled results, the last ones included."""
+    big, few, k = (1 << 24) + 200, 5, 17
+    m, n = (big, few) if side == "A" else (few, big)
+    a, b = ops.fill_(ops.empty(m * k), 1), ops.fill_(ops.empty(n * k), 2)
+    db, wires = ([n, k], [(1, 1)]) if side == "B by rows" else ([k, n], [(1, 0)])
+    c, _, eta = ops.contract(a, [m, k], b, db, wires, precision=SPLIT)
+    assert eta > 0
+    A, B = a.view(m, k), b.view(n, k).T if side == "B by rows" else b.view(k, n)
+    C = c.view(m, n)
+    for i in (0, 200, big // 2, big - 64):
+        rows, cols = (slice(i, i + 64), slice(0, n)) if side == "A" else (slice(0, m), slice(i, i + 64))
+        ref = host(A[rows].contiguous()) @ host(B[:, cols].contiguous())
+        assert np.linalg.norm(host(C[rows, cols].contiguous()) - ref) <= 1e-10 * np.linalg.norm(ref), i
