@@ -446,12 +446,12 @@ __global__ void __launch_bounds__(kPipeNT, 1)
 // The op list and its coefficients are staged in LDS by chunks; an op is one
 // 16-byte record, read by every lane from one address and made uniform.
 //
-// Arithmetic: that of gate_in_lds / diag_in_lds.  Their sums start from 0.0:
-// here the first product's leading term is fma(x, y, +0.0), which is x * y
-// rounded, with an exact -0 turned into the +0 that adding to 0.0 gives, one
-// instruction where a multiply and an add were.  (Only a product that
-// underflows to -0 keeps its sign where 0.0 + -0 gave +0, and that shows only
-// if every other term of the sum is -0 as well.)
+// Arithmetic: that of gate_in_lds / diag_in_lds, whose sums start from 0.0.
+// Here they start from the first product, which is the same but for a sum of
+// zeros: -0 where every product is (exactly or by underflow), and +0 there.  A
+// gate's results do not depend on the signs of zeros among its inputs, so a
+// dense record turns -0 into +0 (two additions per amplitude, kRegSettle) only
+// where a diagonal or the store follows.
 struct RegOp {
   // One bit per op form.  1-qubit gates on register bits 3..0 (kRegG1): one
   // record may hold several, applied from the highest bit down, their
@@ -462,11 +462,12 @@ struct RegOp {
   // significant last (31, a zero bit, where there are fewer than three), and
   // their count in byte 3.  kRegSpecial: 0 for a dense 3-qubit gate, else a
   // change of register bits: kRegRemapFlag and their tile positions, 4 bits each.
+  // Dense gates: kRegSettle or 0.
   uint32_t lane;
   uint32_t outer;  // diagonals: bits of the tile number, likewise (63: a zero bit; no count)
 };
 constexpr int kRegG1 = 0, kRegG2 = 4, kRegSpecial = 16, kRegD0 = 17, kRegD1 = 18, kRegD2 = 22, kRegD3 = 28;
-constexpr uint32_t kRegRemapFlag = 1u << 31, kRegNoLane = 0x1f1f1f, kRegNoOuter = 0x3f3f3f;
+constexpr uint32_t kRegRemapFlag = 1u << 31, kRegSettle = 1u << 30, kRegNoLane = 0x1f1f1f, kRegNoOuter = 0x3f3f3f;
 constexpr int kRegOps = 48, kRegCoef = 384;  // per chunk: with a 32 KiB half tile, four workgroups fit 160 KiB
 struct RegChunk {
   uint32_t op_begin, op_end, coef_begin, coef_end;
@@ -531,9 +532,14 @@ __device__ __forceinline__ void sub_to(double &x, double a, double b) {
   asm("v_add_f64 %0, %1, -%2" : "+v"(x) : "v"(a), "v"(b));
 }
 
-// x g, as the first term of a sum from 0.0.
-__device__ __forceinline__ double2_t cmul_first(double2_t x, double2_t g) {
-  return double2_t{__builtin_fma(x.x, g.x, 0.0) - x.y * g.y, __builtin_fma(x.x, g.y, 0.0) + x.y * g.x};
+// -0 becomes +0; other values stay.
+template <int R>
+__device__ __forceinline__ void rg_settle(double (&re)[1 << R], double (&im)[1 << R]) {
+#pragma unroll
+  for (int r = 0; r < (1 << R); ++r) {
+    asm("v_add_f64 %0, %0, 0" : "+v"(re[r]));
+    asm("v_add_f64 %0, %0, 0" : "+v"(im[r]));
+  }
 }
 
 template <int R, int A>
@@ -544,8 +550,8 @@ __device__ __forceinline__ void rg_gate1(double (&re)[1 << R], double (&im)[1 <<
     if ((r >> A) & 1) continue;
     const int s = r | (1 << A);
     const double2_t a = {re[r], im[r]}, b = {re[s], im[s]};
-    const double2_t p0 = cmul_first(a, g00), q0 = cmul2(b, g10);
-    const double2_t p1 = cmul_first(a, g01), q1 = cmul2(b, g11);
+    const double2_t p0 = cmul2(a, g00), q0 = cmul2(b, g10);
+    const double2_t p1 = cmul2(a, g01), q1 = cmul2(b, g11);
     add_to(re[r], p0.x, q0.x);
     add_to(im[r], p0.y, q0.y);
     add_to(re[s], p1.x, q1.x);
@@ -580,7 +586,7 @@ __device__ __forceinline__ void rg_gate(double (&re)[1 << R], double (&im)[1 << 
 #pragma unroll
       for (int o = 0; o < K; ++o) {
         if (o % 4 == 0) asm volatile("" ::: "memory");  // four coefficients live at a time (a compiler barrier, no code)
-        const double2_t p = i == 0 ? cmul_first(x, g[o]) : cmul2(x, g[i * K + o]);
+        const double2_t p = cmul2(x, g[i * K + o]);
         if (i == 0) {
           ar[o] = p.x;
           ai[o] = p.y;
@@ -780,6 +786,7 @@ __global__ void __launch_bounds__(256, MINW)
           QTNH_REG_G1(1)
           QTNH_REG_G1(0)
 #undef QTNH_REG_G1
+          if (lane & kRegSettle) rg_settle<R>(re, im);
           next();
         }
 #define QTNH_REG_DIAG(BIT, NEED, MASK)                                   \
@@ -827,11 +834,14 @@ __global__ void __launch_bounds__(256, MINW)
           QTNH_REG_CASE(14, 3, (rg_gate<R, 2, 3, 1, 0>(re, im, cbuf + co)))
           QTNH_REG_CASE(15, 3, (rg_gate<R, 2, 3, 2, 0>(re, im, cbuf + co)))
 #undef QTNH_REG_CASE
+          if (lane & kRegSettle) rg_settle<R>(re, im);
           next();
         }
         if (code & (1u << kRegSpecial)) {
-          if constexpr (KD > 2 && R > 2)
+          if constexpr (KD > 2 && R > 2) {
             if (!(lane & kRegRemapFlag)) rg_gate<R, 3, 2, 1, 0>(re, im, cbuf + co);
+            if (lane & kRegSettle) rg_settle<R>(re, im);
+          }
           if (lane & kRegRemapFlag) {
             const uint32_t s0 = reg_slot(base);
             uint32_t sb[R];
@@ -1264,14 +1274,18 @@ void plan_reg_run(const qtnh_circuit_s &c, const qtnh_circuit_s::Run &r, int R, 
       room(ncoef);
       RegOp o{0, (uint32_t)(coef.size() / 2), 0, 0};
       if (op.kind == 0) {
+        // A diagonal or the store comes next (register bits may change in between).
+        if (i + 1 == r.end || c.ops[i + 1].kind == 1) o.lane = kRegSettle;
         const int a = reg_bit(tile_bit(op.q[0])), b = op.k > 1 ? reg_bit(tile_bit(op.q[1])) : 0;
         // A 1-qubit gate joins the record before it if its register bit is below all of that one's.
         RegOp *prev = ops.size() > chunk_op ? &ops.back() : nullptr;
         const bool join = op.k == 1 && prev && prev->code && prev->code < 16u && (prev->code & ((2u << a) - 1u)) == 0;
-        if (join)
+        if (join) {
           prev->code |= 1u << a;
-        else
+          prev->lane |= o.lane;
+        } else {
           o.code = 1u << (op.k == 1 ? kRegG1 + a : op.k == 2 ? kRegG2 + 3 * a + (b > a ? b - 1 : b) : kRegSpecial);
+        }
         coef.insert(coef.end(), op.coef.begin(), op.coef.end());
         if (!join) ops.push_back(o);
         continue;

@@ -298,3 +298,38 @@ def test_register_runs_walk_several_tiles(sizes, dense3):
             assert torch.equal(torch.view_as_real(g).view(torch.int64), torch.view_as_real(w).view(torch.int64))
     finally:
         ops.tune_circuit(12)
+
+
+def _underflowing(rng, size):
+    """Nine in ten magnitudes near 1e-170, whose products underflow to zeros of
+    either sign; the others ordinary."""
+    x = (1e-170 * (1 + rng.random(size))) * rng.choice([-1.0, 1.0], size)
+    return np.where(rng.random(size) < 0.9, x, rng.standard_normal(size))
+
+
+@pytest.mark.parametrize("k", [1, 2, 3])
+@pytest.mark.parametrize("tb", [4, 9, 10, 11, 12])
+def test_signs_of_underflowing_products_bitexact(tb, k):
+    """A gate's sums start from +0, so none is -0 whatever its products underflow
+    to; diagonals after the gate and the stored state show the sign."""
+    n = 13
+    ops.tune_circuit(tb)
+    try:
+        for seed in range(4):
+            rng = np.random.default_rng(seed)
+            c = ops.Circuit(n)
+            for _ in range(seed + 1):
+                for _ in range(2):
+                    c.gate([int(v) for v in rng.choice(n, k, replace=False)],
+                           _underflowing(rng, 1 << 2 * k) + 1j * _underflowing(rng, 1 << 2 * k))
+                c.diag([int(v) for v in rng.choice(n, 2, replace=False)], rng.choice([1, -1, 1j, -1j], 4))
+            if seed == 3:
+                c.gate([0], [1, 0, 0, 1])
+            x = _underflowing(rng, 1 << n) + 1j * _underflowing(rng, 1 << n)
+            ref = oracle_run(c, x)
+            assert np.isfinite(ref.view(np.float64)).all() and (ref == 0).any()
+            s = dev(x)
+            c.run(s)
+            assert same_bits(host(s), ref), seed
+    finally:
+        ops.tune_circuit(12)
