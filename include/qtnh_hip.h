@@ -408,8 +408,8 @@ void qtnh_tune_split_tile(int shape);
 void qtnh_tune_stream(int max_blocks);
 /* Tile bits (3..13) of fused circuit runs, and how many of the lowest state
  * bits every tile keeps (0..8; 2^low x 16 bytes are contiguous in each tile
- * row).  Until set, by the state's size: 10 and 3 up to 18 qubits, 11 and 3 at
- * 19, 12 and 4 from 20.  Results do not depend on them. */
+ * row).  0 tile bits (the default): by the state's size, 10 and 3 up to 18
+ * qubits, 11 and 3 at 19, 12 and 4 from 20.  Results do not depend on them. */
 void qtnh_tune_circuit(int tile_bits, int low_bits);
 /* Kernel of fused runs: 2 (default) keeps 4 to 16 amplitudes per thread in
  * registers through the run (tiles of 4 to 12 bits), 1 pipelined (per-op LDS

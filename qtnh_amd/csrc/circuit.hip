@@ -1814,7 +1814,7 @@ using namespace qtnh_hip;
 extern "C" {
 
 void qtnh_tune_circuit(int tile_bits, int low_bits) {
-  g_tile_bits = std::max(3, std::min(tile_bits, kMaxTileBits));
+  g_tile_bits = tile_bits <= 0 ? 0 : std::max(3, std::min(tile_bits, kMaxTileBits));
   g_low_bits = std::max(0, std::min(low_bits, 8));
 }
 

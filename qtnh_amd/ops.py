@@ -290,9 +290,10 @@ def tune_stream(max_blocks=1 << 20):
     lib().qtnh_tune_stream(max_blocks)
 
 
-def tune_circuit(tile_bits=12, low_bits=4):
+def tune_circuit(tile_bits=0, low_bits=4):
     """Tile bits (3..13) of fused circuit runs and the lowest state bits every
-    tile keeps (0..8), process-wide; results do not depend on them."""
+    tile keeps (0..8), process-wide; without arguments both by the state's size,
+    as at the start.  Results do not depend on them."""
     lib().qtnh_tune_circuit(tile_bits, low_bits)
 
 

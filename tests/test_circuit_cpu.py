@@ -147,3 +147,22 @@ def test_invalid_sizes_rejected():
     c = ops.Circuit(3)
     with pytest.raises(ValueError):
         c.diag([0, 1], [1, 1, 1])
+
+
+def test_tile_setting_can_be_taken_back():
+    """Without arguments (and with 0 tile bits) the tiles go by the state's size again."""
+    def runs():
+        return [ops.Circuit(n).random(3, n).info()[2] for n in (9, 15, 18, 19, 20, 24)]
+
+    by_size = runs()
+    try:
+        for tiles, low in ((4, 1), (12, 4), (13, 0)):
+            ops.tune_circuit(tiles, low)
+            assert runs() != by_size
+            ops.tune_circuit()
+            assert runs() == by_size
+            ops.tune_circuit(tiles, low)
+            ops.tune_circuit(0, 0)
+            assert runs() == by_size
+    finally:
+        ops.tune_circuit()

@@ -333,3 +333,29 @@ def test_signs_of_underflowing_products_bitexact(tb, k):
             assert same_bits(host(s), ref), seed
     finally:
         ops.tune_circuit(12)
+
+
+@pytest.mark.parametrize("n", [9, 10, 11, 17, 18, 19, 20, 21])
+def test_default_tiles_bitexact(n):
+    """The tiles that the state's size picks, around the sizes where they change."""
+    c = _mixed_circuit(n, 60, False, n)
+    x = rnd_state(n, n)
+    ref = oracle_run(c, x)
+    s = dev(x)
+    c.run(s)
+    assert same_bits(host(s), ref)
+
+
+@pytest.mark.parametrize("tb", [0, 9, 11, 12])
+def test_batches_of_several_widths_bitexact(tb):
+    """Circuits of several widths in one launch, under the default and set tiles."""
+    sizes = [3, 4, 7, 10, 11, 13, 16]
+    cs = [_mixed_circuit(n, 60, n == 13, n) for n in sizes]
+    xs = [rnd_state(n, 50 + n) for n in sizes]
+    refs = [oracle_run(c, x) for c, x in zip(cs, xs)]
+    ops.tune_circuit(tb)
+    for first in (0, 1):  # with and without a width that has no register form
+        states = [dev(x) for x in xs[first:]]
+        ops.run_batch(cs[first:], states)
+        for n, s, ref in zip(sizes[first:], states, refs[first:]):
+            assert same_bits(host(s), ref), n
