@@ -361,12 +361,12 @@ qtnh_status qtnh_serve(qtnh_ctx_t ctx, int nq, const qtnh_query *queries, qtnh_q
  * run on this context (results do not depend on it).  Outputs may be NULL:
  * the chosen tile bits, low bits and the best time (ms). */
 qtnh_status qtnh_autotune_circuit(qtnh_ctx_t ctx, int n_qubits, int *tile_bits, int *low_bits, double *ms);
-/* Times this circuit's own fused runs at several tile shapes (12 bits down to
- * 7) on `scratch`, a device buffer of 2^n complex128 elements whose contents
+/* Times this circuit's own fused runs at several tile shapes (the one it takes
+ * without tuning, and 12 bits down to 7) on `scratch`, a device buffer of 2^n complex128 elements whose contents
  * it overwrites, and keeps the fastest for every later fused run of the
  * circuit (any state, any context; results do not depend on it).  Worth it
  * for circuits run many times: the best tile depends on the circuit (QFT-12:
- * 8 bits, 65 against 77 us per run), not only on its size.  Outputs may be
+ * 8 bits, 22.7 against 23.9 us per run), not only on its size.  Outputs may be
  * NULL: tile bits, low bits, time per run (us).  No reference counterpart. */
 qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, int *tile_bits, int *low_bits,
                               double *us);

@@ -2020,9 +2020,11 @@ qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, i
   if (st) return st;
   if (!c || !scratch) return set_error(ctx, QTNH_EINVAL, "circuit_tune: null argument");
   if (c->ops.empty()) return QTNH_OK;
-  // Candidates: the default tile, then smaller tiles (more workgroups per run;
-  // they win for small states whose runs would otherwise occupy a few CUs).
-  const int cand[][2] = {{12, 4}, {11, 4}, {10, 2}, {9, 2}, {8, 2}, {7, 2}};
+  // Candidates: the tile the circuit takes without tuning, then from the largest
+  // to smaller ones (more workgroups per run; they win for small states whose runs
+  // would otherwise occupy a few CUs).
+  int cand[][2] = {{0, 0}, {12, 4}, {11, 4}, {10, 2}, {9, 2}, {8, 2}, {7, 2}};
+  tile_shape(ctx, c->n, &cand[0][0], &cand[0][1]);
   const int reps = c->n >= 20 ? 2 : 10;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   st = check_hip(ctx, hipEventCreate(&e0), "circuit_tune event");
@@ -2031,7 +2033,7 @@ qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, i
   int btb = 0, blow = 0;
   for (const auto &cd : cand) {
     if (st) break;
-    if (cd[0] > std::max(c->n, 7)) continue;
+    if (&cd != cand && (cd[0] > std::max(c->n, 7) || (cd[0] == cand[0][0] && cd[1] == cand[0][1]))) continue;
     c->tuned_tb = cd[0];
     c->tuned_low = cd[1];
     st = run_fused(ctx, *c, (c128 *)scratch);  // compile + warm up

@@ -359,3 +359,18 @@ def test_batches_of_several_widths_bitexact(tb):
         ops.run_batch(cs[first:], states)
         for n, s, ref in zip(sizes[first:], states, refs[first:]):
             assert same_bits(host(s), ref), n
+
+
+def test_tuning_tries_the_untuned_tile():
+    """240 gates on 12 qubits above the lowest 4: 12-bit tiles that keep no low
+    bits take one run, the tuner's own shapes 30 or more."""
+    n = 20
+    c = ops.Circuit(n)
+    for i in range(240):
+        c.gate([n - 5 - i % 12], [0.6, 0.8, 0.8, -0.6])
+    ops.tune_circuit(12, 0)
+    assert c.info()[2] == 1
+    tb, low, us = c.tune()
+    assert (tb, low) == (12, 0) and us > 0
+    ops.tune_circuit()
+    assert c.info()[2] == 1  # the circuit keeps it
