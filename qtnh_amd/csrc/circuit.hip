@@ -22,6 +22,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <vector>
 
 #include "internal.hpp"
@@ -1020,21 +1021,12 @@ struct qtnh_circuit_s {
   std::vector<Op> ops;
   // Tile shape chosen for this circuit by qtnh_circuit_tune (0: the context's).
   int tuned_tb = 0, tuned_low = 0;
-  // Compiled form (device), rebuilt when ops or the tile size change.
-  int compiled_tb = -1;
-  int device = -1;
-  size_t compiled_ops = 0;
-  TileOp *d_ops = nullptr;
-  qtnh_hip::double2_t *d_coef = nullptr;
   struct Run {
     uint32_t begin, end;
     std::vector<int> tbits;  // ascending state bits
   };
-  std::vector<Run> runs;
-  std::vector<TileOp> tops;  // host copy of the compiled ops
-  // Register forms of the runs, by register bits (null: not built).
+  // Register form of the runs with some number of register bits (ops null: not built).
   struct RegForm {
-    void *dev = nullptr;  // ops, chunks, coefficients
     const RegOp *ops = nullptr;
     const RegChunk *chunks = nullptr;
     const qtnh_hip::double2_t *coef = nullptr;
@@ -1043,22 +1035,32 @@ struct qtnh_circuit_s {
     };
     std::vector<Run> runs;
   };
-  RegForm forms[qtnh_hip::kMaxRegBits + 1];
-  bool has3 = false;  // a dense 3-qubit gate among the compiled ops
-  // Uploaded run descriptors of fused runs, per state buffer: a repeated run
-  // on the same state launches kernels only (no copy), so it can be captured
-  // into a graph.  Cleared when the circuit is recompiled.
-  struct DescCache {
-    RunDesc *d = nullptr;
-    std::vector<RunDesc> h;
-    std::vector<size_t> starts;
+  // The ops compiled for one tile shape on one device.
+  struct Compiled {
+    int n = 0;  // qubits
+    int tb = 0, low = 0, device = -1;
+    void *dev = nullptr;  // everything below that is on the device
+    const TileOp *ops = nullptr;
+    const qtnh_hip::double2_t *coef = nullptr;
+    std::vector<Run> runs;
+    std::vector<TileOp> tops;  // host copy of the compiled ops
+    RegForm forms[qtnh_hip::kMaxRegBits + 1];  // by register bits
+    bool has3 = false;  // a dense 3-qubit gate among the ops
+    // Uploaded run descriptors of fused runs, per state buffer: a repeated run
+    // on the same state launches kernels only (no copy), so it can be captured
+    // into a graph.
+    struct DescCache {
+      RunDesc *d = nullptr;
+      std::vector<RunDesc> h;
+      std::vector<size_t> starts;
+    };
+    std::map<const void *, DescCache> desc_cache;
   };
-  std::map<const void *, DescCache> desc_cache;
-  // Device memory of earlier compiled forms of the same ops (another tile
-  // shape or device).  A graph captured from an earlier fused run may still
-  // read it, so it is freed only when ops are appended or the circuit is
-  // destroyed.
-  std::vector<void *> retired;
+  // One for each tile shape and device the circuit has run with since ops were
+  // last appended.  A graph captured from a fused run reads its memory, so all of
+  // them are kept until ops are appended or the circuit is destroyed.
+  std::vector<std::unique_ptr<Compiled>> compiled;
+  size_t compiled_ops = 0;
 };
 
 namespace qtnh_hip {
@@ -1096,8 +1098,8 @@ uint64_t mask_of(const qtnh_circuit_s &c, const qtnh_circuit_s::Op &op) {
 // tb.  Runs are contiguous in op order, so every amplitude sees the ops in
 // program order; with that constraint the greedy (longest feasible run first)
 // gives the fewest runs.
-void plan_runs(qtnh_circuit_s &c, int tb, int low_bits) {
-  c.runs.clear();
+std::vector<qtnh_circuit_s::Run> plan_runs(const qtnh_circuit_s &c, int tb, int low_bits) {
+  std::vector<qtnh_circuit_s::Run> runs;
   const int tbe = std::min(tb, c.n);
   const uint64_t low = (1ull << std::min(std::min(low_bits, tbe - 3 > 0 ? tbe - 3 : 0), c.n)) - 1;
   uint64_t cur = low;
@@ -1111,7 +1113,7 @@ void plan_runs(qtnh_circuit_s &c, int tb, int low_bits) {
     r.end = end;
     for (int b = 0; b < c.n; ++b)
       if ((m >> b) & 1) r.tbits.push_back(b);
-    c.runs.push_back(r);
+    runs.push_back(r);
   };
   for (uint32_t i = 0; i < c.ops.size(); ++i) {
     const uint64_t m = mask_of(c, c.ops[i]);
@@ -1123,30 +1125,19 @@ void plan_runs(qtnh_circuit_s &c, int tb, int low_bits) {
     cur |= m;
   }
   close((uint32_t)c.ops.size());
+  return runs;
 }
 
-// Detaches the current compiled form; its device memory moves to `retired`.
-void retire_compiled(qtnh_circuit_s &c) {
-  for (auto &kv : c.desc_cache)
-    if (kv.second.d) c.retired.push_back(kv.second.d);
-  c.desc_cache.clear();
-  for (void *p : {(void *)c.d_ops, (void *)c.d_coef})
-    if (p) c.retired.push_back(p);
-  for (auto &f : c.forms) {
-    if (f.dev) c.retired.push_back(f.dev);
-    f = qtnh_circuit_s::RegForm{};
-  }
-  c.d_ops = nullptr;
-  c.d_coef = nullptr;
-  c.compiled_tb = -1;
-}
+using Compiled = qtnh_circuit_s::Compiled;
 
-// Frees the current and every retired compiled form (the caller has drained
-// the streams that used them).
+// Frees every compiled form (the caller has drained the streams that used them).
 void free_compiled(qtnh_circuit_s &c) {
-  retire_compiled(c);
-  for (void *p : c.retired) (void)hipFree(p);
-  c.retired.clear();
+  for (const auto &k : c.compiled) {
+    if (k->dev) (void)hipFree(k->dev);
+    for (auto &d : k->desc_cache)
+      if (d.second.d) (void)hipFree(d.second.d);
+  }
+  c.compiled.clear();
 }
 
 // Register bits for a launch of runs of tb-bit tiles: 64 to 256 threads per
@@ -1159,9 +1150,9 @@ int reg_bits(int tb, bool has3) { return std::max(has3 ? 3 : kMinRegBits, std::m
 
 // Register forms a circuit with tb-bit tiles needs: the one for its own runs,
 // and the widest (launches that mix circuits of several widths).
-bool wants_form(const qtnh_circuit_s &c, int tb, int R) {
+bool wants_form(int tb, bool has3, int R) {
   if (tb < kMaxRegBits || tb > 12) return false;
-  return R == kMaxRegBits || R == reg_bits(tb, c.has3);
+  return R == kMaxRegBits || R == reg_bits(tb, has3);
 }
 
 // The register form (R register bits) of run r: appends its ops, coefficients
@@ -1339,34 +1330,17 @@ void plan_reg_run(const qtnh_circuit_s &c, const qtnh_circuit_s::Run &r, int R, 
   fr->where_out = where(map);
 }
 
-// Builds and uploads the register form of R bits of the planned runs.
-qtnh_status build_form(qtnh_ctx_t ctx, qtnh_circuit_s &c, int R) {
-  std::vector<RegOp> ops;
-  std::vector<RegChunk> chunks;
-  std::vector<double> coef;
-  auto &f = c.forms[R];
-  for (const auto &r : c.runs) {
-    qtnh_circuit_s::RegForm::Run fr;
-    fr.chunk_begin = (uint32_t)chunks.size();
-    plan_reg_run(c, r, R, ops, coef, chunks, &fr);
-    fr.chunk_end = (uint32_t)chunks.size();
-    f.runs.push_back(fr);
+// Device tables gathered on the host, for one allocation and one copy.
+struct Tables {
+  std::vector<char> host;
+  template <typename T>
+  size_t add(const std::vector<T> &v) {
+    const size_t at = (host.size() + 255) & ~(size_t)255, bytes = v.size() * sizeof(T);
+    host.resize(at + bytes);
+    if (bytes) memcpy(host.data() + at, v.data(), bytes);
+    return at;
   }
-  auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t ob = pad(ops.size() * sizeof(RegOp)), cb = pad(chunks.size() * sizeof(RegChunk)),
-               fb = coef.size() * sizeof(double);
-  std::vector<char> host(ob + cb + fb + 16);
-  if (!ops.empty()) memcpy(host.data(), ops.data(), ops.size() * sizeof(RegOp));
-  if (!chunks.empty()) memcpy(host.data() + ob, chunks.data(), chunks.size() * sizeof(RegChunk));
-  if (!coef.empty()) memcpy(host.data() + ob + cb, coef.data(), fb);
-  qtnh_status st = check_hip(ctx, hipMalloc(&f.dev, host.size()), "circuit form alloc");
-  if (st) return st;
-  f.ops = (const RegOp *)f.dev;
-  f.chunks = (const RegChunk *)((char *)f.dev + ob);
-  f.coef = (const double2_t *)((char *)f.dev + ob + cb);
-  return check_hip(ctx, hipMemcpyAsync(f.dev, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream),
-                   "circuit form upload");
-}
+};
 
 // Tile shape for an n-qubit circuit: the autotuned one of this context, else the process default.
 void tile_shape(qtnh_ctx_t ctx, int n, int *tb, int *low) {
@@ -1377,31 +1351,35 @@ void tile_shape(qtnh_ctx_t ctx, int n, int *tb, int *low) {
   *low = ctx->circ_low[n];
 }
 
-qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
+// The circuit compiled for its tile shape on the context's device.
+qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c, Compiled **out) {
   int tb, low;
   tile_shape(ctx, c.n, &tb, &low);
   if (c.tuned_tb > 0) {
     tb = c.tuned_tb;
     low = c.tuned_low;
   }
-  if (c.compiled_tb == tb * 16 + low && c.device == ctx->device && c.compiled_ops == c.ops.size()) return QTNH_OK;
-  if (c.d_ops || c.d_coef) {
-    if (c.compiled_ops == c.ops.size()) {
-      // Same ops, another tile shape or device: graphs captured from the
-      // earlier form stay valid, so its memory is kept.
-      retire_compiled(c);
-    } else {
-      qtnh_status st = check_hip(ctx, hipStreamSynchronize(ctx->stream), "circuit recompile sync");
-      if (st) return st;
-      free_compiled(c);
-    }
+  if (c.compiled_ops != c.ops.size() && !c.compiled.empty()) {
+    qtnh_status st = check_hip(ctx, hipStreamSynchronize(ctx->stream), "circuit recompile sync");
+    if (st) return st;
+    free_compiled(c);
   }
-  plan_runs(c, tb, low);
-  c.has3 = false;
-  for (const auto &op : c.ops) c.has3 = c.has3 || (op.kind == 0 && op.k == 3);
+  c.compiled_ops = c.ops.size();
+  for (const auto &k : c.compiled)
+    if (k->tb == tb && k->low == low && k->device == ctx->device) {
+      *out = k.get();
+      return QTNH_OK;
+    }
+  std::unique_ptr<Compiled> k(new Compiled);
+  k->n = c.n;
+  k->tb = tb;
+  k->low = low;
+  k->device = ctx->device;
+  k->runs = plan_runs(c, tb, low);
+  for (const auto &op : c.ops) k->has3 = k->has3 || (op.kind == 0 && op.k == 3);
   std::vector<TileOp> tops(std::max<size_t>(c.ops.size(), 1));
   std::vector<double> coef;
-  for (const auto &r : c.runs) {
+  for (const auto &r : k->runs) {
     for (uint32_t i = r.begin; i < r.end; ++i) {
       const auto &op = c.ops[i];
       TileOp t;
@@ -1447,41 +1425,52 @@ qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c) {
     }
   }
   if (coef.empty()) coef.assign(2, 0.0);
-  qtnh_status st = check_hip(ctx, hipMalloc((void **)&c.d_ops, tops.size() * sizeof(TileOp)), "circuit alloc");
-  if (!st) st = check_hip(ctx, hipMalloc((void **)&c.d_coef, coef.size() * sizeof(double)), "circuit alloc");
-  if (!st)
-    st = check_hip(ctx, hipMemcpyAsync(c.d_ops, tops.data(), tops.size() * sizeof(TileOp), hipMemcpyHostToDevice,
-                                       ctx->stream),
-                   "circuit upload");
-  if (!st)
-    st = check_hip(ctx, hipMemcpyAsync(c.d_coef, coef.data(), coef.size() * sizeof(double), hipMemcpyHostToDevice,
-                                       ctx->stream),
-                   "circuit upload");
-  for (int R = kMinRegBits; R <= kMaxRegBits && !st; ++R)
-    if (wants_form(c, std::min(tb, c.n), R)) st = build_form(ctx, c, R);
-  if (st) {
-    // Only this attempt's buffers: no launch has used them (retired forms stay).
-    (void)hipStreamSynchronize(ctx->stream);
-    for (void *p : {(void *)c.d_ops, (void *)c.d_coef})
-      if (p) (void)hipFree(p);
-    for (auto &f : c.forms) {
-      if (f.dev) (void)hipFree(f.dev);
-      f = qtnh_circuit_s::RegForm{};
+  Tables tables;
+  const size_t ops_at = tables.add(tops), coef_at = tables.add(coef);
+  size_t form_at[kMaxRegBits + 1][3] = {};
+  for (int R = kMinRegBits; R <= kMaxRegBits; ++R) {
+    if (!wants_form(std::min(tb, c.n), k->has3, R)) continue;
+    std::vector<RegOp> rops;
+    std::vector<RegChunk> chunks;
+    std::vector<double> rcoef;
+    for (const auto &r : k->runs) {
+      qtnh_circuit_s::RegForm::Run fr;
+      fr.chunk_begin = (uint32_t)chunks.size();
+      plan_reg_run(c, r, R, rops, rcoef, chunks, &fr);
+      fr.chunk_end = (uint32_t)chunks.size();
+      k->forms[R].runs.push_back(fr);
     }
-    c.d_ops = nullptr;
-    c.d_coef = nullptr;
-    c.compiled_tb = -1;
+    form_at[R][0] = tables.add(rops);
+    form_at[R][1] = tables.add(chunks);
+    form_at[R][2] = tables.add(rcoef);
+  }
+  tables.host.resize(tables.host.size() + 16);  // (an address for empty tables)
+  qtnh_status st = check_hip(ctx, hipMalloc(&k->dev, tables.host.size()), "circuit alloc");
+  if (st) return st;
+  st = check_hip(ctx, hipMemcpyAsync(k->dev, tables.host.data(), tables.host.size(), hipMemcpyHostToDevice, ctx->stream),
+                 "circuit upload");
+  if (st) {
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(k->dev);
     return st;
   }
-  c.tops = tops;
-  c.compiled_tb = tb * 16 + low;
-  c.device = ctx->device;
-  c.compiled_ops = c.ops.size();
+  const char *dev = (const char *)k->dev;
+  k->ops = (const TileOp *)(dev + ops_at);
+  k->coef = (const double2_t *)(dev + coef_at);
+  for (int R = kMinRegBits; R <= kMaxRegBits; ++R) {
+    if (!wants_form(std::min(tb, c.n), k->has3, R)) continue;
+    k->forms[R].ops = (const RegOp *)(dev + form_at[R][0]);
+    k->forms[R].chunks = (const RegChunk *)(dev + form_at[R][1]);
+    k->forms[R].coef = (const double2_t *)(dev + form_at[R][2]);
+  }
+  k->tops = std::move(tops);
+  c.compiled.push_back(std::move(k));
+  *out = c.compiled.back().get();
   return QTNH_OK;
 }
 
 // Descriptor of run ri on psi, with its register form of R bits (0: none).
-RunDesc make_desc(const qtnh_circuit_s &c, size_t ri, c128 *psi, uint64_t first, int R) {
+RunDesc make_desc(const Compiled &c, size_t ri, c128 *psi, uint64_t first, int R) {
   const qtnh_circuit_s::Run &r = c.runs[ri];
   RunDesc d;
   memset(&d, 0, sizeof(d));
@@ -1497,8 +1486,8 @@ RunDesc make_desc(const qtnh_circuit_s &c, size_t ri, c128 *psi, uint64_t first,
     d.where_out = f.runs[ri].where_out;
     d.rbits = R;
   }
-  d.ops = c.d_ops;
-  d.coef = c.d_coef;
+  d.ops = c.ops;
+  d.coef = c.coef;
   d.psi = (double2_t *)psi;
   d.first = first;
   d.op_begin = r.begin;
@@ -1518,7 +1507,7 @@ uint64_t desc_tiles(const RunDesc &d) { return 1ull << d.n_outer; }
 
 // Run ri of circuit c on psi, one of a launch's runs.
 struct RunRef {
-  const qtnh_circuit_s *c;
+  const Compiled *c;
   size_t ri;
   c128 *psi;
 };
@@ -1536,12 +1525,12 @@ void add_group(const std::vector<RunRef> &refs, std::vector<RunDesc> &descs, std
   }
   int R = reg_bits(tb_max, has3);
   for (const RunRef &r : refs)
-    if (!r.c->forms[R].dev) {
+    if (!r.c->forms[R].ops) {
       R = kMaxRegBits;
       break;
     }
   for (const RunRef &r : refs)
-    if (!r.c->forms[R].dev) {
+    if (!r.c->forms[R].ops) {
       R = 0;
       break;
     }
@@ -1645,10 +1634,11 @@ qtnh_status launch_run_groups(qtnh_ctx_t ctx, const std::vector<RunDesc> &descs,
 constexpr size_t kDescCacheMax = 64;  // states per circuit with cached descriptors
 
 qtnh_status run_fused(qtnh_ctx_t ctx, qtnh_circuit_s &c, c128 *psi) {
-  qtnh_status st = compile(ctx, c);
+  Compiled *k = nullptr;
+  qtnh_status st = compile(ctx, c, &k);
   if (st) return st;
-  auto hit = c.desc_cache.find(psi);
-  if (hit != c.desc_cache.end()) return launch_groups(ctx, hit->second.d, hit->second.h, hit->second.starts);
+  auto hit = k->desc_cache.find(psi);
+  if (hit != k->desc_cache.end()) return launch_groups(ctx, hit->second.d, hit->second.h, hit->second.starts);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
     (void)hipGetLastError();
@@ -1658,23 +1648,21 @@ qtnh_status run_fused(qtnh_ctx_t ctx, qtnh_circuit_s &c, c128 *psi) {
     return set_error(ctx, QTNH_EUNSUPPORTED,
                      "circuit_run: first fused run of this circuit on this state during graph capture "
                      "(run it once on the state before capturing)");
-  qtnh_circuit_s::DescCache dc;
-  for (size_t ri = 0; ri < c.runs.size(); ++ri) {
-    add_group({RunRef{&c, ri, psi}}, dc.h, dc.starts);
-  }
+  Compiled::DescCache dc;
+  for (size_t ri = 0; ri < k->runs.size(); ++ri) add_group({RunRef{k, ri, psi}}, dc.h, dc.starts);
   dc.starts.push_back(dc.h.size());
   if (dc.h.empty()) return QTNH_OK;
-  if (c.desc_cache.size() >= kDescCacheMax) return launch_run_groups(ctx, dc.h, dc.starts);
+  if (k->desc_cache.size() >= kDescCacheMax) return launch_run_groups(ctx, dc.h, dc.starts);
   const uint64_t bytes = dc.h.size() * sizeof(RunDesc);
   st = check_hip(ctx, hipMalloc((void **)&dc.d, bytes), "run descriptor alloc");
   if (st) return st;
-  auto &e = c.desc_cache[psi];
+  auto &e = k->desc_cache[psi];
   e = std::move(dc);
   st = check_hip(ctx, hipMemcpyAsync(e.d, e.h.data(), bytes, hipMemcpyHostToDevice, ctx->stream),
                  "run descriptor upload");
   if (st) {
     (void)hipFree(e.d);
-    c.desc_cache.erase(psi);
+    k->desc_cache.erase(psi);
     return st;
   }
   return launch_groups(ctx, e.d, e.h, e.starts);
@@ -1779,19 +1767,21 @@ bool qubits_valid(int n, int k, const uint16_t *q) {
 namespace qtnh_hip {
 
 qtnh_status circuit_run_count(qtnh_ctx_t ctx, qtnh_circuit_t c, int *nruns) {
-  qtnh_status st = compile(ctx, *c);
+  Compiled *k = nullptr;
+  qtnh_status st = compile(ctx, *c, &k);
   if (st) return st;
-  *nruns = (int)c->runs.size();
+  *nruns = (int)k->runs.size();
   return QTNH_OK;
 }
 
 qtnh_status circuit_advance(qtnh_ctx_t ctx, int count, const qtnh_circuit_t *cs, void *const *states,
                             const int *first_run, const int *nrun) {
   int kmax = 0;
+  std::vector<Compiled *> ks(count);
   for (int i = 0; i < count; ++i) {
-    qtnh_status st = compile(ctx, *cs[i]);
+    qtnh_status st = compile(ctx, *cs[i], &ks[i]);
     if (st) return st;
-    if (first_run[i] < 0 || nrun[i] < 0 || (size_t)first_run[i] + (size_t)nrun[i] > cs[i]->runs.size())
+    if (first_run[i] < 0 || nrun[i] < 0 || (size_t)first_run[i] + (size_t)nrun[i] > ks[i]->runs.size())
       return set_error(ctx, QTNH_EINVAL, "circuit advance: runs out of range");
     kmax = std::max(kmax, nrun[i]);
   }
@@ -1800,7 +1790,7 @@ qtnh_status circuit_advance(qtnh_ctx_t ctx, int count, const qtnh_circuit_t *cs,
   for (int k = 0; k < kmax; ++k) {
     std::vector<RunRef> refs;
     for (int i = 0; i < count; ++i)
-      if (k < nrun[i]) refs.push_back(RunRef{cs[i], (size_t)(first_run[i] + k), (c128 *)states[i]});
+      if (k < nrun[i]) refs.push_back(RunRef{ks[i], (size_t)(first_run[i] + k), (c128 *)states[i]});
     add_group(refs, descs, starts);
   }
   starts.push_back(descs.size());
@@ -1833,8 +1823,8 @@ qtnh_status qtnh_circuit_create(int n_qubits, qtnh_circuit_t *out) {
 
 qtnh_status qtnh_circuit_destroy(qtnh_circuit_t c) {
   if (!c) return QTNH_EINVAL;
-  if (c->device >= 0) {
-    (void)hipSetDevice(c->device);
+  for (const auto &k : c->compiled) {
+    (void)hipSetDevice(k->device);
     (void)hipDeviceSynchronize();
   }
   free_compiled(*c);
@@ -1956,13 +1946,9 @@ qtnh_status qtnh_circuit_info(qtnh_circuit_t c, int *n_qubits, uint64_t *n_ops, 
   if (n_qubits) *n_qubits = c->n;
   if (n_ops) *n_ops = c->ops.size();
   if (n_runs) {
-    qtnh_circuit_s tmp;
-    tmp.n = c->n;
-    tmp.ops = c->ops;
     int tb = c->tuned_tb, low = c->tuned_low;
     if (tb <= 0) default_tile(c->n, &tb, &low);
-    plan_runs(tmp, tb, low);
-    *n_runs = tmp.runs.size();
+    *n_runs = plan_runs(*c, tb, low).size();
   }
   return QTNH_OK;
 }
@@ -1992,13 +1978,14 @@ qtnh_status qtnh_circuit_run_batch(qtnh_ctx_t ctx, int count, const qtnh_circuit
   if (st) return st;
   if (count < 0 || (count > 0 && (!cs || !states))) return set_error(ctx, QTNH_EINVAL, "run_batch: bad arguments");
   size_t steps = 0;
+  std::vector<Compiled *> ks(count);
   for (int i = 0; i < count; ++i) {
     if (!cs[i] || !states[i]) return set_error(ctx, QTNH_EINVAL, "run_batch: null circuit or state %d", i);
     for (int j = 0; j < i; ++j)
       if (states[j] == states[i]) return set_error(ctx, QTNH_EINVAL, "run_batch: state %d repeats state %d", i, j);
-    st = compile(ctx, *cs[i]);
+    st = compile(ctx, *cs[i], &ks[i]);
     if (st) return st;
-    steps = std::max(steps, cs[i]->runs.size());
+    steps = std::max(steps, ks[i]->runs.size());
   }
   // Step s runs the s-th run of every circuit that has one, in one launch.
   std::vector<RunDesc> descs;
@@ -2006,7 +1993,7 @@ qtnh_status qtnh_circuit_run_batch(qtnh_ctx_t ctx, int count, const qtnh_circuit
   for (size_t s = 0; s < steps; ++s) {
     std::vector<RunRef> refs;
     for (int i = 0; i < count; ++i)
-      if (s < cs[i]->runs.size()) refs.push_back(RunRef{cs[i], s, (c128 *)states[i]});
+      if (s < ks[i]->runs.size()) refs.push_back(RunRef{ks[i], s, (c128 *)states[i]});
     add_group(refs, descs, starts);
   }
   starts.push_back(descs.size());
@@ -2055,7 +2042,8 @@ qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, i
   c->tuned_low = st ? 0 : blow;
   if (st) return st;
   // Leave the winning shape compiled, so the next run launches without a recompile.
-  st = compile(ctx, *c);
+  Compiled *k = nullptr;
+  st = compile(ctx, *c, &k);
   if (st) return st;
   if (tile_bits) *tile_bits = btb;
   if (low_bits) *low_bits = blow;

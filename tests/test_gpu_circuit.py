@@ -374,3 +374,20 @@ def test_tuning_tries_the_untuned_tile():
     assert (tb, low) == (12, 0) and us > 0
     ops.tune_circuit()
     assert c.info()[2] == 1  # the circuit keeps it
+
+
+def test_ops_appended_after_runs_under_several_tiles():
+    """A circuit keeps what it compiled for each tile shape; appended ops reach
+    every shape, on states seen before and new ones."""
+    n = 13
+    c = _mixed_circuit(n, 30, True, 1)
+    x = rnd_state(n, 3)
+    s = dev(x)
+    for more in range(3):
+        for tb in (12, 8, 0, 12):
+            ops.tune_circuit(tb)
+            for t in (s, dev(x)):
+                x0 = host(t)
+                c.run(t)
+                assert same_bits(host(t), oracle_run(c, x0)), (more, tb)
+        c.gate([more], [0.6, 0.8, 0.8, -0.6]).diag([12, more], [1, 1j, -1, -1j])
