@@ -1072,15 +1072,22 @@ int g_tile_bits = 0;  // 0: by the state's size (default_tile)
 int g_circuit_mode = 2;
 int g_low_bits = 4;  // lowest state bits in every tile: 2^4 x 16 B = 256 B contiguous rows
 
-// Tile bits and low bits of an n-qubit circuit where nothing else is set.
-// 12-bit tiles make the fewest passes, which large states need; a state of
-// fewer tiles than compute units is bound by one tile's latency and takes
-// smaller tiles, more passes over more workgroups (12 / 10-bit tiles: QFT-12
-// 35 / 24 us, random circuits of 16 and 18 qubits 168 / 124 and 163 / 126; 11
-// bits at 19 qubits 262 / 228; at 20 qubits 372 us with 12 bits, 431 with 11).
-void default_tile(int n, int *tb, int *low) {
-  *tb = g_tile_bits ? g_tile_bits : n <= 18 ? 10 : n == 19 ? 11 : 12;
-  *low = g_tile_bits ? g_low_bits : n <= 19 ? 3 : 4;
+// Tile bits and low bits of an n-qubit circuit in launches over about 2^bits
+// amplitudes (its own state's and the others' of a batch), where nothing else is
+// set.  12-bit tiles make the fewest passes, which large states need; a launch of
+// fewer tiles than compute units is bound by one tile's latency and takes smaller
+// tiles, more passes over more workgroups (12 / 10-bit tiles: QFT-12 35 / 24 us,
+// random circuits of 16 and 18 qubits 168 / 124 and 163 / 126; 11 bits at 19
+// qubits 262 / 228; at 20 qubits 372 us with 12 bits, 431 with 11).  So do
+// batches: depth-4 random circuits, 10 / 11 / 12 bits, 8 of 15 qubits 79 / 84 / 102
+// us, 16 of them 107 / 98 / 113, 16 of 16 qubits 179 / 158 / 135; of 19 qubits 11
+// bits are the best for two, too (175, and 194 with 12).  States that one tile
+// holds need a single pass, which eight of them make faster than two over smaller
+// tiles (32 of 12 qubits 84 / 87 / 60).
+void default_tile(int n, int bits, int *tb, int *low) {
+  const bool large = bits >= (n == 19 ? 21 : 20) || (n <= 12 && bits >= n + 3);
+  *tb = g_tile_bits ? g_tile_bits : large ? 12 : bits >= 19 ? 11 : 10;
+  *low = g_tile_bits ? g_low_bits : large ? 4 : 3;
 }
 
 // State bits an op needs inside the tile: all of a gate's; none of a
@@ -1342,23 +1349,29 @@ struct Tables {
   }
 };
 
-// Tile shape for an n-qubit circuit: the autotuned one of this context, else the process default.
-void tile_shape(qtnh_ctx_t ctx, int n, int *tb, int *low) {
+// Tile shape for an n-qubit circuit in launches over about 2^bits amplitudes: the
+// autotuned one of this context, else the process default.
+void tile_shape(qtnh_ctx_t ctx, int n, int bits, int *tb, int *low) {
   const bool tuned = n < 64 && ctx->circ_tb[n] > 0;
-  default_tile(n, tb, low);
+  default_tile(n, bits, tb, low);
   if (!tuned) return;
   *tb = ctx->circ_tb[n];
   *low = ctx->circ_low[n];
 }
 
-// The circuit compiled for its tile shape on the context's device.
-qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c, Compiled **out) {
+// ... and for a circuit: its own tuned one first.
+void tile_shape(qtnh_ctx_t ctx, const qtnh_circuit_s &c, int bits, int *tb, int *low) {
+  tile_shape(ctx, c.n, bits, tb, low);
+  if (c.tuned_tb <= 0) return;
+  *tb = c.tuned_tb;
+  *low = c.tuned_low;
+}
+
+// The circuit compiled on the context's device, for its tile shape in launches
+// over about 2^bits amplitudes.
+qtnh_status compile(qtnh_ctx_t ctx, qtnh_circuit_s &c, int bits, Compiled **out) {
   int tb, low;
-  tile_shape(ctx, c.n, &tb, &low);
-  if (c.tuned_tb > 0) {
-    tb = c.tuned_tb;
-    low = c.tuned_low;
-  }
+  tile_shape(ctx, c, bits, &tb, &low);
   if (c.compiled_ops != c.ops.size() && !c.compiled.empty()) {
     qtnh_status st = check_hip(ctx, hipStreamSynchronize(ctx->stream), "circuit recompile sync");
     if (st) return st;
@@ -1635,7 +1648,7 @@ constexpr size_t kDescCacheMax = 64;  // states per circuit with cached descript
 
 qtnh_status run_fused(qtnh_ctx_t ctx, qtnh_circuit_s &c, c128 *psi) {
   Compiled *k = nullptr;
-  qtnh_status st = compile(ctx, c, &k);
+  qtnh_status st = compile(ctx, c, c.n, &k);
   if (st) return st;
   auto hit = k->desc_cache.find(psi);
   if (hit != k->desc_cache.end()) return launch_groups(ctx, hit->second.d, hit->second.h, hit->second.starts);
@@ -1766,20 +1779,18 @@ bool qubits_valid(int n, int k, const uint16_t *q) {
 
 namespace qtnh_hip {
 
-qtnh_status circuit_run_count(qtnh_ctx_t ctx, qtnh_circuit_t c, int *nruns) {
-  Compiled *k = nullptr;
-  qtnh_status st = compile(ctx, *c, &k);
-  if (st) return st;
-  *nruns = (int)k->runs.size();
-  return QTNH_OK;
+int circuit_run_count(qtnh_ctx_t ctx, qtnh_circuit_t c, int bits) {
+  int tb, low;
+  tile_shape(ctx, *c, bits, &tb, &low);
+  return (int)plan_runs(*c, tb, low).size();
 }
 
 qtnh_status circuit_advance(qtnh_ctx_t ctx, int count, const qtnh_circuit_t *cs, void *const *states,
-                            const int *first_run, const int *nrun) {
+                            const int *first_run, const int *nrun, int bits) {
   int kmax = 0;
   std::vector<Compiled *> ks(count);
   for (int i = 0; i < count; ++i) {
-    qtnh_status st = compile(ctx, *cs[i], &ks[i]);
+    qtnh_status st = compile(ctx, *cs[i], bits, &ks[i]);
     if (st) return st;
     if (first_run[i] < 0 || nrun[i] < 0 || (size_t)first_run[i] + (size_t)nrun[i] > ks[i]->runs.size())
       return set_error(ctx, QTNH_EINVAL, "circuit advance: runs out of range");
@@ -1947,7 +1958,7 @@ qtnh_status qtnh_circuit_info(qtnh_circuit_t c, int *n_qubits, uint64_t *n_ops, 
   if (n_ops) *n_ops = c->ops.size();
   if (n_runs) {
     int tb = c->tuned_tb, low = c->tuned_low;
-    if (tb <= 0) default_tile(c->n, &tb, &low);
+    if (tb <= 0) default_tile(c->n, c->n, &tb, &low);
     *n_runs = plan_runs(*c, tb, low).size();
   }
   return QTNH_OK;
@@ -1978,12 +1989,16 @@ qtnh_status qtnh_circuit_run_batch(qtnh_ctx_t ctx, int count, const qtnh_circuit
   if (st) return st;
   if (count < 0 || (count > 0 && (!cs || !states))) return set_error(ctx, QTNH_EINVAL, "run_batch: bad arguments");
   size_t steps = 0;
-  std::vector<Compiled *> ks(count);
+  uint64_t amplitudes = 0;
   for (int i = 0; i < count; ++i) {
     if (!cs[i] || !states[i]) return set_error(ctx, QTNH_EINVAL, "run_batch: null circuit or state %d", i);
     for (int j = 0; j < i; ++j)
       if (states[j] == states[i]) return set_error(ctx, QTNH_EINVAL, "run_batch: state %d repeats state %d", i, j);
-    st = compile(ctx, *cs[i], &ks[i]);
+    amplitudes += 1ull << cs[i]->n;
+  }
+  std::vector<Compiled *> ks(count);
+  for (int i = 0; i < count; ++i) {
+    st = compile(ctx, *cs[i], floor_log2(amplitudes), &ks[i]);
     if (st) return st;
     steps = std::max(steps, ks[i]->runs.size());
   }
@@ -2011,7 +2026,7 @@ qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, i
   // to smaller ones (more workgroups per run; they win for small states whose runs
   // would otherwise occupy a few CUs).
   int cand[][2] = {{0, 0}, {12, 4}, {11, 4}, {10, 2}, {9, 2}, {8, 2}, {7, 2}};
-  tile_shape(ctx, c->n, &cand[0][0], &cand[0][1]);
+  tile_shape(ctx, c->n, c->n, &cand[0][0], &cand[0][1]);
   const int reps = c->n >= 20 ? 2 : 10;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   st = check_hip(ctx, hipEventCreate(&e0), "circuit_tune event");
@@ -2043,7 +2058,7 @@ qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, i
   if (st) return st;
   // Leave the winning shape compiled, so the next run launches without a recompile.
   Compiled *k = nullptr;
-  st = compile(ctx, *c, &k);
+  st = compile(ctx, *c, c->n, &k);
   if (st) return st;
   if (tile_bits) *tile_bits = btb;
   if (low_bits) *low_bits = blow;
@@ -2070,7 +2085,7 @@ qtnh_status qtnh_autotune_circuit(qtnh_ctx_t ctx, int n_qubits, int *tile_bits, 
   if (!st) st = check_hip(ctx, hipEventCreate(&e1), "autotune event");
   double best = 1e30;
   int btb, blow;
-  default_tile(np, &btb, &blow);
+  default_tile(np, np, &btb, &blow);
   for (const auto &cd : cand) {
     if (st) break;
     if (cd[0] > std::max(np, 10)) continue;

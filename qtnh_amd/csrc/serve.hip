@@ -181,9 +181,9 @@ qtnh_status plan_amplitude(qtnh_ctx_t ctx, const qtnh_query &q, qtnh_circuit_t c
   uint64_t steps = 0, dev = 0;
   double flops = 0, nbytes = 0;
   if (!st) st = qtnh_net_info(h.net, nullptr, &steps, nullptr, &flops, &nbytes, &dev);
-  int nruns = 0;
-  if (!st && !all) st = circuit_run_count(ctx, c, &nruns);
   if (st) return st;
+  // (The passes of the largest tiles, which the estimate's time per run goes by.)
+  const int nruns = all ? 0 : circuit_run_count(ctx, c, 62);
   *use_net = all || network_route_s((double)steps, flops, nbytes, split) < state_route_s(n, nruns);
   *bytes = dev;
   return QTNH_OK;
@@ -346,7 +346,6 @@ extern "C" qtnh_status qtnh_serve(qtnh_ctx_t ctx, int nq, const qtnh_query *quer
       if (st) return st;
       f.h = ch;
       st = init_state(ctx, f.buf, key.n);
-      if (!st) st = circuit_run_count(ctx, f.h->c, &f.nruns);
       if (st) {
         (void)hipFree(f.buf);
         return st;
@@ -397,7 +396,11 @@ extern "C" qtnh_status qtnh_serve(qtnh_ctx_t ctx, int nq, const qtnh_query *quer
     std::vector<qtnh_circuit_t> cs;
     std::vector<void *> ss;
     std::vector<int> first, count;
+    const int bits = floor_log2(inflight_bytes / sizeof(double2_t));
     for (auto &f : flight) {
+      // The runs of its tiles in this step's launches.  (States of up to 22 qubits
+      // end in this step, and the tiles of larger ones are the same in any.)
+      if (f.next == 0) f.nruns = circuit_run_count(ctx, f.h->c, bits);
       const int left = f.nruns - f.next;
       const int adv = f.key.n <= 22 ? left : f.key.n <= 25 ? std::min(left, 8) : std::min(left, 1);
       cs.push_back(f.h->c);
@@ -406,7 +409,7 @@ extern "C" qtnh_status qtnh_serve(qtnh_ctx_t ctx, int nq, const qtnh_query *quer
       count.push_back(adv);
       f.next += adv;
     }
-    st = circuit_advance(ctx, (int)cs.size(), cs.data(), ss.data(), first.data(), count.data());
+    st = circuit_advance(ctx, (int)cs.size(), cs.data(), ss.data(), first.data(), count.data(), bits);
     if (st) return st;
     st = check_hip(ctx, hipStreamSynchronize(ctx->stream), "serve step sync");
     if (st) return st;

@@ -391,3 +391,24 @@ def test_ops_appended_after_runs_under_several_tiles():
                 c.run(t)
                 assert same_bits(host(t), oracle_run(c, x0)), (more, tb)
         c.gate([more], [0.6, 0.8, 0.8, -0.6]).diag([12, more], [1, 1j, -1, -1j])
+
+
+@pytest.mark.parametrize("n,count", [(11, 8), (12, 7), (12, 8), (15, 16), (16, 16), (18, 2), (18, 4), (19, 2), (19, 4)])
+def test_batch_tiles_by_all_states_bitexact(n, count):
+    """The tile of a batch goes by the amplitudes of all its states; circuits that
+    run alone before and after keep their own."""
+    cs = [_mixed_circuit(n, 40, i == 1, i) for i in range(count)]
+    want = [ops.fill_(ops.empty(1 << n), i) for i in range(count)]
+    got = [w.clone() for w in want]
+    for c, g, w in zip(cs, got, want):
+        for _ in range(4):
+            c.run(w, _lib.RUN_PER_GATE)
+    cs[0].run(got[0])
+    ops.run_batch(cs[1:], got[1:])
+    ops.run_batch(cs, got)
+    for c, g in zip(cs[1:], got[1:]):
+        c.run(g)
+    ops.run_batch(cs[:1], got[:1])
+    ops.run_batch(cs, got)
+    for g, w in zip(got, want):
+        assert torch.equal(torch.view_as_real(g).view(torch.int64), torch.view_as_real(w).view(torch.int64))
