@@ -741,3 +741,38 @@ def test_contract_gemm_more_small_tiles_than_a_launch_takes():
         assert np.linalg.norm(host(got.view(m, n)[i:i + 64]) - want) <= 1e-12 * np.linalg.norm(want), i
     del a, got, rows
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("da,db,wires,repl1,repl2", [
+    # 2^33 elements of dims 2; the open axis of B first in the result
+    ([2] * 33, [2, 2, 2, 2, 2], [(0, 0), (1, 1), (2, 3), (3, 4)], [X] * 4 + list(range(1, 30)), [X, X, 0, X, X]),
+    # 3 x 2^31 elements; the open axis of B last
+    ([16, 3, 1 << 27], [2, 16], [(0, 1)], [X, 0, 1], [2, X]),
+    # the largest that the kernels with 32-bit offsets take
+    ([2] * 32, [2, 2, 2, 2, 2], [(0, 0), (1, 1), (2, 3), (3, 4)], [X] * 4 + list(range(1, 29)), [X, X, 0, X, X]),
+    ([16, 3, 89478485], [2, 16], [(0, 1)], [X, 0, 1], [2, X]),
+])
+def test_contract_direct_around_32_bits_bitexact(da, db, wires, repl1, repl2):
+    """The direct kernels of tensors of 2^32 elements and more, against the
+    oracle on stretches of the result (16 terms each, from all over A)."""
+    torch.cuda.empty_cache()
+    n = math.prod(da)
+    if torch.cuda.mem_get_info()[0] < 160 << 30:
+        pytest.skip("needs 150 GiB of free device memory")
+    a = ops.fill_(ops.empty(n), 11)
+    b = rnd(math.prod(db), 12)
+    got, dc, _ = ops.contract(a, da, dev(b), db, wires, repl1, repl2)
+    inner = n // 16  # results of each B output, consecutive elements of A for each term
+    A = a.view(16, inner)
+    C = got.view(2, inner) if repl2[0] == X else got.view(inner, 2)
+    for i in (0, inner // 3, inner - 1024):
+        piece = host(A[:, i:i + 1024].contiguous()).reshape(-1)
+        if repl2[0] == X:
+            ref, _ = oracle.contract(piece, [2] * 4 + [1024], b, db, wires, [X] * 4 + [1], [X, X, 0, X, X])
+            part = host(C[:, i:i + 1024].contiguous()).reshape(-1)
+        else:
+            ref, _ = oracle.contract(piece, [16, 1024], b, db, wires, [X, 0], [1, X])
+            part = host(C[i:i + 1024].contiguous()).reshape(-1)
+        assert same_bits(part, np.asarray(ref).reshape(-1)), i
+    del a, got, A, C
+    torch.cuda.empty_cache()
