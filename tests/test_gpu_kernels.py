@@ -776,3 +776,21 @@ def test_contract_direct_around_32_bits_bitexact(da, db, wires, repl1, repl2):
         assert same_bits(part, np.asarray(ref).reshape(-1)), i
     del a, got, A, C
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dims,ptup", [([65537, 65537], [1, 0]), ([48, 35, 81, 22, 1500], [4, 1, 3, 0, 2])])
+def test_permute_ragged_beyond_32_bits(dims, ptup):
+    """Boxes with 64-bit offsets (64 GiB a side), on slices of the first, the
+    middle and the last index of every axis."""
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 150 << 30:
+        pytest.skip("needs 140 GiB of free device memory")
+    x = ops.fill_(ops.empty(math.prod(dims)), 4)
+    y = ops.permute(x, dims, ptup)
+    inv = [ptup.index(i) for i in range(len(ptup))]
+    want, got = x.view(dims).permute(inv), y.view([dims[i] for i in inv])
+    for axis, d in enumerate(got.shape):
+        for i in (0, d // 2, d - 1):
+            assert torch.equal(want.select(axis, i), got.select(axis, i)), (axis, i)
+    del x, y, want, got
+    torch.cuda.empty_cache()
