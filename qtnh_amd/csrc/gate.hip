@@ -435,10 +435,11 @@ constexpr unsigned kGateLds = 53000;
 // fit: 1-qubit gates on bits 6 to 23 of 2^28 elements take 1.26 to 1.48 ms
 // so and 1.28 to 1.56 with all (bits 25 to 27: within 2%), 2-qubit gates 2% less
 // on average unless both bits are high (25 and 20: 1.83 against 1.75 ms, 21 and 20:
-// 1.87 against 1.75), 3-qubit gates 3% more as often as less.
+// 1.87 against 1.75; with 18 as the lower bit, 2^24 to 2^32 elements, 2% more on
+// average and up to 7%), 3-qubit gates 3% more as often as less.
 template <int KB>
 bool few_workgroups(const int *ascending_bits) {
-  return KB == 1 || (KB == 2 && ascending_bits[0] < 19);
+  return KB == 1 || (KB == 2 && ascending_bits[0] < 18);
 }
 
 template <int KB>
