@@ -402,8 +402,9 @@ void qtnh_tune_split(int slices);
  * 128 x 128, one workgroup per compute unit; 1 64 x 64, two per compute unit;
  * 2 128 x 64; 3 64 x 64 with eight narrow waves.  Results do not depend on it. */
 void qtnh_tune_split_tile(int shape);
-/* Most workgroups (256..2^22, default 2^20) of the streaming gate kernel for
- * gates on high bits, which loops over the rest.  (The diagonal kernel and the
+/* Most workgroups (256..2^22) of the streaming gate kernel for gates on high
+ * bits, which loops over the rest.  0 (the default): 2^20, and up to 2^22 for
+ * 1-qubit gates and 2-qubit gates with a bit below 18.  (The diagonal kernel and the
  * kernels for gates on the lowest 6 bits size their grids to the state.) */
 void qtnh_tune_stream(int max_blocks);
 /* Tile bits (3..13) of fused circuit runs, and how many of the lowest state

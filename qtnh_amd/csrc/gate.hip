@@ -22,9 +22,10 @@ namespace {
 
 constexpr int kGateThreads = 256;
 
-// Most workgroups of the streaming gate and diagonal kernels (they loop over
-// the rest): enough to keep many requests in flight on every CU.
-unsigned g_stream_blocks = 1u << 20;
+// Most workgroups of the streaming gate kernels (they loop over the rest), where
+// set: enough to keep many requests in flight on every CU.
+unsigned g_stream_blocks = 0;
+constexpr unsigned kStreamBlocks = 1u << 20, kFewBlocks = 1u << 22;  // ... and where not
 // Grid limit of the kernels sized to one element (or row) per thread: a launch
 // takes fewer than 2^32 threads.  They loop over the rest, too.
 constexpr unsigned kMaxStreamBlocks = 1u << 23;
@@ -370,7 +371,7 @@ qtnh_status launch_gate_low3(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *m
   // tile's loads in flight, are slower: 5.38 at two tiles per wave, 5.29 at
   // sixteen, 5.09 (before the scalar coefficient loads) at 512 workgroups.
   const uint64_t n_tiles = n >> 9;
-  const unsigned blocks = grid_for(n_tiles * 64, kGateThreads, g_stream_blocks);
+  const unsigned blocks = grid_for(n_tiles * 64, kGateThreads, g_stream_blocks ? g_stream_blocks : kStreamBlocks);
   hipLaunchKernelGGL(gate_low3_kernel, dim3(blocks), dim3(kGateThreads), 0, ctx->stream, psi, args, n_tiles);
   return check_hip(ctx, hipGetLastError(), "gate launch");
 }
@@ -470,8 +471,16 @@ qtnh_status launch_gate_bits(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *m
     return launch_gate_lanes<KB, (KB >= 3 ? 2 : 0)>(ctx, psi, n, msb_bits, G);
   }
   const uint64_t groups = n >> KB;
-  const unsigned blocks = grid_for(groups, kGateThreads, g_stream_blocks);
-  const unsigned lds = few_workgroups<KB>(args.zpos) ? kGateLds : 0;
+  // Few workgroups in flight go with a grid in which a thread takes one group, or
+  // two: a grid that ends at 2^20 workgroups makes a thread walk 1-qubit gates from
+  // 2^30 elements (bits 6 to 30 of 2^31 11.0 to 13.0 ms, 10.2 to 12.0 with 2^22, 10.7 to
+  // 12.7 with 2^20 and all that fit).  From 2^32 elements it depends on the
+  // allocation: 2-qubit gates took 0.81 to 1.16 times the time so in one run and
+  // another, 0.87 to 1.00 with all that fit and 2^20 workgroups.
+  const bool few = few_workgroups<KB>(args.zpos) && n <= 1ull << 31;
+  const unsigned lds = few ? kGateLds : 0;
+  const unsigned most = g_stream_blocks ? g_stream_blocks : few ? kFewBlocks : kStreamBlocks;
+  const unsigned blocks = grid_for(groups, kGateThreads, most);
   if (args.zpos[0] >= 3)
     hipLaunchKernelGGL((gate_bits_kernel<KB, true>), dim3(blocks), dim3(kGateThreads), lds, ctx->stream, psi, args,
                        groups);
@@ -484,7 +493,7 @@ qtnh_status launch_gate_bits(qtnh_ctx_t ctx, c128 *psi, uint64_t n, const int *m
 }  // namespace
 
 extern "C" void qtnh_tune_stream(int max_blocks) {
-  g_stream_blocks = (unsigned)std::max(256, std::min(max_blocks, 1 << 22));
+  g_stream_blocks = max_blocks <= 0 ? 0 : (unsigned)std::max(256, std::min(max_blocks, 1 << 22));
 }
 
 qtnh_status launch_gate(qtnh_ctx_t ctx, c128 *state, int rank, const uint64_t *dims, int k, const uint16_t *axes,

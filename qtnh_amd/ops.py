@@ -285,8 +285,9 @@ def tune_split_tile(shape=0):
     lib().qtnh_tune_split_tile(int(shape))
 
 
-def tune_stream(max_blocks=1 << 20):
-    """Most workgroups of the streaming kernel for gates on high bits (process-wide)."""
+def tune_stream(max_blocks=0):
+    """Most workgroups of the streaming kernel for gates on high bits (process-wide;
+    0: by gate, as at the start)."""
     lib().qtnh_tune_stream(max_blocks)
 
 

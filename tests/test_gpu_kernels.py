@@ -794,3 +794,20 @@ def test_permute_ragged_beyond_32_bits(dims, ptup):
             assert torch.equal(want.select(axis, i), got.select(axis, i)), (axis, i)
     del x, y, want, got
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("axes", [[3], [20], [2, 12], [5, 1], [4, 12, 19]])
+def test_gate_grids_bitwise(axes):
+    """A thread per group and grids that walk the state give the same bits."""
+    n = 22
+    g = rnd(1 << 2 * len(axes), 3)
+    outs = []
+    try:
+        for blocks in (0, 256, 1000, 1 << 20):
+            ops.tune_stream(blocks)
+            x = ops.fill_(ops.empty(1 << n), 6)
+            outs.append(host(ops.gate_apply_(x, [2] * n, axes, g)))
+    finally:
+        ops.tune_stream()
+    for o in outs[1:]:
+        assert same_bits(o, outs[0])
