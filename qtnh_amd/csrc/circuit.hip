@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(kPipeNT, 1)
 // zeros: -0 where every product is (exactly or by underflow), and +0 there.  A
 // gate's results do not depend on the signs of zeros among its inputs, so a
 // dense record turns -0 into +0 (two additions per amplitude, kRegSettle) only
-// where a diagonal or the store follows.
+// where a diagonal or the end of the circuit follows.
 struct RegOp {
   // One bit per op form.  1-qubit gates on register bits 3..0 (kRegG1): one
   // record may hold several, applied from the highest bit down, their
@@ -1272,8 +1272,8 @@ void plan_reg_run(const qtnh_circuit_s &c, const qtnh_circuit_s::Run &r, int R, 
       room(ncoef);
       RegOp o{0, (uint32_t)(coef.size() / 2), 0, 0};
       if (op.kind == 0) {
-        // A diagonal or the store comes next (register bits may change in between).
-        if (i + 1 == r.end || c.ops[i + 1].kind == 1) o.lane = kRegSettle;
+        // A diagonal comes next, or the circuit ends (a run ends before a dense gate).
+        if (i + 1 == c.ops.size() || c.ops[i + 1].kind == 1) o.lane = kRegSettle;
         const int a = reg_bit(tile_bit(op.q[0])), b = op.k > 1 ? reg_bit(tile_bit(op.q[1])) : 0;
         // A 1-qubit gate joins the record before it if its register bit is below all of that one's.
         RegOp *prev = ops.size() > chunk_op ? &ops.back() : nullptr;
