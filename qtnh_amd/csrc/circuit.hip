@@ -12,8 +12,8 @@
 //  * fused: consecutive ops are grouped into runs touching at most `tb`
 //    distinct index bits.  A run is one pass over the state: each workgroup
 //    gathers a tile of 2^tb amplitudes (the run's bits vary, every other bit
-//    is fixed) into LDS, applies the run's ops in order, and scatters the tile
-//    back.  Every op does the same arithmetic on the same values as the per
+//    is fixed) into registers (some forms: LDS), applies the run's ops in order,
+//    and scatters the tile back.  Every op does the same arithmetic on the same values as the per
 //    gate kernel (sum over inputs in row-major order from zero, products
 //    without FMA), so both executors agree bit for bit; the fused one reads
 //    and writes the state once per run instead of once per op.
