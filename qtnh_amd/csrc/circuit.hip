@@ -485,12 +485,19 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T *as_const(c
 // so that the lanes of an access fall on different banks for nearly every
 // choice of register bits (the vectors were searched for; at most two-way for
 // contiguous ones).  Linear over XOR.
-__host__ __device__ __forceinline__ uint32_t reg_slot(uint32_t l) {
-  constexpr uint32_t kMix[7] = {31, 11, 28, 26, 25, 3, 9};
+constexpr uint32_t kSlotMix[7] = {31, 11, 28, 26, 25, 3, 9};
+__device__ __forceinline__ uint32_t reg_slot(uint32_t l) {
   uint32_t s = l;
 #pragma unroll
-  for (int i = 0; i < 7; ++i) s ^= (0u - ((l >> (5 + i)) & 1u)) & kMix[i];
+  for (int i = 0; i < 7; ++i) s ^= (0u - ((l >> (5 + i)) & 1u)) & kSlotMix[i];
   return s;
+}
+// That of tile bit b (uniform) alone, from the vectors packed five bits a tile bit.
+__device__ __forceinline__ uint32_t reg_slot_bit(uint32_t b) {
+  uint64_t packed = 0;
+#pragma unroll
+  for (int i = 0; i < 7; ++i) packed |= (uint64_t)kSlotMix[i] << (5 * (5 + i));
+  return (1u << b) ^ ((uint32_t)(packed >> (5 * b)) & 31u);
 }
 
 // Deposit over runs of set bits: mask is uniform, so its few runs are walked
@@ -560,11 +567,17 @@ __device__ __forceinline__ void rg_gate1(double (&re)[1 << R], double (&im)[1 <<
   }
 }
 
-// KB-qubit gate on register bits A, B, C (most significant first).
-template <int R, int KB, int A, int B, int C>
+// KB-qubit gate on register bits A, B, C (most significant first).  ROOM: registers
+// for the next input's coefficients.
+template <int R, int KB, int A, int B, int C, bool ROOM>
 __device__ __forceinline__ void rg_gate(double (&re)[1 << R], double (&im)[1 << R], const double2_t *g) {
   constexpr int K = 1 << KB;
   constexpr int M = (1 << A) | (1 << B) | (KB > 2 ? (1 << C) : 0);
+  double2_t row[2][K];  // (ROOM) this input's coefficients and the next one's
+  if (ROOM) {
+#pragma unroll
+    for (int o = 0; o < K; ++o) row[0][o] = g[o];
+  }
 #pragma unroll
   for (int r0 = 0; r0 < (1 << R); ++r0) {
     if (r0 & M) continue;
@@ -584,10 +597,15 @@ __device__ __forceinline__ void rg_gate(double (&re)[1 << R], double (&im)[1 << 
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const double2_t x = {re[idx[i]], im[idx[i]]};
+      if (ROOM) {
+#pragma unroll
+        for (int o = 0; o < K; ++o) row[(i + 1) & 1][o] = g[(i + 1) % K * K + o];
+        __builtin_amdgcn_sched_barrier(0);  // requested before this input's products
+      }
 #pragma unroll
       for (int o = 0; o < K; ++o) {
-        if (o % 4 == 0) asm volatile("" ::: "memory");  // four coefficients live at a time (a compiler barrier, no code)
-        const double2_t p = cmul2(x, g[i * K + o]);
+        if (!ROOM && o % 4 == 0) asm volatile("" ::: "memory");  // four coefficients live at a time (likewise)
+        const double2_t p = cmul2(x, ROOM ? row[i & 1][o] : g[i * K + o]);
         if (i == 0) {
           ar[o] = p.x;
           ai[o] = p.y;
@@ -677,13 +695,25 @@ struct RegRefs {
   }
 };
 
-// KD: most qubits of a dense gate among the launch's ops.
+// KD: most qubits of a dense gate among the launch's ops.  MINW of 2: for launches
+// that leave a compute unit one or two tiles, so one or two waves per SIMD that
+// hide little of one another.  Registers and LDS are there to spare: an exchange
+// takes both parts at once, and a gate of 2 or 3 qubits requests the next input's
+// coefficients before this one's products.  20 qubits, one tile each: a 2-qubit
+// gate 1.7 -> 1.4 us, a 3-qubit one 2.95 -> 2.6, an exchange 1.15 -> 0.8; 24 random
+// 2-qubit gates 107 -> 93 us (86 with the tile in LDS between phases).  With four tiles
+// (22 qubits) the 128-register form is the faster, 80 against 90 us for 24 1-qubit gates.
+constexpr bool reg_room(int minw) { return minw <= 2; }
+constexpr size_t reg_slot_bytes(int minw) { return reg_room(minw) ? sizeof(double2_t) : sizeof(double); }
+
 template <int R, int KD, int MINW>
 __global__ void __launch_bounds__(256, MINW)
     circuit_reg_kernel(const RunDesc *__restrict__ runs, int nruns, uint64_t total_tiles, int lds_tb) {
   constexpr int E = 1 << R;
+  constexpr bool ROOM = reg_room(MINW);
   extern __shared__ double smem[];
-  double2_t *cbuf = reinterpret_cast<double2_t *>(smem + (1u << lds_tb));
+  char *bytes = reinterpret_cast<char *>(smem);
+  double2_t *cbuf = reinterpret_cast<double2_t *>(bytes + (reg_slot_bytes(MINW) << lds_tb));
   uint4 *obuf = reinterpret_cast<uint4 *>(cbuf + kRegCoef);
   const uint32_t thread = threadIdx.x;
   const RegChunk *staged = nullptr;  // the chunk now in LDS
@@ -729,6 +759,16 @@ __global__ void __launch_bounds__(256, MINW)
     };
     uint32_t map = D.map0;
     uint32_t base = reg_base<R>(tid, map);
+    // LDS places under these register bits (bytes): of element 0, and what each
+    // register bit adds to it.
+    uint32_t slot0, slotb[R];
+    auto slots = [&]() {
+      constexpr uint32_t kBytes = reg_slot_bytes(MINW);
+      slot0 = reg_slot(base) * kBytes;
+#pragma unroll
+      for (int k = 0; k < R; ++k) slotb[k] = reg_slot_bit((map >> (4 * k)) & 15u) * kBytes;
+    };
+    slots();
     double re[E], im[E];
 #pragma unroll
     for (int r = 0; r < E; ++r) {
@@ -822,56 +862,67 @@ __global__ void __launch_bounds__(256, MINW)
 #define QTNH_REG_CASE(BIT, NEED, CALL) \
   if constexpr (NEED < R)              \
     if (code & (1u << BIT)) CALL;
-          QTNH_REG_CASE(4, 1, (rg_gate<R, 2, 0, 1, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(5, 2, (rg_gate<R, 2, 0, 2, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(6, 3, (rg_gate<R, 2, 0, 3, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(7, 1, (rg_gate<R, 2, 1, 0, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(8, 2, (rg_gate<R, 2, 1, 2, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(9, 3, (rg_gate<R, 2, 1, 3, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(10, 2, (rg_gate<R, 2, 2, 0, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(11, 2, (rg_gate<R, 2, 2, 1, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(12, 3, (rg_gate<R, 2, 2, 3, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(13, 3, (rg_gate<R, 2, 3, 0, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(14, 3, (rg_gate<R, 2, 3, 1, 0>(re, im, cbuf + co)))
-          QTNH_REG_CASE(15, 3, (rg_gate<R, 2, 3, 2, 0>(re, im, cbuf + co)))
+          QTNH_REG_CASE(4, 1, (rg_gate<R, 2, 0, 1, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(5, 2, (rg_gate<R, 2, 0, 2, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(6, 3, (rg_gate<R, 2, 0, 3, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(7, 1, (rg_gate<R, 2, 1, 0, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(8, 2, (rg_gate<R, 2, 1, 2, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(9, 3, (rg_gate<R, 2, 1, 3, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(10, 2, (rg_gate<R, 2, 2, 0, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(11, 2, (rg_gate<R, 2, 2, 1, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(12, 3, (rg_gate<R, 2, 2, 3, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(13, 3, (rg_gate<R, 2, 3, 0, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(14, 3, (rg_gate<R, 2, 3, 1, 0, ROOM>(re, im, cbuf + co)))
+          QTNH_REG_CASE(15, 3, (rg_gate<R, 2, 3, 2, 0, ROOM>(re, im, cbuf + co)))
 #undef QTNH_REG_CASE
           if (lane & kRegSettle) rg_settle<R>(re, im);
           next();
         }
         if (code & (1u << kRegSpecial)) {
           if constexpr (KD > 2 && R > 2) {
-            if (!(lane & kRegRemapFlag)) rg_gate<R, 3, 2, 1, 0>(re, im, cbuf + co);
+            if (!(lane & kRegRemapFlag)) rg_gate<R, 3, 2, 1, 0, ROOM>(re, im, cbuf + co);
             if (lane & kRegSettle) rg_settle<R>(re, im);
           }
           if (lane & kRegRemapFlag) {
-            const uint32_t s0 = reg_slot(base);
+            const uint32_t s0 = slot0;
             uint32_t sb[R];
 #pragma unroll
-            for (int k = 0; k < R; ++k) sb[k] = reg_slot(1u << ((map >> (4 * k)) & 15u));
+            for (int k = 0; k < R; ++k) sb[k] = slotb[k];
             map = lane;
             base = reg_base<R>(tid, map);
-            const uint32_t s1 = reg_slot(base);
-            uint32_t sn[R];
-#pragma unroll
-            for (int k = 0; k < R; ++k) sn[k] = reg_slot(1u << ((map >> (4 * k)) & 15u));
-            auto slot = [](uint32_t s, const uint32_t (&b)[R], int r) {
+            slots();
+            // Element r's place in LDS (bytes).
+            auto at = [](uint32_t s, const uint32_t (&b)[R], int r) {
+              uint32_t x = 0;
 #pragma unroll
               for (int k = 0; k < R; ++k)
-                if ((r >> k) & 1) s ^= b[k];
-              return s;
+                if ((r >> k) & 1) x ^= b[k];
+              return s ^ x;
             };
             lds_barrier();  // the previous exchange has been read
+            if constexpr (ROOM) {
 #pragma unroll
-            for (int r = 0; r < E; ++r) smem[slot(s0, sb, r)] = re[r];
-            lds_barrier();
+              for (int r = 0; r < E; ++r) *reinterpret_cast<double2_t *>(bytes + at(s0, sb, r)) = double2_t{re[r], im[r]};
+              lds_barrier();
 #pragma unroll
-            for (int r = 0; r < E; ++r) re[r] = smem[slot(s1, sn, r)];
-            lds_barrier();
+              for (int r = 0; r < E; ++r) {
+                const double2_t x = *reinterpret_cast<const double2_t *>(bytes + at(slot0, slotb, r));
+                re[r] = x.x;
+                im[r] = x.y;
+              }
+            } else {
 #pragma unroll
-            for (int r = 0; r < E; ++r) smem[slot(s0, sb, r)] = im[r];
-            lds_barrier();
+              for (int r = 0; r < E; ++r) *reinterpret_cast<double *>(bytes + at(s0, sb, r)) = re[r];
+              lds_barrier();
 #pragma unroll
-            for (int r = 0; r < E; ++r) im[r] = smem[slot(s1, sn, r)];
+              for (int r = 0; r < E; ++r) re[r] = *reinterpret_cast<const double *>(bytes + at(slot0, slotb, r));
+              lds_barrier();
+#pragma unroll
+              for (int r = 0; r < E; ++r) *reinterpret_cast<double *>(bytes + at(s0, sb, r)) = im[r];
+              lds_barrier();
+#pragma unroll
+              for (int r = 0; r < E; ++r) im[r] = *reinterpret_cast<const double *>(bytes + at(slot0, slotb, r));
+            }
           }
           next();
         }
@@ -1565,7 +1616,7 @@ template <int R, int KD, int MINW>
 void launch_reg(qtnh_ctx_t ctx, const RunDesc *d, int nr, uint64_t total, int tb) {
   const unsigned threads = std::max(64, 1 << (tb - R));
   const unsigned blocks = (unsigned)std::min(total, kRegMaxBlocks);
-  const size_t lds = (sizeof(double) << tb) + kRegCoef * sizeof(double2_t) + (kRegOps + 2) * sizeof(RegOp);
+  const size_t lds = (reg_slot_bytes(MINW) << tb) + kRegCoef * sizeof(double2_t) + (kRegOps + 2) * sizeof(RegOp);
   hipLaunchKernelGGL((circuit_reg_kernel<R, KD, MINW>), dim3(blocks), dim3(threads), lds, ctx->stream, d, nr, total, tb);
 }
 
@@ -1594,6 +1645,8 @@ qtnh_status launch_groups(qtnh_ctx_t ctx, const RunDesc *dd, const std::vector<R
         launch_reg<2, 2, 4>(ctx, dd + b, nr, total, tbmax);
       else if (descs[b].rbits == 3)
         g3 ? launch_reg<3, 3, 4>(ctx, dd + b, nr, total, tbmax) : launch_reg<3, 2, 4>(ctx, dd + b, nr, total, tbmax);
+      else if (total <= 2ull * ctx->num_cus)  // one or two tiles a compute unit
+        g3 ? launch_reg<4, 3, 2>(ctx, dd + b, nr, total, tbmax) : launch_reg<4, 2, 2>(ctx, dd + b, nr, total, tbmax);
       else
         g3 ? launch_reg<4, 3, 3>(ctx, dd + b, nr, total, tbmax) : launch_reg<4, 2, 4>(ctx, dd + b, nr, total, tbmax);
       st = check_hip(ctx, hipGetLastError(), "circuit register launch");

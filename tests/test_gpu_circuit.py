@@ -412,3 +412,16 @@ def test_batch_tiles_by_all_states_bitexact(n, count):
     ops.run_batch(cs, got)
     for g, w in zip(got, want):
         assert torch.equal(torch.view_as_real(g).view(torch.int64), torch.view_as_real(w).view(torch.int64))
+
+
+@pytest.mark.parametrize("dense3", [False, True])
+@pytest.mark.parametrize("n", [20, 21, 22, 23])
+def test_few_and_many_tiles_bitexact(n, dense3):
+    """One and two tiles for a compute unit, and more (other registers and LDS):
+    every form of op, against one launch per gate."""
+    c = _mixed_circuit(n, 150, dense3, n)
+    got = ops.fill_(ops.empty(1 << n), n)
+    want = got.clone()
+    c.run(got)
+    c.run(want, _lib.RUN_PER_GATE)
+    assert torch.equal(torch.view_as_real(got).view(torch.int64), torch.view_as_real(want).view(torch.int64))
