@@ -366,7 +366,7 @@ qtnh_status qtnh_autotune_circuit(qtnh_ctx_t ctx, int n_qubits, int *tile_bits, 
  * it overwrites, and keeps the fastest for every later fused run of the
  * circuit (any state, any context; results do not depend on it).  Worth it
  * for circuits run many times: the best tile depends on the circuit (QFT-12:
- * 8 bits, 22.7 against 23.9 us per run), not only on its size.  Outputs may be
+ * 8 bits, 21.7 against 23.0 us per run), not only on its size.  Outputs may be
  * NULL: tile bits, low bits, time per run (us).  No reference counterpart. */
 qtnh_status qtnh_circuit_tune(qtnh_ctx_t ctx, qtnh_circuit_t c, void *scratch, int *tile_bits, int *low_bits,
                               double *us);
